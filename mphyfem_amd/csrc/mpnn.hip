@@ -61,8 +61,8 @@ struct mpf_mpnn {
   mpf::DevBuf<uint16_t> ab[mpf::kLayers + 1];  // bf16 [h_l | a_{l+1}] (the next GEMM's input rows)
   mpf::DevBuf<uint16_t> r[mpf::kLayers + 1];  // relu outputs (bf16) -> relu masks
   mpf::DevBuf<float> y, dy, dh, dcat;      // [N][FOUT], [N][FOUT], [N][W], [N][2W]
-  mpf::DevBuf<uint16_t> db16;              // bf16 copy of the current upstream gradient [N][2W max]
-  mpf::DevBuf<float> part;                 // weight-gradient partials
+  mpf::DevBuf<uint16_t> db16;              // bf16 copy of the current upstream gradient [N][W max]
+  mpf::DevBuf<float> part;                 // weight- and bias-gradient partials
   mpf::DevBuf<double> red;                 // loss partials
   hipStream_t stream = nullptr;
   int64_t adam_t = 0;
@@ -93,7 +93,7 @@ __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint
 
 // ---- GEMM over rows: C[N][COUT] = A[N][KIN] (bf16, row stride lda) * B[KIN][COUT] (bf16, given as
 // its transpose Bt[COUT][KIN] so each lane reads 8 consecutive k), one wavefront per 16 rows ----
-enum { EPI_ENC = 0, EPI_MP = 1, EPI_OUT = 2, EPI_PLAIN = 3 };
+enum { EPI_ENC = 0, EPI_MP = 1, EPI_OUT = 2, EPI_PLAIN = 3, EPI_DCAT = 4 };
 
 struct MMArgs {
   int64_t n;
@@ -106,6 +106,7 @@ struct MMArgs {
   uint16_t* outb;      // bf16 copy of out (row stride ldob), or null
   int ldob;
   uint16_t* rb;        // EPI_MP / EPI_ENC: relu output (bf16) [N][COUT]
+  const int32_t* nbptr;  // EPI_DCAT: columns from W on are divided by the row's number of neighbours
 };
 
 template <int KIN, int COUT, int EPI>
@@ -142,7 +143,8 @@ __global__ void __launch_bounds__(256) k_mm(MMArgs a) {
       const int64_t row = r0 + kg * 4 + i;
       if (row >= a.n) continue;
       float v = acc[t][i];
-      if (EPI != EPI_PLAIN) v += a.bias[c];
+      if (EPI == EPI_ENC || EPI == EPI_MP || EPI == EPI_OUT) v += a.bias[c];
+      if (EPI == EPI_DCAT && t * 16 >= kW) v /= (float)(a.nbptr[row + 1] - a.nbptr[row]);
       if (EPI == EPI_ENC || EPI == EPI_MP) {
         const float rr = v > 0.f ? v : 0.f;
         a.rb[row * COUT + c] = f2bf(rr);
@@ -154,78 +156,148 @@ __global__ void __launch_bounds__(256) k_mm(MMArgs a) {
   }
 }
 
-// ---- weight gradient: part[blk][K][C] = sum over the block's rows of A[r][k] * D[r][c] ----
-// A bf16 [N][K] (row stride lda), D bf16 [N][C] (row stride ldd); rows in chunks of 32 staged in LDS
-// transposed so both MFMA operands are 8 consecutive rows.
-template <int K, int C>
+// ---- weight and bias gradient of one layer, with the ReLU mask of its output ----
+// D[r][c] = src[r][c] (fp32, zero where MASK and the ReLU output rl[r][c] is 0); db receives D in bf16
+// (the next product's operand), and
+//   part[blk][k C + c] = sum over the block's rows of A[r][k] bf16(D[r][c]),   A bf16 (row stride lda)
+//   part[blk][K C + c] = sum over the block's rows of D[r][c]                  (unrounded).
+// One pass over src, rl and A in chunks of 32 rows.  A thread loads two adjacent columns of 8 rows (each
+// row's loads of a wavefront are one contiguous segment) and stores each column's 8 rows as one 16-byte
+// LDS write, so that both MFMA operands (8 consecutive rows of one column per lane) are one 16-byte LDS
+// read; the next chunk's loads are issued before the products of this one.  What bounds it is the latency
+// of a chunk, so the rows are split over up to kGradBlocks workgroups (two a compute unit).
+// Measured on 171 k rows (60 beams), layer gradient K = 128, C = 64: separate mask pass 41 us, products
+// 1115 us (4096 rows a workgroup, 2-byte transposing stores) and bias sums 1087 us before;
+// 33 us for all three now, and 7 us to sum the partials.
+constexpr int kGradChunk = 32;
+constexpr int64_t kGradBlocks = 512;
+
+template <int K, int C, bool MASK>
 __global__ void __launch_bounds__(256) k_wgrad(int64_t n, int64_t rows_per_block, const uint16_t* __restrict__ A,
-                                               int lda, const uint16_t* __restrict__ D, int ldd,
+                                               int lda, const float* __restrict__ src,
+                                               const uint16_t* __restrict__ rl, uint16_t* __restrict__ db,
                                                float* __restrict__ part) {
-  constexpr int NT = (K / 16) * (C / 16);
-  constexpr int TPW = (NT + 3) / 4;  // tiles per wave
-  __shared__ uint16_t sAt[K][40];  // [k][r] (32 rows, padded)
-  __shared__ uint16_t sDt[C][40];  // [c][r]
+  constexpr int NK = K / 16, NC = C / 16;
+  constexpr int NW = NK < 4 ? NK : 4;      // wavefronts along k; the rest of the four along c
+  constexpr int TK = NK / NW, TC = NC / (4 / NW);
+  static_assert(NK % NW == 0 && 4 % NW == 0 && NC % (4 / NW) == 0, "tiles over four wavefronts");
+  constexpr int UA = K / 2 * 4, UD = C / 2 * 4;  // (column pair, 8-row group) units of a chunk
+  static_assert(UA <= 256 && UD <= 256, "one unit per thread");
+  constexpr int LD = kGradChunk + 8;  // LDS rows per column, padded to 80 bytes
+  __shared__ __align__(16) uint16_t sA[2][K * LD];
+  __shared__ __align__(16) uint16_t sD[2][C * LD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t rb0 = (int64_t)blockIdx.x * rows_per_block;
   const int64_t rb1 = min(n, rb0 + rows_per_block);
-  f32x4 acc[TPW];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int64_t c0 = rb0; c0 < rb1; c0 += 32) {
-    __syncthreads();
-    for (int t = tid; t < 32 * K; t += 256) {
-      const int r = t / K, k = t % K;
-      sAt[k][r] = (c0 + r < rb1) ? A[(c0 + r) * lda + k] : (uint16_t)0;
-    }
-    for (int t = tid; t < 32 * C; t += 256) {
-      const int r = t / C, c = t % C;
-      sDt[c][r] = (c0 + r < rb1) ? D[(c0 + r) * ldd + c] : (uint16_t)0;
-    }
-    __syncthreads();
-    const int kg = lane >> 4;
-#pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-      const int t = wave * TPW + q;
-      if (t >= NT) break;
-      const int tk = t / (C / 16), tc = t % (C / 16);
-      bf16x8_s av, bv;
+  const int ca = 2 * (tid % (K / 2)), ga = tid / (K / 2);  // this thread's A unit (tid < UA)
+  const int cd = 2 * (tid % (C / 2)), gd = tid / (C / 2);  // and D unit (tid < UD)
+  uint32_t va[8], vm[8];
+  float2 vd[8];
+  auto load = [&](int64_t c0) {
+    if (tid < UA) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        av[j] = (short)sAt[tk * 16 + (lane & 15)][kg * 8 + j];
-        bv[j] = (short)sDt[tc * 16 + (lane & 15)][kg * 8 + j];
+        const int64_t r = c0 + 8 * ga + j;
+        va[j] = r < rb1 ? *reinterpret_cast<const uint32_t*>(A + r * lda + ca) : 0u;
       }
-      acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv),
-                                                      acc[q], 0, 0, 0);
     }
-  }
-  float* P = part + (size_t)blockIdx.x * K * C;
+    if (tid < UD) {
 #pragma unroll
-  for (int q = 0; q < TPW; ++q) {
-    const int t = wave * TPW + q;
-    if (t >= NT) break;
-    const int tk = t / (C / 16), tc = t % (C / 16);
+      for (int j = 0; j < 8; ++j) {
+        const int64_t r = c0 + 8 * gd + j;
+        vd[j] = r < rb1 ? *reinterpret_cast<const float2*>(src + r * C + cd) : make_float2(0.f, 0.f);
+        vm[j] = MASK ? (r < rb1 ? *reinterpret_cast<const uint32_t*>(rl + r * C + cd) : 0u) : 0u;
+      }
+    }
+  };
+  f32x4 acc[TK][TC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) P[(tk * 16 + (lane >> 4) * 4 + i) * C + tc * 16 + (lane & 15)] = acc[q][i];
+  for (int i = 0; i < TK; ++i)
+#pragma unroll
+    for (int j = 0; j < TC; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float bs0 = 0.f, bs1 = 0.f;
+  const int wk = (wave % NW) * TK, wc = (wave / NW) * TC;  // this wavefront's first tiles
+  const int m16 = lane & 15, kg = lane >> 4;
+  if (rb0 < rb1) load(rb0);
+  int buf = 0;
+  for (int64_t c0 = rb0; c0 < rb1; c0 += kGradChunk, buf ^= 1) {
+    if (tid < UA) {
+      bf16x8_s lo, hi;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { lo[j] = (short)(va[j] & 0xffffu); hi[j] = (short)(va[j] >> 16); }
+      *reinterpret_cast<bf16x8_s*>(&sA[buf][ca * LD + 8 * ga]) = lo;
+      *reinterpret_cast<bf16x8_s*>(&sA[buf][(ca + 1) * LD + 8 * ga]) = hi;
+    }
+    if (tid < UD) {
+      bf16x8_s lo, hi;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float x = vd[j].x, y = vd[j].y;
+        if (MASK) {
+          if ((vm[j] & 0xffffu) == 0) x = 0.f;
+          if ((vm[j] >> 16) == 0) y = 0.f;
+        }
+        const uint16_t bx = f2bf(x), by = f2bf(y);
+        lo[j] = (short)bx;
+        hi[j] = (short)by;
+        const int64_t r = c0 + 8 * gd + j;
+        if (r < rb1) *reinterpret_cast<uint32_t*>(db + r * C + cd) = (uint32_t)bx | ((uint32_t)by << 16);
+        bs0 += x;
+        bs1 += y;
+      }
+      *reinterpret_cast<bf16x8_s*>(&sD[buf][cd * LD + 8 * gd]) = lo;
+      *reinterpret_cast<bf16x8_s*>(&sD[buf][(cd + 1) * LD + 8 * gd]) = hi;
+    }
+    __syncthreads();  // the other buffer's readers have passed the previous one
+    if (c0 + kGradChunk < rb1) load(c0 + kGradChunk);
+    bf16x8_s av[TK], bv[TC];
+#pragma unroll
+    for (int i = 0; i < TK; ++i)
+      av[i] = *reinterpret_cast<const bf16x8_s*>(&sA[buf][((wk + i) * 16 + m16) * LD + kg * 8]);
+#pragma unroll
+    for (int j = 0; j < TC; ++j)
+      bv[j] = *reinterpret_cast<const bf16x8_s*>(&sD[buf][((wc + j) * 16 + m16) * LD + kg * 8]);
+#pragma unroll
+    for (int i = 0; i < TK; ++i)
+#pragma unroll
+      for (int j = 0; j < TC; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[i]),
+                                                           __builtin_bit_cast(bf16x8, bv[j]), acc[i][j], 0, 0, 0);
   }
+  float* P = part + (size_t)blockIdx.x * (K * C + C);
+#pragma unroll
+  for (int i = 0; i < TK; ++i)
+#pragma unroll
+    for (int j = 0; j < TC; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        P[((wk + i) * 16 + kg * 4 + q) * C + (wc + j) * 16 + m16] = acc[i][j][q];
+  // bias: the four 8-row groups of a column pair, in group order
+  __shared__ float sB[4][C];
+  if (tid < UD) { sB[gd][cd] = bs0; sB[gd][cd + 1] = bs1; }
+  __syncthreads();
+  if (tid < C) P[K * C + tid] = ((sB[0][tid] + sB[1][tid]) + sB[2][tid]) + sB[3][tid];
 }
 
-// g[K*C] += sum over blocks of part (block order); bias gradient g_b[c] += sum_r D32[r][c] (fp32 D)
-__global__ void k_wgrad_reduce(int nblk, int KC, const float* __restrict__ part, float* __restrict__ g) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= KC) return;
+// g[i] += sum over blocks of part[b][i], i < m (a layer's weights and then its bias, contiguous in g):
+// 32 outputs and 8 slices of the blocks per workgroup, the slices then summed in order.
+__global__ void __launch_bounds__(256) k_wgrad_reduce(int nblk, int m, const float* __restrict__ part,
+                                                      float* __restrict__ g) {
+  __shared__ float sh[8][32];
+  const int o = threadIdx.x & 31, sl = threadIdx.x >> 5;
+  const int i = blockIdx.x * 32 + o;
   float s = 0.f;
-  for (int b = 0; b < nblk; ++b) s += part[(size_t)b * KC + i];
-  g[i] += s;
-}
-
-__global__ void __launch_bounds__(256) k_bgrad(int64_t n, int C, const float* __restrict__ D, int ldd,
-                                               int64_t rows_per_block, float* __restrict__ part) {
-  // part[blk][C]
-  const int64_t r0 = (int64_t)blockIdx.x * rows_per_block, r1 = min(n, r0 + rows_per_block);
-  for (int c = threadIdx.x; c < C; c += blockDim.x) {
-    float s = 0.f;
-    for (int64_t r = r0; r < r1; ++r) s += D[r * ldd + c];
-    part[(size_t)blockIdx.x * C + c] = s;
+  if (i < m) {
+#pragma unroll 8
+    for (int b = sl; b < nblk; b += 8) s += part[(size_t)b * m + i];
+  }
+  sh[sl][o] = s;
+  __syncthreads();
+  if (sl == 0 && i < m) {
+    float t = sh[0][o];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) t += sh[k][o];
+    g[i] += t;
   }
 }
 
@@ -250,47 +322,29 @@ __global__ void k_agg_fwd(int64_t n, const int32_t* __restrict__ nbptr, const in
   *reinterpret_cast<bf16x8_s*>(out + i * ldo + cg * 8) = o;
 }
 
-// dh[j] += sum_{i in NB(j)} da[i] / |NB(i)|   (NB symmetric), fp32
-__global__ void k_agg_bwd(int64_t n, const int32_t* __restrict__ nbptr, const int32_t* __restrict__ nb,
-                          const float* __restrict__ da, int ldda, float* __restrict__ dh) {
+// dh[j] += dc[j][0..W) + sum_{i in NB(j)} dc[i][W..2W)   (NB symmetric; the second half holds the
+// aggregation's gradient already divided by |NB(i)|), fp32.  16 lanes a node, four channels a lane: the
+// rows are gathered from L2 in 256-byte pieces, four neighbours in flight a lane.
+__global__ void __launch_bounds__(256) k_agg_bwd(int64_t n, const int32_t* __restrict__ nbptr,
+                                                 const int32_t* __restrict__ nb, const float* __restrict__ dc,
+                                                 float* __restrict__ dh) {
+  static_assert(kW == 64, "16 lanes of four channels");
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t j = t >> 6;
-  const int c = (int)(t & 63);
+  const int64_t j = t >> 4;
+  const int c = (int)(t & 15) * 4;
   if (j >= n) return;
-  float s = 0.f;
-  for (int q = nbptr[j]; q < nbptr[j + 1]; ++q) {
-    const int i = nb[q];
-    s += da[(int64_t)i * ldda + c] / (float)(nbptr[i + 1] - nbptr[i]);
-  }
-  dh[j * kW + c] += s;
-}
-
-// dst[i][c] = mask(r[i][c] > 0) * src[i][c] (fp32) and a bf16 copy
-__global__ void k_relu_bwd(int64_t n, int C, const float* __restrict__ src, int lds, const uint16_t* __restrict__ r,
-                           float* __restrict__ dst, uint16_t* __restrict__ dstb) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * C) return;
-  const int64_t i = t / C;
-  const int c = (int)(t % C);
-  const float v = r[t] != 0 ? src[i * lds + c] : 0.f;
-  dst[t] = v;
-  dstb[t] = f2bf(v);
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  const int q1 = nbptr[j + 1];
+#pragma unroll 4
+  for (int q = nbptr[j]; q < q1; ++q) s += *reinterpret_cast<const f32x4*>(dc + (int64_t)nb[q] * (2 * kW) + kW + c);
+  const f32x4 own = *reinterpret_cast<const f32x4*>(dc + j * (2 * kW) + c);
+  f32x4* d = reinterpret_cast<f32x4*>(dh + j * kW + c);
+  *d = (*d + own) + s;
 }
 
 __global__ void k_fill0(int64_t n, double* __restrict__ a) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) a[t] = 0.0;
-}
-
-__global__ void k_to_bf16(int64_t n, const float* __restrict__ a, uint16_t* __restrict__ b) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) b[t] = f2bf(a[t]);
-}
-
-__global__ void k_add(int64_t n, const float* __restrict__ a, int lda, int C, float* __restrict__ b) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * C) return;
-  b[t] += a[(t / C) * lda + t % C];
 }
 
 // bf16 weight copies [K][C] and [C][K] from the fp32 parameter vector
@@ -516,30 +570,30 @@ mpf_status ensure_cap(mpf_mpnn* net, int64_t n) {
   MPF_TRY(net->dy.alloc((size_t)c * kFout));
   MPF_TRY(net->dh.alloc((size_t)c * kW));
   MPF_TRY(net->dcat.alloc((size_t)c * 2 * kW));
-  MPF_TRY(net->db16.alloc((size_t)c * 2 * kW));
+  MPF_TRY(net->db16.alloc((size_t)c * kW));
   net->cap = c;
   return MPF_OK;
 }
-
-constexpr int64_t kRowsPerGradBlock = 4096;
 
 // offsets of the bf16 weight matrices inside wb / wtb
 constexpr int kWbOff[kLayers + 2] = {0, kFin * kW, kFin * kW + 2 * kW * kW, kFin * kW + 4 * kW * kW,
                                      kFin * kW + 6 * kW * kW};
 constexpr int kWbTotal = kFin * kW + 6 * kW * kW + kW * kFout;
 
-template <int K, int C>
-mpf_status wgrad(mpf_mpnn* net, int64_t n, const uint16_t* A, int lda, const uint16_t* D, int ldd, const float* D32,
-                 int ldd32, float* gW, float* gB) {
+// g[0 .. K C + C) += the gradient of a layer's weights and bias; db = its upstream gradient in bf16.  Rows a
+// workgroup: whole chunks, at least 256 rows (a chunk's latency is then paid eight times) and at most
+// kGradBlocks workgroups (the partials a reduction reads).
+template <int K, int C, bool MASK>
+mpf_status wgrad(mpf_mpnn* net, int64_t n, const uint16_t* A, int lda, const float* src, const uint16_t* rl,
+                 uint16_t* db, float* g) {
   hipStream_t s = net->stream;
-  const int nblk = (int)((n + kRowsPerGradBlock - 1) / kRowsPerGradBlock);
-  const size_t need = (size_t)nblk * K * C;
-  if (net->part.n < need) MPF_TRY(net->part.alloc(need));
-  hipLaunchKernelGGL((k_wgrad<K, C>), dim3(nblk), dim3(256), 0, s, n, kRowsPerGradBlock, A, lda, D, ldd,
-                     net->part.ptr);
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(g256(K * C)), dim3(256), 0, s, nblk, K * C, net->part.ptr, gW);
-  hipLaunchKernelGGL(k_bgrad, dim3(nblk), dim3(64), 0, s, n, C, D32, ldd32, kRowsPerGradBlock, net->part.ptr);
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(g256(C)), dim3(256), 0, s, nblk, C, net->part.ptr, gB);
+  const int64_t rows = std::max<int64_t>(256, (((n + kGradBlocks - 1) / kGradBlocks + kGradChunk - 1) / kGradChunk) *
+                                                  kGradChunk);
+  const int nblk = (int)((n + rows - 1) / rows);
+  constexpr int m = K * C + C;
+  if (net->part.n < (size_t)nblk * m) MPF_TRY(net->part.alloc((size_t)nblk * m));
+  hipLaunchKernelGGL((k_wgrad<K, C, MASK>), dim3(nblk), dim3(256), 0, s, n, rows, A, lda, src, rl, db, net->part.ptr);
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3((m + 31) / 32), dim3(256), 0, s, nblk, m, net->part.ptr, g);
   MPF_HIP(hipGetLastError());
   return MPF_OK;
 }
@@ -580,33 +634,25 @@ mpf_status mpnn_backward(mpf_mpnn* net, int64_t n, const int32_t* nbptr, const i
   const unsigned gmm = (unsigned)((n + 63) / 64);
   float* g = net->g.ptr;
   // output layer: dWo = h3^T dy, dbo = sum dy; dh = dy Wo^T
-  hipLaunchKernelGGL(k_to_bf16, dim3(g256(n * kFout)), dim3(256), 0, s, n * kFout, net->dy.ptr, net->db16.ptr);
-  MPF_TRY((wgrad<kW, kFout>(net, n, net->ab[kLayers].ptr, 2 * kW, net->db16.ptr, kFout, net->dy.ptr, kFout,
-                            g + MpnnParams::WO, g + MpnnParams::BO)));
+  MPF_TRY((wgrad<kW, kFout, false>(net, n, net->ab[kLayers].ptr, 2 * kW, net->dy.ptr, nullptr, net->db16.ptr,
+                                   g + MpnnParams::WO)));
   MMArgs a{};
   a.n = n; a.A = net->db16.ptr; a.lda = kFout; a.Bt = net->wb.ptr + kWbOff[kLayers + 1]; a.out = net->dh.ptr;
   hipLaunchKernelGGL((k_mm<kFout, kW, EPI_PLAIN>), dim3(gmm), dim3(256), 0, s, a);
   for (int l = kLayers; l >= 1; --l) {
-    // dr = dh * (r_l > 0)  -> dcat[:, :W] (fp32) and db16 (bf16)
-    hipLaunchKernelGGL(k_relu_bwd, dim3(g256(n * kW)), dim3(256), 0, s, n, kW, net->dh.ptr, kW, net->r[l].ptr,
-                       net->dcat.ptr, net->db16.ptr);
-    const int wl = MpnnParams::WL + (l - 1) * MpnnParams::LSZ;
-    MPF_TRY((wgrad<2 * kW, kW>(net, n, net->ab[l - 1].ptr, 2 * kW, net->db16.ptr, kW, net->dcat.ptr, kW, g + wl,
-                               g + wl + 2 * kW * kW)));
-    // d[h | a] = dr W_l^T  (N x 2W) into dcat
+    // dr = dh * (r_l > 0) (db16), and its products with the layer's input rows
+    MPF_TRY((wgrad<2 * kW, kW, true>(net, n, net->ab[l - 1].ptr, 2 * kW, net->dh.ptr, net->r[l].ptr, net->db16.ptr,
+                                     g + MpnnParams::WL + (l - 1) * MpnnParams::LSZ)));
+    // d[h | a] = dr W_l^T  (N x 2W) into dcat, the second half over each node's neighbour count
     MMArgs b{};
-    b.n = n; b.A = net->db16.ptr; b.lda = kW; b.Bt = net->wb.ptr + kWbOff[l]; b.out = net->dcat.ptr;
-    hipLaunchKernelGGL((k_mm<kW, 2 * kW, EPI_PLAIN>), dim3(gmm), dim3(256), 0, s, b);
-    // dh_{l-1} = dh_l + d[:, :W] + agg_bwd(d[:, W:])
-    hipLaunchKernelGGL(k_add, dim3(g256(n * kW)), dim3(256), 0, s, n, net->dcat.ptr, 2 * kW, kW, net->dh.ptr);
-    hipLaunchKernelGGL(k_agg_bwd, dim3(g256(n * 64)), dim3(256), 0, s, n, nbptr, nb, net->dcat.ptr + kW, 2 * kW,
-                       net->dh.ptr);
+    b.n = n; b.A = net->db16.ptr; b.lda = kW; b.Bt = net->wb.ptr + kWbOff[l]; b.out = net->dcat.ptr; b.nbptr = nbptr;
+    hipLaunchKernelGGL((k_mm<kW, 2 * kW, EPI_DCAT>), dim3(gmm), dim3(256), 0, s, b);
+    // dh_{l-1} = dh_l + d[:, :W] + the neighbours' d[:, W:]
+    hipLaunchKernelGGL(k_agg_bwd, dim3(g256(n * 16)), dim3(256), 0, s, n, nbptr, nb, net->dcat.ptr, net->dh.ptr);
   }
   // encoder: dz0 = dh0 * (r0 > 0); dW0 = x^T dz0
-  hipLaunchKernelGGL(k_relu_bwd, dim3(g256(n * kW)), dim3(256), 0, s, n, kW, net->dh.ptr, kW, net->r[0].ptr,
-                     net->dcat.ptr, net->db16.ptr);
-  MPF_TRY((wgrad<kFin, kW>(net, n, net->x.ptr, kFin, net->db16.ptr, kW, net->dcat.ptr, kW, g + MpnnParams::W0,
-                           g + MpnnParams::B0)));
+  MPF_TRY((wgrad<kFin, kW, true>(net, n, net->x.ptr, kFin, net->dh.ptr, net->r[0].ptr, net->db16.ptr,
+                                 g + MpnnParams::W0)));
   MPF_HIP(hipGetLastError());
   return MPF_OK;
 }

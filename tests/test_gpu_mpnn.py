@@ -111,3 +111,40 @@ def test_guess_without_network_is_linear_extrapolation(mpf, gpu):
     net.guess(P, uk, ukm1, 0.5, False, out)
     ref = uk + 0.5 * (uk - ukm1)
     assert torch.allclose(out, ref, rtol=1e-15, atol=1e-15)
+
+
+@pytest.mark.parametrize("edges", [[1], [5, 7], [20]])
+def test_mpnn_backward_row_remainders_vs_oracle(mpf, gpu, edges):
+    """Layer gradients over 8, 728 and 9 261 rows: fewer rows than one 32-row chunk, several 256-row
+    workgroups, and last chunks of 8, 24 and 13 rows.  Tolerance: a value that FP32 and FP64 sums put on
+    different sides of a BF16 rounding boundary moves one row's product by 2^-8 of itself, and the sum of
+    n random rows is sqrt(n) rows long; eight such rows adding up are 8 / 256 / sqrt(9261) = 3.2e-4
+    (measured 1e-4 there, 1e-6 and less at the smaller sizes).  Leaving out the last row (planted in the
+    oracle) moves a gradient by about 1 / sqrt(n) >= 1e-2 of its length."""
+    import torch
+    tol = 3.2e-4
+    B = mpf.mesh_batch_hex(edges)
+    P = mpf.Problem(mpf.HEX8, B.X, B.conn, mpf.matl_from_E_nu(1e3, 0.3, tangent=mpf.TANGENT_CONSISTENT))
+    for m in range(len(edges)):
+        P.add_dirichlet(B.bottom[m], -1)
+    P.prepare_matrix_pattern()
+    n = len(B.X)
+    ptr, nb = node_graph(B.conn, n)
+    net = mpf.Mpnn(seed=11)
+    w, _ = net.params()
+    rng = np.random.default_rng(n)
+    x = O.bf16(rng.standard_normal((n, O.FIN)))
+    xt = torch.from_numpy((x.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).view(np.int16)).to(gpu)
+    dy = rng.standard_normal((n, O.FOUT)).astype(np.float32)
+    net.forward(P, xt, None)
+    net.zero_grad()
+    net.backward(P, torch.from_numpy(dy).to(gpu))
+    G = O.unpack(net.params()[1])
+    _, cache = O.forward(w.astype(np.float64), x, ptr, nb, bf16_ops=True)
+    R = O.unpack(O.backward(w.astype(np.float64), cache, dy.astype(np.float64), ptr, nb, bf16_ops=True))
+    for k in R:
+        print(f"[mpnn] {n} rows, grad {k}: {_rel(G[k], R[k]):.2e}", flush=True)
+        assert _rel(G[k], R[k]) < tol, k
+    dy[-1] = 0.0
+    bad = O.unpack(O.backward(w.astype(np.float64), cache, dy.astype(np.float64), ptr, nb, bf16_ops=True))
+    assert _rel(G["bo"], bad["bo"]) > 4 * tol and _rel(G["Wo"], bad["Wo"]) > 4 * tol
