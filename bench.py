@@ -172,7 +172,7 @@ def bench_batch(M, a) -> int:
     log(f"batch: {a.nmesh} blocks, {nElem} elements, {nNode} nodes, setup {t_setup:.2f} s")
     T, L, ms_it = P.batch_autotune()
     amode, acap, ams = P.batch_assembly_choice()
-    aname = {M.ASSEMBLY_GATHER: f"gather, chunk kernel staging <= {acap} elements",
+    aname = {M.ASSEMBLY_GATHER: "gather",
              M.ASSEMBLY_GATHER_DIRECT: "gather, direct record reads",
              M.ASSEMBLY_COLORED_SCATTER: "coloured scatter"}[amode]
     log(f"autotune: {aname} ({ams:.2f} ms per assembly); tile {T}, {L} lanes per row, {ms_it:.3f} ms per CG iteration")
@@ -376,7 +376,7 @@ def assembly_bench(M, a, wl: str, n: int):
     bpe = BYTES_PER_ELEM[wl]
     achieved = bpe * nElem / (ms_kern * 1e-3) / 1e9
     if a.assembly != "scatter":
-        kname = "k_stage + k_flat + k_rhs + k_lift (row-owner gather, 4 launches"
+        kname = "k_elem_records + k_rows (row-owner gather, 2 launches"
     else:
         kname = {"tet10": "tet10_kernel<4,false>", "hex8": "hex8_kernel<8,false>",
                  "hex8p0": "hex8p0_kernel<true>"}[wl] + f" ({ncolors} colour launches"
@@ -451,8 +451,7 @@ def main(argv=None) -> int:
     ap.add_argument("--no-secondary", action="store_true",
                     help="tet10: skip the Hex8 assembly and load-step objects beside the headline line")
     ap.add_argument("--assembly", choices=["gather", "direct", "scatter"], default="gather",
-                    help="row-owner gather assembly (default; Hex8 stages chunks of element records in LDS), "
-                         "the gather with every item reading the records directly, or coloured element scatter")
+                    help="row-owner gather assembly (default; 'direct' runs the same kernels), or coloured element scatter")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only copy 1 GiB device-to-device 3 times (reference run for the HBM byte counters)")
     a = ap.parse_args(argv)

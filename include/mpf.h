@@ -147,21 +147,20 @@ mpf_status mpf_add_traction(mpf_problem* p, int32_t nf, const int32_t* faces, do
 mpf_status mpf_add_traction_tri6(mpf_problem* p, int32_t nf, const int32_t* faces, double v0, double v1);
 
 /* Assembly algorithm used by mpf_assemble (same K and R either way):                           */
-/*   MPF_ASSEMBLY_GATHER (default): per-element Gauss-point staging, then the (element, node)     */
-/*     contributions to each node's rows are summed in element order and every CSR value and    */
-/*     rhs entry is written once (no zero fill, no atomics, bitwise reproducible).              */
+/*   MPF_ASSEMBLY_GATHER (default): every element's pair blocks as a dense record, then the        */
+/*     (element, node) contributions to each node's rows are summed in element order and every  */
+/*     CSR value and rhs entry is written once (no zero fill, no atomics, bitwise reproducible). */
 /*   MPF_ASSEMBLY_COLORED_SCATTER: elements of one colour per launch add their K_e/R_e blocks into  */
 /*     CSR through the per-element slot map (no two elements of a launch share a node).           */
-/*   MPF_ASSEMBLY_GATHER_DIRECT: the gather with every item reading the staging records directly   */
-/*     (for Hex8 the default copies the records of each chunk of 8 wavefronts to LDS first).      */
+/*   MPF_ASSEMBLY_GATHER_DIRECT: the same kernels as MPF_ASSEMBLY_GATHER (kept for callers that     */
+/*     select it; the records are always read directly).                                          */
 /* The gather tables hold up to 64 elements and 128 coupled nodes per node; for a mesh beyond    */
 /* that the problem switches itself to the coloured scatter (mpf_get_assembly_mode reports it).  */
 enum { MPF_ASSEMBLY_GATHER = 0, MPF_ASSEMBLY_COLORED_SCATTER = 1, MPF_ASSEMBLY_GATHER_DIRECT = 2 };
 mpf_status mpf_set_assembly_mode(mpf_problem* p, int32_t mode);
 mpf_status mpf_get_assembly_mode(const mpf_problem* p, int32_t* mode);
-/* Hex8 gather tuning: the largest number of distinct elements (0..32, default 32) whose staging  */
-/* records a chunk of 8 wavefronts copies to LDS; a chunk with more reads them directly (same     */
-/* values).  No counterpart in the reference; 0 makes every chunk take the direct reads.         */
+/* Accepted (0..32) and reported by mpf_batch_assembly_choice, without effect: the gather reads   */
+/* every element record directly.  No counterpart in the reference.                              */
 mpf_status mpf_set_chunk_stage_cap(mpf_problem* p, int32_t cap);
 
 /* prepareMatrixPattern (femSolidmechanics2.cpp:121-478) on the device: DOF numbering, pressure   */
@@ -372,11 +371,9 @@ typedef struct {
 } mpf_batch_report;
 
 /* Element batch and Jacobi-PCG tile shape by measurement, on the batch's own system: first the     */
-/* assembly (the row-owner gather whose chunk kernel stages at most 8, 16, 24 or 32 distinct       */
-/* elements per chunk in LDS, the gather reading each record directly, or the coloured scatter),   */
-/* each timed over three assemblies, then every (tile, lanes_per_row)                              */
-/* candidate over a few CG iterations; the fastest are kept for mpf_batch_newton_solve.  The       */
-/* gather variants give bitwise the same system.                                                   */
+/* assembly (the row-owner gather or the coloured scatter), each timed over three assemblies, then */
+/* every (tile, lanes_per_row) candidate over a few CG iterations; the fastest are kept for         */
+/* mpf_batch_newton_solve.                                                                          */
 mpf_status mpf_batch_autotune(mpf_problem* p, int32_t* tile, int32_t* lanes_per_row, double* ms_per_cg_iter);
 /* The autotuner's assembly pick: MPF_ASSEMBLY_* mode, staged-element cap, ms per assembly          */
 /* (MPF_ERR_STATE before mpf_batch_autotune).                                                      */

@@ -693,11 +693,11 @@ class Problem:
         return it.value, rep
 
     def set_assembly_mode(self, mode: int):
-        """ASSEMBLY_GATHER (row-owner, default), ASSEMBLY_COLORED_SCATTER or ASSEMBLY_GATHER_DIRECT."""
+        """ASSEMBLY_GATHER (row-owner, default), ASSEMBLY_COLORED_SCATTER or ASSEMBLY_GATHER_DIRECT (as GATHER)."""
         _check(lib().mpf_set_assembly_mode(self._h, mode), "mpf_set_assembly_mode")
 
     def set_chunk_stage_cap(self, cap: int):
-        """Hex8 gather: most distinct elements a chunk of 8 wavefronts stages in LDS (0..32)."""
+        """Accepted (0..32) without effect: the gather reads every element record directly."""
         _check(lib().mpf_set_chunk_stage_cap(self._h, cap), "mpf_set_chunk_stage_cap")
 
     def band_stats(self):

@@ -710,20 +710,15 @@ mpf_status batch_autotune(mpf_problem* p, int32_t* T_out, int32_t* LPR_out, doub
   hipEvent_t e0, e1;
   MPF_HIP(hipEventCreate(&e0));
   MPF_HIP(hipEventCreate(&e1));
-  // element batch: the row-owner gather with its chunk kernel staging at most cap distinct elements
-  // per chunk in LDS (cap 8 .. 32), the gather reading every record directly, or the coloured scatter,
-  // each timed over three first-iteration assemblies
+  // element batch: the row-owner gather or the coloured scatter, each timed over three first-iteration
+  // assemblies
   {
-    struct Cand { int32_t mode, cap; };
-    std::vector<Cand> cands;
-    for (int32_t cap : {8, 16, 24, 32}) cands.push_back({MPF_ASSEMBLY_GATHER, cap});
-    cands.push_back({MPF_ASSEMBLY_GATHER_DIRECT, p->chunk_cap});
-    cands.push_back({MPF_ASSEMBLY_COLORED_SCATTER, p->chunk_cap});
+    struct Cand { int32_t mode; };
+    const Cand cands[] = {{MPF_ASSEMBLY_GATHER}, {MPF_ASSEMBLY_COLORED_SCATTER}};
     double abest = 1e300;
     Cand pick = cands[0];
     for (const Cand& c : cands) {
       p->asm_mode = c.mode;
-      p->chunk_cap = c.cap;
       if (c.mode != MPF_ASSEMBLY_COLORED_SCATTER) MPF_TRY(ensure_gather_tables(p));
       MPF_TRY(enqueue_assembly(p, true, 1.0, 1));  // warm-up
       MPF_HIP(hipEventRecord(e0, s));
@@ -736,9 +731,8 @@ mpf_status batch_autotune(mpf_problem* p, int32_t* T_out, int32_t* LPR_out, doub
       if (ms / reps < abest) { abest = ms / reps; pick = c; }
     }
     p->asm_mode = pick.mode;
-    p->chunk_cap = pick.cap;
     B.asm_mode = pick.mode;
-    B.asm_cap = pick.cap;
+    B.asm_cap = p->chunk_cap;
     B.asm_ms = abest;
   }
   const int Ts[] = {512, 1024, 2048, 4096};

@@ -136,26 +136,8 @@ __device__ __forceinline__ void hex8_dN(int gp, double d[3][8]) {
   }
 }
 
-// dN/dxi of one Hex8 node a at Gauss point gp: the same products as hex8_dN.
-__device__ __forceinline__ void hex8_dN_node(int gp, int a, double d[3]) {
-  const double x1 = (gp == 1 || gp == 2 || gp == 5 || gp == 6) ? kGP2 : -kGP2;
-  const double x2 = (gp == 2 || gp == 3 || gp == 6 || gp == 7) ? kGP2 : -kGP2;
-  const double x3 = (gp >= 4) ? kGP2 : -kGP2;
-  const int iu = (a == 1 || a == 2 || a == 5 || a == 6) ? 1 : 0;
-  const int iv = (a == 2 || a == 3 || a == 6 || a == 7) ? 1 : 0;
-  const int iw = (a >= 4) ? 1 : 0;
-  const double Nu = iu ? 0.5 * (1.0 + x1) : 0.5 * (1.0 - x1);
-  const double Nv = iv ? 0.5 * (1.0 + x2) : 0.5 * (1.0 - x2);
-  const double Nw = iw ? 0.5 * (1.0 + x3) : 0.5 * (1.0 - x3);
-  const double du = iu ? 0.5 : -0.5, dv = iv ? 0.5 : -0.5, dw = iw ? 0.5 : -0.5;
-  d[0] = du * Nv * Nw;
-  d[1] = Nu * dv * Nw;
-  d[2] = Nu * Nv * dw;
-}
-
 // g = grad_x N from dN/dxi (d) and the inverse Jacobian Bi (row-major, Bi[r][c] = dxi_c/dx_r in the
-// element_point convention), with explicit fused multiply-adds so that every kernel that forms g
-// from a stored Bi gets the same bits as the stage kernel.
+// gauss_state convention), with explicit fused multiply-adds.
 __device__ __forceinline__ void grad_jinv(const double* Bi, const double d[3], double g[3]) {
   g[0] = fma(d[2], Bi[2], fma(d[1], Bi[1], d[0] * Bi[0]));
   g[1] = fma(d[2], Bi[5], fma(d[1], Bi[4], d[0] * Bi[3]));
@@ -213,33 +195,34 @@ __device__ __forceinline__ double group_sum(double v) {
 
 __device__ __forceinline__ int rank3(int mask, int i) { return __popc(mask & ((1 << i) - 1)); }
 
-// One Gauss point of one element: reference Jacobian from X, F from u (and Fn from u_prev for the
-// mixed element), current Jacobian from x = X + u, Neo-Hookean state.  Writes g_a, (b g)_a for all
-// nodes into G[a*6 + c] and returns the Gauss-point scalars; the residual contribution of node a,
-// -dv sum_m g_a,m sigma_i,m, is reduced over the NGP lanes of the element (consecutive lanes,
-// lane & (NGP-1) == gp) and stored by the lane gp == a % NGP into R[a*3 + i].
-// Elem_Solid_3D_Disp.cpp:250-330; ElementBase2.cpp:350-470.
-// COMPACT output (the gather path's Hex8 staging records): the inverse Jacobian Bi (9 doubles,
-// row-major) at G, from which g of every node is formed with grad_jinv, and the six components
-// b00 b11 b22 b01 b02 b12 of the symmetric b at Bv, instead of g and b g of every node at G + a * 6.
-// GPAD output (the gather path's Tet10 staging records): g of every node at G + a * 4 (g0 g1 g2 0)
-// and the six components of b at Bv.
-template <int NPE, int NGP, bool MIXED, bool COMPACT = false, bool GPAD = false>
-__device__ __forceinline__ void element_point(const double (*X)[3], const double (*U)[3], const double (*UP)[3],
-                                              const double* Pn, const double (*d)[NPE], int gp, double wgp,
-                                              double mu, double K, int Utype, bool consistent, bool writer,
-                                              double* G, double* S, double* R, bool& negJ, double* Bv = nullptr) {
-  double B[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, Bi[3][3];
-#pragma unroll
+// State of one element at one Gauss point.
+struct GaussState {
+  NHPoint nh;        // stress, b and the tangent scalars
+  double Bi[3][3];   // inverse current Jacobian: grad_x N_a from grad_jinv
+  double dv, dv0;    // current and reference volume weights
+  double thetahat, resip;  // mixed elements: 1 / U'', and the pressure equation J - Jhat - thetahat p
+  bool negJ;         // det F < 0
+};
+
+// Reference Jacobian from X, F from u (and Fn from u_prev for the mixed element), current Jacobian from
+// x = X + u, Neo-Hookean state.  Elem_Solid_3D_Disp.cpp:250-330; ElementBase2.cpp:350-470.
+// UN: nodes per unrolled step (all at once keep their nodal data in registers).
+template <int NPE, int NGP, bool MIXED, int UN = NPE>
+__device__ __forceinline__ void gauss_state(const double (*X)[3], const double (*U)[3], const double (*UP)[3],
+                                            const double* Pn, const double (*d)[NPE], int gp, double wgp, double mu,
+                                            double K, int Utype, bool consistent, GaussState& Q) {
+  double B[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+  double (&Bi)[3][3] = Q.Bi;
+#pragma unroll UN
   for (int a = 0; a < NPE; ++a)
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double xc = X[a][c];
       B[0][c] += xc * d[0][a]; B[1][c] += xc * d[1][a]; B[2][c] += xc * d[2][a];
     }
-  const double dv0 = wgp * inv3(B, Bi);
+  Q.dv0 = wgp * inv3(B, Bi);
   double F[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}}, Fn[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
-#pragma unroll
+#pragma unroll UN
   for (int a = 0; a < NPE; ++a) {
     const double gx = d[0][a] * Bi[0][0] + d[1][a] * Bi[0][1] + d[2][a] * Bi[0][2];
     const double gy = d[0][a] * Bi[1][0] + d[1][a] * Bi[1][1] + d[2][a] * Bi[1][2];
@@ -254,26 +237,27 @@ __device__ __forceinline__ void element_point(const double (*X)[3], const double
       }
     }
   }
-  double Jhat = 1.0, thetahat = 0.0;
+  double Jhat = 1.0;
+  Q.thetahat = 0.0;
   if (MIXED && Utype != -1) {  // compute_constants_volumetric_functions (utilitiesmaterialHyperelastic.cpp:144-173)
     const double Jn = det3(Fn);
     double d1, d2;
     vol_derivs(Utype, K, Jn, d1, d2);
     Jhat = Jn - d1 / d2;
-    thetahat = 1.0 / d2;
+    Q.thetahat = 1.0 / d2;
   }
   const double J = det3(F);
-  negJ = J < 0.0;
+  Q.negJ = J < 0.0;
 #pragma unroll
   for (int r = 0; r < 3; ++r) B[r][0] = B[r][1] = B[r][2] = 0.0;
-#pragma unroll
+#pragma unroll UN
   for (int a = 0; a < NPE; ++a)
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double xc = X[a][c] + U[a][c];
       B[0][c] += xc * d[0][a]; B[1][c] += xc * d[1][a]; B[2][c] += xc * d[2][a];
     }
-  const double dv = wgp * inv3(B, Bi);
+  Q.dv = wgp * inv3(B, Bi);
   double pres = 0.0;
   if (MIXED) {
     if constexpr (NPE == 8) {
@@ -285,31 +269,37 @@ __device__ __forceinline__ void element_point(const double (*X)[3], const double
       for (int q = 0; q < 4; ++q) pres += Np[q] * Pn[q];
     }
   }
-  NHPoint P;
-  neohooke_point(F, J, mu, K, Utype, MIXED, pres, dv, consistent, P);
-  if (writer && COMPACT) {
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) G[3 * r + c] = Bi[r][c];
-  }
+  neohooke_point(F, J, mu, K, Utype, MIXED, pres, Q.dv, consistent, Q.nh);
+  Q.resip = J - Jhat - Q.thetahat * pres;
+}
+
+// One Gauss point of one element: writes g_a, (b g)_a for all nodes into G[a*6 + c] and the Gauss-point
+// scalars into S; the residual contribution of node a, -dv sum_m g_a,m sigma_i,m, is reduced over the
+// NGP lanes of the element (consecutive lanes, lane & (NGP-1) == gp) and stored by the lane
+// gp == a % NGP into R[a*3 + i].
+template <int NPE, int NGP, bool MIXED>
+__device__ __forceinline__ void element_point(const double (*X)[3], const double (*U)[3], const double (*UP)[3],
+                                              const double* Pn, const double (*d)[NPE], int gp, double wgp,
+                                              double mu, double K, int Utype, bool consistent, bool writer,
+                                              double* G, double* S, double* R, bool& negJ) {
+  GaussState Q;
+  gauss_state<NPE, NGP, MIXED>(X, U, UP, Pn, d, gp, wgp, mu, K, Utype, consistent, Q);
+  const NHPoint& P = Q.nh;
+  negJ = Q.negJ;
 #pragma unroll
   for (int a = 0; a < NPE; ++a) {
     double ga[3];
     const double da[3] = {d[0][a], d[1][a], d[2][a]};
-    grad_jinv(&Bi[0][0], da, ga);
+    grad_jinv(&Q.Bi[0][0], da, ga);
     const double g0 = ga[0], g1 = ga[1], g2 = ga[2];
-    if (writer && GPAD) {
-      double* Ga = G + a * 4;
-      Ga[0] = g0; Ga[1] = g1; Ga[2] = g2; Ga[3] = 0.0;
-    } else if (writer && !COMPACT) {
+    if (writer) {
       double* Ga = G + a * 6;
       Ga[0] = g0; Ga[1] = g1; Ga[2] = g2;
       Ga[3] = P.b[0][0] * g0 + P.b[0][1] * g1 + P.b[0][2] * g2;
       Ga[4] = P.b[1][0] * g0 + P.b[1][1] * g1 + P.b[1][2] * g2;
       Ga[5] = P.b[2][0] * g0 + P.b[2][1] * g1 + P.b[2][2] * g2;
     }
-    const double b0 = dv * g0, b1 = dv * g1, b2 = dv * g2;
+    const double b0 = Q.dv * g0, b1 = Q.dv * g1, b2 = Q.dv * g2;
     double r[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -321,15 +311,11 @@ __device__ __forceinline__ void element_point(const double (*X)[3], const double
   }
   if (writer) {
     S[0] = P.s1; S[1] = P.s2; S[2] = P.s3; S[3] = P.s4; S[4] = P.s5;
-    if (MIXED) { S[4] = dv; S[5] = dv0; S[6] = thetahat; S[7] = J - Jhat - thetahat * pres; }
-    if (COMPACT || GPAD) {
-      Bv[0] = P.b[0][0]; Bv[1] = P.b[1][1]; Bv[2] = P.b[2][2];
-      Bv[3] = P.b[0][1]; Bv[4] = P.b[0][2]; Bv[5] = P.b[1][2];
-    }
+    if (MIXED) { S[4] = Q.dv; S[5] = Q.dv0; S[6] = Q.thetahat; S[7] = Q.resip; }
   }
 }
 
-// b g from the six stored components of the symmetric b (same products and order as element_point).
+// b g from the six components b00 b11 b22 b01 b02 b12 of the symmetric b.
 __device__ __forceinline__ void bsym_times(const double* B6, const double g[3], double bg[3]) {
   bg[0] = B6[0] * g[0] + B6[3] * g[1] + B6[4] * g[2];
   bg[1] = B6[3] * g[0] + B6[1] * g[1] + B6[5] * g[2];

@@ -5,19 +5,17 @@
 // (SolverPetsc.cpp:357-378, 434-502) with the first-iteration Dirichlet lift (ElementBase.cpp:567-594,
 // 717-782), organised for the GPU in two kernels:
 //
-//   stage kernel  (one wavefront per EPW elements, lane = (element, Gauss point)):
-//       per element and Gauss point, grad_x N and b grad_x N of every node and the tangent
-//       scalars, plus the element residual, into a staging record of TS doubles per element.
-//   matrix kernel (one wavefront per 64 laid-out items of one node n):
-//       for every element e around n and every node b of e, the 3x3 block K_{n b} (and the u-p
-//       couplings) from e's staging record, visited in (column block, element id) order from a table
-//       built once with the pattern; each column block's run of contributions is summed in element
-//       order, then every CSR value of n's rows and n's right-hand-side entries are written once.
-//       Hex8 runs it per chunk of 8 wavefronts whose elements' records are first copied to LDS.
+//   element kernel: per element, the 3x3 tangent blocks of its node pairs (each unordered pair once:
+//       K_e is symmetric), its u-p couplings and its residual with the lift, as one dense record.
+//   row kernel (one wavefront per 64 laid-out items of one or more nodes): every item is one element
+//       around a node and one node of it; its block is read from the element's record, the blocks of
+//       each column are summed in element order in LDS, and the node's CSR rows and right-hand side go
+//       out with consecutive lanes on consecutive values.
 //
 // Nothing is read-modify-written, so there is no zero fill, no colouring and no atomics on the FP64
 // path, and the result is bitwise reproducible.  Each column block's contributions are summed in
-// element order, the reference's own order for a given row (femSolidmechanics2.cpp:1061).
+// element order, the reference's own order for a given row (femSolidmechanics2.cpp:1061); (n, m) and
+// (m, n) sum the same records in the same order, so the matrix is exactly symmetric.
 
 #include <hipcub/hipcub.hpp>
 
@@ -35,233 +33,444 @@ using namespace dev;
 constexpr int kMaxAdj = 64;   // elements around one node
 constexpr int kMaxNB = 128;   // nodes coupled to one node (column blocks of its rows)
 
-// Staging record layout (doubles) per element:
-//   Tet10, Tet10/P1:  G [NGP][NPE][4]  g_a (3) and a zero (two 16-byte groups per node)
-//   Hex8:      J [NGP][9]       the inverse Jacobian (g_a = grad_jinv(J, dN_a/dxi))
-//   B  [NGP][6]        b00 b11 b22 b01 b02 b12 (b g formed on use; Tet10/P1 records 248 doubles
-//                      instead of 304 with b g stored, Hex8 184 instead of 448)
-//   S  [NGP][SS]       displacement elements: s1..s5 (SS = 5); mixed elements: s1..s4, dv, dv0,
-//                      thetahat, resip (SS = 8)
-//   W  [26]            Hex8 Q1/P0 only: Kup [NPE][3], Kpp, 0 (the static condensation's coupling)
-//   R  [NPE][3]        element residual (no lift; Q1/P0: condensed, Fu - Kup Fp / Kpp)
-// The first SL doubles (G or J, B, S, W) are what the matrix kernel reads for a block.
+// Element record (doubles).  Node pairs by the distance d = (b - a) mod NPE of their local indices:
+//   U  [NPE][H][9]   block (a, (a + d) mod NPE), d < H = NPE / 2, row-major 3x3: the H blocks of a node are
+//                    contiguous, so that a row of the matrix reads few lines of each element
+//      [NPE / 2][9]  block (a, a + H), a < H; block (b, a) of a stored (a, b) is its transpose
+//   Q  [NPE][4][3]   Tet10/P1: Kup(3a + i, q); Kpu is its transpose
+//   P  [4][4]        Tet10/P1: Kpp
+//   R  [NPE][3]      residual, and RP [4] the pressure rows' (Tet10/P1); lift included on a first
+//                    iteration.  Q1/P0: condensed, Fu - Kup Fp / Kpp, as its blocks are
 // MIXED with NPE = 8 is the Hex8 Q1/P0 element (one pressure per element, condensed; the system has
 // displacement rows only), with NPE = 10 the Tet10/P1 element (pressure rows on the corner nodes).
-template <int NPE, int NGP, bool MIXED>
-struct Stage {
+// Records and their two parts are multiples of 128 bytes (a line completed at different times reaches memory
+// twice): 352 doubles Hex8, 544 Tet10, 688 Tet10/P1.
+template <int NPE, bool MIXED>
+struct Rec {
   static constexpr bool P0 = MIXED && NPE == 8;
   static constexpr bool P1 = MIXED && NPE != 8;
-  static constexpr bool COMPACT = NPE == 8;      // g formed from the inverse Jacobian
-  static constexpr int GW = COMPACT ? 3 : 4;      // doubles per node and Gauss point of g (LDS copies, Tet10 records)
-  static constexpr int SS = MIXED ? 8 : 5;
-  static constexpr int G0 = 0;
-  static constexpr int B0 = COMPACT ? NGP * 9 : NGP * NPE * GW;
-  static constexpr int S0 = B0 + NGP * 6;
-  static constexpr int W0 = S0 + NGP * SS;
-  static constexpr int WN = P0 ? 26 : 0;
-  static constexpr int R0 = W0 + WN;
-  static constexpr int SL = R0;
-  static constexpr int TS = ((R0 + NPE * 3) + 7) / 8 * 8;
-  static_assert(B0 % 2 == 0 && S0 % 2 == 0 && W0 % 2 == 0 && SL % 2 == 0, "16-byte groups");
+  static constexpr int H = NPE / 2;
+  static constexpr int ROW = H * 9;                         // a node's stored blocks
+  static constexpr int UN = NPE * ROW;
+  static constexpr int T0 = (UN + 15) / 16 * 16;            // then pairs (a, a + H), Q, P, R, RP
+  static constexpr int Q0 = T0 + (H * 9 + 1) / 2 * 2;
+  static constexpr int P0f = Q0 + (P1 ? NPE * 12 : 0);
+  static constexpr int R0 = P0f + (P1 ? 16 : 0);
+  static constexpr int RP0 = R0 + NPE * 3;
+  static constexpr int TN = (RP0 + (P1 ? 4 : 0) - T0 + 1) / 2 * 2;  // its length
+  static constexpr int TS = (T0 + TN + 15) / 16 * 16;
+  static_assert(UN % 2 == 0 && TN % 2 == 0, "16-byte groups");
 };
 
-// Hex8 Q1/P0: the static condensation's part of block (a, b), -Kup_a Kup_b^T / Kpp
-// (Elem_Solid_3D_Mixed0.cpp:93-104), from the record's W
-__device__ __forceinline__ void add_condensed(const double* W, int a, int b, double Kb[9]) {
-  const double kpp = W[24];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) Kb[3 * i + j] = Kb[3 * i + j] - W[3 * a + i] * (W[3 * b + j] / kpp);
+// Where block (a, b) of a record starts, and whether the stored block is its transpose.
+template <int NPE, bool MIXED>
+__device__ __forceinline__ int pair_slot(int a, int b, bool& tr) {
+  constexpr int H = NPE / 2;
+  int d = b - a;
+  if (d < 0) d += NPE;
+  tr = d > H || (d == H && a >= H);
+  const int dd = tr ? NPE - d : d, aa = tr ? b : a;
+  return dd < H ? (aa * H + dd) * 9 : Rec<NPE, MIXED>::T0 + aa * 9;
 }
 
-// g, b g of node c at Gauss point gp from a staging record, either layout
-// (dN: Hex8 dN/dxi table [NGP][NPE][3], e.g. in LDS; null: computed here)
-template <int NPE, int NGP, bool MIXED>
-__device__ __forceinline__ void record_g(const double* rec, int gp, int c, double g[3], double bg[3],
-                                         const double* dN = nullptr) {
-  using St = Stage<NPE, NGP, MIXED>;
-  if (St::COMPACT) {
-    double d[3];
-    if (dN) {
-      d[0] = dN[3 * (gp * NPE + c)]; d[1] = dN[3 * (gp * NPE + c) + 1]; d[2] = dN[3 * (gp * NPE + c) + 2];
-    } else {
-      hex8_dN_node(gp, c, d);
+// Gauss-point data of one element in LDS, per point: g of every node by component ([3][NPE], so that the
+// lanes (element, node) of a wavefront read consecutive addresses), the six components of b, the
+// tangent scalars (s1..s5; mixed s1..s4, dv, dv0, thetahat, resip), and the residual's tensor T (dv sigma, six
+// components; with the lift nine, not symmetric, and the mixed element's div of the lift).
+template <int NPE, bool MIXED, bool LIFT, int NGP>
+struct GaussLds {
+  static constexpr int SS = MIXED ? 8 : 5;
+  static constexpr int B0 = 3 * NPE, S0 = B0 + 6, T0 = S0 + SS;
+  static constexpr int PER = T0 + (LIFT ? (MIXED ? 10 : 9) : 6);
+  // element stride: the elements of half a wavefront start on different LDS banks
+  static constexpr int pad(int n) {
+    while (n % 32 != NPE && n % 32 != 32 - NPE) ++n;
+    return n;
+  }
+  static constexpr int SLP = pad(NGP * PER);
+};
+
+// Element kernel.  A workgroup takes EPB elements; lane (element, Gauss point) runs the geometry and the
+// material (gauss_state) and puts its point's data in LDS.  Then two groups of lanes (element, node a)
+// accumulate over the Gauss points in order: the first the pair blocks of the shorter distances and the
+// residual, the second the other distances and the couplings (one lane with all of a node's blocks keeps so
+// many registers that a compute unit holds two thirds of the wavefronts).  The records then go through LDS
+// to memory as 16-byte stores of whole contiguous lines.
+//   BLOCKS = false: only R (and RP) of the records (a residual assembly), one group of lanes.
+//   LIFT: the residual also loses K_e times the prescribed increments (dispApplied on prescribed dofs): with
+//     H_ki = sum_b ubar_b,k g_b,i per Gauss point it is T += s1 H^T + (s2 tr H + s3 b:H) I + s3 tr(H) b + s4 H b + s5 H.
+// Bound by FP64 arithmetic (about 30 kFLOP a Hex8 element: 1.6 of its 3.1 ms on 128^3) and, Tet10, by the record writes
+// (7.1 GB in 2.5 ms on 60^3 x 6).
+template <int NPE, bool MIXED>
+struct ElemSplit {
+  static constexpr int ND = NPE / 2 + 1;
+  static constexpr int DH = NPE == 8 ? 2 : 3;  // distances of the first group
+  static constexpr int NA = DH > ND - DH ? DH : ND - DH;
+};
+
+template <int NPE, bool MIXED>
+struct NodeSums {
+  double acc[ElemSplit<NPE, MIXED>::NA][9];
+  double r[3], rp;                  // residual, pressure row (first group)
+  double up[12], pp[4];             // Tet10/P1 couplings (second group)
+  double kup[3], kpp, fp, fpl;      // Q1/P0 (both groups)
+};
+
+// Node a's sums over the NG Gauss points whose data starts at o (element stride applied): distances D0 <= d < D1.
+template <int NPE, bool MIXED, bool LIFT, int NG, int D0, int D1, bool RES, bool COUP>
+__device__ __forceinline__ void node_sums(const double* o, int a, NodeSums<NPE, MIXED>& N) {
+  using Rc = Rec<NPE, MIXED>;
+  using Gl = GaussLds<NPE, MIXED, LIFT, NG>;
+  constexpr int H = Rc::H;
+#pragma unroll
+  for (int d = 0; d < D1 - D0; ++d)
+#pragma unroll
+    for (int t = 0; t < 9; ++t) N.acc[d][t] = 0.0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) N.r[i] = N.kup[i] = 0.0;
+#pragma unroll
+  for (int i = 0; i < 12; ++i) N.up[i] = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) N.pp[i] = 0.0;
+  N.rp = N.kpp = N.fp = N.fpl = 0.0;
+#pragma unroll 1
+  for (int gp = 0; gp < NG; ++gp, o += Gl::PER) {
+    const double ga[3] = {o[a], o[NPE + a], o[2 * NPE + a]};
+    const double* S = o + Gl::S0;
+    const double* t = o + Gl::T0;
+    if constexpr (RES) {
+      if constexpr (LIFT) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) N.r[i] -= t[3 * i] * ga[0] + t[3 * i + 1] * ga[1] + t[3 * i + 2] * ga[2];
+      } else {
+        N.r[0] -= t[0] * ga[0] + t[3] * ga[1] + t[4] * ga[2];
+        N.r[1] -= t[3] * ga[0] + t[1] * ga[1] + t[5] * ga[2];
+        N.r[2] -= t[4] * ga[0] + t[5] * ga[1] + t[2] * ga[2];
+      }
     }
-    grad_jinv(rec + St::G0 + gp * 9, d, g);
-    bsym_times(rec + St::B0 + gp * 6, g, bg);
-  } else {
-    const double* p = rec + St::G0 + (gp * NPE + c) * St::GW;
-    g[0] = p[0]; g[1] = p[1]; g[2] = p[2];
-    bsym_times(rec + St::B0 + gp * 6, g, bg);
-  }
-}
-
-// 3x3 tangent block (a, b) of one element from its staging record, either layout
-template <int NPE, int NGP, bool MIXED>
-__device__ __forceinline__ void record_block(const double* rec, int a, int b, double Kb[9],
-                                             const double* dN = nullptr) {
-  using St = Stage<NPE, NGP, MIXED>;
+    if constexpr (D1 > D0) {
+      double B6[6], ba[3];
 #pragma unroll
-  for (int t = 0; t < 9; ++t) Kb[t] = 0.0;
-#pragma unroll 2
-  for (int gp = 0; gp < NGP; ++gp) {
-    double ga[3], ba[3], gb[3], bb[3];
-    record_g<NPE, NGP, MIXED>(rec, gp, a, ga, ba, dN);
-    record_g<NPE, NGP, MIXED>(rec, gp, b, gb, bb, dN);
-    const double* S = rec + St::S0 + gp * St::SS;
-    tangent_gp<!MIXED>(ga, ba, gb, bb, S[0], S[1], S[2], S[3], MIXED ? 0.0 : S[4], Kb);
+      for (int q = 0; q < 6; ++q) B6[q] = o[Gl::B0 + q];
+      bsym_times(B6, ga, ba);
+      const double s1 = S[0], s2 = S[1], s3 = S[2], s4 = S[3], s5 = MIXED ? 0.0 : S[4];
+#pragma unroll
+      for (int d = D0; d < D1; ++d) {
+        if (d == H && a >= H) continue;
+        int b = a + d;
+        if (b >= NPE) b -= NPE;
+        const double gb[3] = {o[b], o[NPE + b], o[2 * NPE + b]};
+        double bb[3];
+        bsym_times(B6, gb, bb);
+        tangent_gp<!MIXED>(ga, ba, gb, bb, s1, s2, s3, s4, s5, N.acc[d - D0]);
+      }
+    }
+    if constexpr (Rc::P1 && (RES || COUP)) {  // ElementBase2.cpp:500-539
+      double Np[4];
+      tet_Np(gp, Np);
+      const double Na = a == 0 ? Np[0] : a == 1 ? Np[1] : a == 2 ? Np[2] : Np[3];
+      const double dv = S[4], dv0 = S[5], th = S[6], resip = S[7];
+      if constexpr (RES) {
+        if (a < 4) {
+          N.rp -= (dv0 * Na) * resip;
+          if constexpr (LIFT) N.rp -= (dv * Na) * t[9];
+        }
+      }
+      if constexpr (COUP) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const double b1 = dv * ga[i];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) N.up[3 * q + i] += b1 * Np[q];
+        }
+        if (a < 4) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) N.pp[q] -= ((dv0 * Na) * th) * Np[q];
+        }
+      }
+    }
+    if constexpr (Rc::P0) {  // Kup_a = sum dv g_a, Kpp = -sum dv0 thetahat, Fp = -sum dv0 resip (Np = 1)
+      const double dv = S[4], dv0 = S[5];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) N.kup[i] += dv * ga[i];
+      N.kpp -= dv0 * S[6];
+      if constexpr (RES) {
+        N.fp -= dv0 * S[7];
+        if constexpr (LIFT) N.fpl += dv * t[9];
+      }
+    }
   }
-  if (St::P0) add_condensed(rec + St::W0, a, b, Kb);
 }
 
-// Stage kernel.  OUT_LDS: the wavefront's EPW records are written to LDS and then copied to the
-// staging array, which holds them contiguously, with 16-byte stores that each cover 1 KiB (written
-// directly, every lane's stores land 8 bytes apiece on 64 different cache lines).  Measured per
-// assembly: Hex8 128^3 8.81 ms through LDS vs 9.53 ms direct; Tet10/P1 60^3x6 8.94 vs 9.08 ms.
-#ifndef MPF_STAGE_LDS_HEX
-#define MPF_STAGE_LDS_HEX 1
-#endif
-#ifndef MPF_STAGE_LDS_TET
-#define MPF_STAGE_LDS_TET 1
-#endif
-// Q1/P0 (qKup, qKpp, qFp non-null): each element's Kup [24], Kpp and Fp also go to these arrays for
-// the pressure recovery after the solve.
-template <int NPE, int NGP, bool MIXED, int EPW, bool OUT_LDS>
-__global__ void __launch_bounds__(64) k_stage(ElemArgs A, int32_t nElem, double* __restrict__ GS,
-                                              double* __restrict__ qKup, double* __restrict__ qKpp,
-                                              double* __restrict__ qFp) {
-  static_assert(EPW * NGP == 64, "one wavefront holds EPW elements x NGP Gauss points");
-  using St = Stage<NPE, NGP, MIXED>;
-  static_assert(St::TS % 2 == 0, "16-byte records");
-  static_assert(!St::P0 || NGP == NPE, "Q1/P0: one node per Gauss-point lane in the condensation");
-  __shared__ double sX[EPW][NPE][3], sU[EPW][NPE][3], sUP[MIXED ? EPW : 1][NPE][3], sP[EPW][4];
+// Q1/P0: the condensation's share of the group's blocks (Elem_Solid_3D_Mixed0.cpp:93-104), from every
+// node's Kup of the element at kup.
+template <int NPE, bool MIXED, int D0, int D1>
+__device__ __forceinline__ void condense_blocks(const double* kup, int a, NodeSums<NPE, MIXED>& N) {
+#pragma unroll
+  for (int d = D0; d < D1; ++d) {
+    if (d == NPE / 2 && a >= NPE / 2) continue;
+    int b = a + d;
+    if (b >= NPE) b -= NPE;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const double w = kup[3 * b + j] / N.kpp;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) N.acc[d - D0][3 * i + j] -= N.kup[i] * w;
+    }
+  }
+}
+
+template <int NPE, int NGP, bool MIXED, int EPB, bool BLOCKS, bool LIFT>
+__global__ void __launch_bounds__((EPB * NPE + 63) / 64 * 64 * (BLOCKS ? 2 : 1))
+    __attribute__((amdgpu_waves_per_eu(BLOCKS ? 3 : 2)))
+    k_elem_records(ElemArgs A, int32_t nElem, const double* __restrict__ dispApplied,
+                   const int32_t* __restrict__ nodeinfo, double* __restrict__ KE, double* __restrict__ qKup,
+                   double* __restrict__ qKpp, double* __restrict__ qFp) {
+  using Rc = Rec<NPE, MIXED>;
+  using Gl = GaussLds<NPE, MIXED, LIFT, NGP>;
+  using Sp = ElemSplit<NPE, MIXED>;
+  constexpr int NL = EPB * NGP, NC = EPB * NPE, GRP = (NC + 63) / 64 * 64, WG = GRP * (BLOCKS ? 2 : 1);
+  static_assert(NL <= WG, "Gauss-point lanes");
+  constexpr int H = Rc::H, ND = Sp::ND, DH = Sp::DH;
+  constexpr int FLD = (MIXED ? 3 : 2) + (LIFT ? 1 : 0);  // nodal fields: X, u, (u_prev), (ubar)
+  constexpr int ER = NPE == 8 ? EPB : EPB / 2;  // elements whose blocks go out together
+  static_assert(EPB % ER == 0, "rounds");
+  constexpr int nU = ER * Rc::UN, nT = EPB * Rc::TN, nOut = nU > nT ? nU : nT;
+  constexpr int n1 = EPB * Gl::SLP, n2 = BLOCKS ? nOut : 0, n3 = EPB * (FLD * NPE * 3 + 4);
+  constexpr int n12 = n1 > n2 ? n1 : n2, NS = n12 > n3 ? n12 : n3;
+  __shared__ double2 sm2[(NS + 1) / 2];
   __shared__ double sdN[NGP][3][NPE];
-  __shared__ double2 sOut[OUT_LDS ? EPW * St::TS / 2 : 1];
-  __shared__ double sQ[St::P0 ? EPW * NGP * 26 : 1];  // per lane: dv g_a (24), -dv0 thetahat, -dv0 resip
-  const int lane = threadIdx.x;
-  const int base = blockIdx.x * EPW;
-  if (lane < NGP) {
+  double* const sm = reinterpret_cast<double*>(sm2);
+  const int tid = threadIdx.x;
+  const int base = blockIdx.x * EPB;
+  if (tid < NGP) {
     double d[3][NPE];
     if (NPE == 8) {
-      hex8_dN(lane, (double(*)[8])d);
+      hex8_dN(tid, (double(*)[8])d);
     } else {
       double x1, x2, x3;
-      tet_gp(lane, x1, x2, x3);
+      tet_gp(tid, x1, x2, x3);
       tet10_dN(x1, x2, x3, (double*)d[0], (double*)d[1], (double*)d[2]);
     }
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
-      for (int a = 0; a < NPE; ++a) sdN[lane][r][a] = d[r][a];
+      for (int a = 0; a < NPE; ++a) sdN[tid][r][a] = d[r][a];
   }
-  {
-    // the wavefront's (element, node) pairs, NT per lane: every connectivity load issued, then every
-    // node-data load, then the LDS stores (two round trips to memory instead of two per pair)
-    constexpr int NT = (EPW * NPE + 63) / 64;
-    size_t nd[NT];
-    int ev[NT];
+  // nodal data, one (element, node) pair per lane: sm as [field][element][node][3], then the pressures
+  constexpr int FS = EPB * NPE * 3;
+  double* const sP = sm + FLD * FS;
+  if (tid < NC) {
+    const int k = tid / NPE, a = tid - k * NPE;
+    const int e = base + k < nElem ? base + k : base;  // idle slots repeat the first element
+    const size_t nd = (size_t)A.conn[(size_t)e * NPE + a];
+    const int info = LIFT ? nodeinfo[nd] : 0;
+    double v[FLD][3], pv = 0.0;
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int t = lane + 64 * i, k = t / NPE, a = t % NPE;
-      ev[i] = (base + k < nElem) ? base + k : base;  // idle slots repeat the first element
-      nd[i] = t < EPW * NPE ? (size_t)A.conn[(size_t)ev[i] * NPE + a] : 0;
+    for (int c = 0; c < 3; ++c) {
+      v[0][c] = A.X[3 * nd + c];
+      v[1][c] = A.u[3 * nd + c];
+      if constexpr (MIXED) v[2][c] = A.uprev[3 * nd + c];
+      if constexpr (LIFT) v[FLD - 1][c] = ((info >> c) & 1) ? 0.0 : dispApplied[3 * nd + c];
     }
-    double xv[NT][3], uv[NT][3], upv[NT][3], pv[NT];
+    if (Rc::P1 && a < 4) pv = A.pres[nd];
+    if (Rc::P0 && a == 0) pv = A.pres[e];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int t = lane + 64 * i, a = t % NPE;
-      const bool on = t < EPW * NPE;
+    for (int f = 0; f < FLD; ++f)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        xv[i][c] = on ? A.X[3 * nd[i] + c] : 0.0;
-        uv[i][c] = on ? A.u[3 * nd[i] + c] : 0.0;
-        upv[i][c] = (MIXED && on) ? A.uprev[3 * nd[i] + c] : 0.0;
+      for (int c = 0; c < 3; ++c) sm[f * FS + tid * 3 + c] = v[f][c];
+    if (Rc::P1 && a < 4) sP[4 * k + a] = pv;
+    if (Rc::P0 && a == 0) sP[4 * k] = pv;
+  }
+  __syncthreads();
+  const int sk = tid / NGP, sgp = tid % NGP;
+  const bool stage = tid < NL;
+  GaussState Q;
+  double T[9], trH = 0.0;  // T: residual tensor (row i, column m)
+  if (stage) {
+    const int e = base + sk < nElem ? base + sk : base;
+    const double wgp = (NPE == 8) ? 1.0 : 0.2500000000000000 * (1.0 / 6.0);  // QuadratureUtil.cpp:466-492, 706-709
+    double mu, K;
+    elem_material(A, e, mu, K);
+    const auto field = [&](int f) { return reinterpret_cast<const double(*)[3]>(sm + f * FS + sk * NPE * 3); };
+    gauss_state<NPE, NGP, MIXED, 2>(field(0), field(1), MIXED ? field(2) : nullptr, MIXED ? sP + 4 * sk : nullptr,
+                                 sdN[sgp], sgp, wgp, mu, K, A.Utype, Rc::P0 ? false : A.consistent != 0, Q);
+    if (Q.negJ && base + sk < nElem) flag_bad(A.bad, e);
+    const NHPoint& P = Q.nh;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int m = 0; m < 3; ++m) T[3 * i + m] = Q.dv * P.sig[i][m];
+    if constexpr (LIFT) {
+      const double(*ub)[3] = field(FLD - 1);
+      double Hh[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};  // Hh[k][i]
+      bool any = false;
+#pragma unroll
+      for (int a = 0; a < NPE; ++a) any = any || ub[a][0] != 0.0 || ub[a][1] != 0.0 || ub[a][2] != 0.0;
+      if (any) {
+#pragma unroll 2
+        for (int a = 0; a < NPE; ++a) {
+          double g[3];
+          const double da[3] = {sdN[sgp][0][a], sdN[sgp][1][a], sdN[sgp][2][a]};
+          grad_jinv(&Q.Bi[0][0], da, g);
+#pragma unroll
+          for (int kk = 0; kk < 3; ++kk)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) Hh[kk][i] += ub[a][kk] * g[i];
+        }
+        trH = Hh[0][0] + Hh[1][1] + Hh[2][2];
+        double bH = 0.0;
+#pragma unroll
+        for (int kk = 0; kk < 3; ++kk)
+#pragma unroll
+          for (int l = 0; l < 3; ++l) bH += P.b[kk][l] * Hh[kk][l];
+        const double iso = P.s2 * trH + P.s3 * bH;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int m = 0; m < 3; ++m) {
+            const double hb = Hh[i][0] * P.b[0][m] + Hh[i][1] * P.b[1][m] + Hh[i][2] * P.b[2][m];
+            T[3 * i + m] += P.s1 * Hh[m][i] + P.s3 * trH * P.b[i][m] + P.s4 * hb + P.s5 * Hh[i][m] + (i == m ? iso : 0.0);
+          }
       }
-      pv[i] = 0.0;
-      if (St::P1 && on && a < 4) pv[i] = A.pres[nd[i]];
-      if (St::P0 && on && a == 0) pv[i] = A.pres[ev[i]];
-    }
-#pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const int t = lane + 64 * i, k = t / NPE, a = t % NPE;
-      if (t >= EPW * NPE) continue;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        sX[k][a][c] = xv[i][c];
-        sU[k][a][c] = uv[i][c];
-        if (MIXED) sUP[k][a][c] = upv[i][c];
-      }
-      if (St::P1 && a < 4) sP[k][a] = pv[i];
-      if (St::P0 && a == 0) sP[k][0] = pv[i];
     }
   }
   __syncthreads();
-  const int k = lane / NGP, gp = lane % NGP;
-  const int e = base + k;
-  const bool writer = e < nElem;
-  double* rec = OUT_LDS ? reinterpret_cast<double*>(sOut) + k * St::TS : GS + (size_t)(writer ? e : base) * St::TS;
-  const double wgp = (NPE == 8) ? 1.0 : 0.2500000000000000 * (1.0 / 6.0);  // QuadratureUtil.cpp:466-492, 706-709
-  bool negJ = false;
-  double mu, K;
-  elem_material(A, writer ? e : base, mu, K);
-  element_point<NPE, NGP, MIXED, St::COMPACT, !St::COMPACT>(sX[k], sU[k], MIXED ? sUP[k] : nullptr, MIXED ? sP[k] : nullptr, sdN[gp],
-                                              gp, wgp, mu, K, A.Utype, St::P0 ? false : A.consistent != 0, writer,
-                                              rec + St::G0 + gp * (St::COMPACT ? 9 : NPE * St::GW),
-                                              rec + St::S0 + gp * St::SS, rec + St::R0, negJ, rec + St::B0 + gp * 6);
-  if (writer && negJ) flag_bad(A.bad, e);
-  if constexpr (St::P0) {
-    // Kup_a = sum_gp dv g_a (ElementBase2.cpp:500-505 with Np = 1), Kpp = -sum_gp dv0 thetahat,
-    // Fp = -sum_gp dv0 resip (:510-539), each summed in Gauss-point order by the lane of node a = gp;
-    // g_a from this lane's inverse Jacobian as element_point formed it
-    const double* Sg = rec + St::S0 + gp * St::SS;
-    double* q = sQ + (size_t)lane * 26;
-    double Jr[9];
+  if (stage) {
+    double* o = sm + sk * Gl::SLP + sgp * Gl::PER;
 #pragma unroll
-    for (int i = 0; i < 9; ++i) Jr[i] = rec[St::G0 + gp * 9 + i];
-    const double dv = Sg[4], dv0 = Sg[5];
-#pragma unroll
-    for (int a = 0; a < NPE; ++a) {
+    for (int c = 0; c < NPE; ++c) {
       double g[3];
-      const double da[3] = {sdN[gp][0][a], sdN[gp][1][a], sdN[gp][2][a]};
-      grad_jinv(Jr, da, g);
-      q[3 * a] = dv * g[0]; q[3 * a + 1] = dv * g[1]; q[3 * a + 2] = dv * g[2];
+      const double dc[3] = {sdN[sgp][0][c], sdN[sgp][1][c], sdN[sgp][2][c]};
+      grad_jinv(&Q.Bi[0][0], dc, g);
+      o[c] = g[0]; o[NPE + c] = g[1]; o[2 * NPE + c] = g[2];
     }
-    q[24] = dv0 * Sg[6];
-    q[25] = dv0 * Sg[7];
-    __syncthreads();
-    const int a = gp;
-    const double* q0 = sQ + (size_t)k * NGP * 26;
-    double u3[3] = {0.0, 0.0, 0.0}, kpp = 0.0, fp = 0.0;
-    for (int g2 = 0; g2 < NGP; ++g2) {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) u3[i] += q0[g2 * 26 + 3 * a + i];
-      fp -= q0[g2 * 26 + 25];
-      kpp -= q0[g2 * 26 + 24];
+    const NHPoint& P = Q.nh;
+    double* B = o + Gl::B0;
+    B[0] = P.b[0][0]; B[1] = P.b[1][1]; B[2] = P.b[2][2];
+    B[3] = P.b[0][1]; B[4] = P.b[0][2]; B[5] = P.b[1][2];
+    double* S = o + Gl::S0;
+    S[0] = P.s1; S[1] = P.s2; S[2] = P.s3; S[3] = P.s4;
+    if constexpr (MIXED) {
+      S[4] = Q.dv; S[5] = Q.dv0; S[6] = Q.thetahat; S[7] = Q.resip;
+    } else {
+      S[4] = P.s5;
     }
-    if (writer) {
-      double* W = rec + St::W0;
-      double* R = rec + St::R0;
-      const double fps = fp / kpp;
+    double* t = o + Gl::T0;
+    if constexpr (LIFT) {
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        W[3 * a + i] = u3[i];
-        R[3 * a + i] = R[3 * a + i] - u3[i] * fps;  // the lane that wrote node a's residual (a = gp)
-        qKup[(size_t)e * 24 + 3 * a + i] = u3[i];
-      }
-      if (a == 0) {
-        W[24] = kpp;
-        W[25] = 0.0;
-        qKpp[e] = kpp;
-        qFp[e] = fp;
-      }
+      for (int i = 0; i < 9; ++i) t[i] = T[i];
+      if constexpr (MIXED) t[9] = trH;
+    } else {
+      t[0] = T[0]; t[1] = T[4]; t[2] = T[8]; t[3] = T[1]; t[4] = T[2]; t[5] = T[5];
     }
   }
-  if (OUT_LDS) {
+  __syncthreads();
+  const bool second = BLOCKS && tid >= GRP;  // uniform per wavefront
+  const int ct = second ? tid - GRP : tid;
+  const int k = ct / NPE, a = ct - k * NPE;
+  const bool comp = ct < NC, live = comp && base + k < nElem;
+  NodeSums<NPE, MIXED> N;
+  if (comp) {
+    const double* o = sm + k * Gl::SLP;
+    if constexpr (!BLOCKS) node_sums<NPE, MIXED, LIFT, NGP, 0, 0, true, false>(o, a, N);
+    else if (!second) node_sums<NPE, MIXED, LIFT, NGP, 0, DH, true, false>(o, a, N);
+    else node_sums<NPE, MIXED, LIFT, NGP, DH, ND, false, true>(o, a, N);
+  }
+  __syncthreads();
+  if constexpr (Rc::P0) {
+    if (comp && !second) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) sm[ct * 3 + i] = N.kup[i];
+    }
     __syncthreads();
-    const int nv = nElem - base < EPW ? nElem - base : EPW;
-    double2* dst = reinterpret_cast<double2*>(GS + (size_t)base * St::TS);
-    for (int t = lane; t < nv * (St::TS / 2); t += 64) dst[t] = sOut[t];
+    if (comp) {
+      const double* kup = sm + k * NPE * 3;
+      if (!second) {  // the lift takes Kpu ubar from the pressure equation
+        const double fps = (LIFT ? N.fp - N.fpl : N.fp) / N.kpp;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) N.r[i] = N.r[i] - N.kup[i] * fps;
+        if (live) {
+          const size_t e = (size_t)(base + k);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) qKup[e * 24 + 3 * a + i] = N.kup[i];
+          if (a == 0) { qKpp[e] = N.kpp; qFp[e] = N.fp; }
+        }
+        if constexpr (BLOCKS) condense_blocks<NPE, MIXED, 0, DH>(kup, a, N);
+      } else {
+        condense_blocks<NPE, MIXED, DH, ND>(kup, a, N);
+      }
+    }
+    __syncthreads();
+  }
+  if constexpr (!BLOCKS) {
+    if (live) {
+      double* o = KE + (size_t)(base + k) * Rc::TS;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) o[Rc::R0 + 3 * a + i] = N.r[i];
+      if (Rc::P1 && a < 4) o[Rc::RP0 + a] = N.rp;
+    }
+  } else {
+    // self blocks: their (i, k) and (k, i) entries agree to rounding; the mean makes them exactly symmetric
+    if (!second) {
+      double* c = N.acc[0];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = i + 1; j < 3; ++j) c[3 * i + j] = c[3 * j + i] = 0.5 * (c[3 * i + j] + c[3 * j + i]);
+    }
+    const int nv = nElem - base < EPB ? nElem - base : EPB;
+    // out: n2w 16-byte groups of each of elements k0 .. k1 - 1, contiguous in LDS, to the records' offset off
+    const auto copy_out = [&](int k0, int k1, int n2w, int off) {
+      const int kn = min(k1, nv) - k0;
+      for (int t = tid; t < kn * n2w; t += WG) {
+        const int kk = t / n2w, c = t - kk * n2w;
+        reinterpret_cast<double2*>(KE + (size_t)(base + k0 + kk) * Rc::TS + off)[c] = sm2[t];
+      }
+    };
+#pragma unroll
+    for (int k0 = 0; k0 < EPB; k0 += ER) {
+      if (comp && k >= k0 && k < k0 + ER) {
+        double* o = sm + (k - k0) * Rc::UN + a * Rc::ROW;
+        if (second) {
+#pragma unroll
+          for (int d = DH; d < H; ++d)
+#pragma unroll
+            for (int t = 0; t < 9; ++t) o[d * 9 + t] = N.acc[d - DH][t];
+        } else {
+#pragma unroll
+          for (int d = 0; d < DH; ++d)
+#pragma unroll
+            for (int t = 0; t < 9; ++t) o[d * 9 + t] = N.acc[d][t];
+        }
+      }
+      __syncthreads();
+      copy_out(k0, k0 + ER, Rc::UN / 2, 0);
+      __syncthreads();
+    }
+    if (comp) {
+      double* o = sm + k * Rc::TN - Rc::T0;
+      if (second) {
+        if (a < H) {
+#pragma unroll
+          for (int t = 0; t < 9; ++t) o[Rc::T0 + a * 9 + t] = N.acc[H - DH][t];
+        }
+        if constexpr (Rc::P1) {
+#pragma unroll
+          for (int t = 0; t < 12; ++t) o[Rc::Q0 + a * 12 + t] = N.up[t];
+          if (a < 4) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[Rc::P0f + 4 * a + q] = N.pp[q];
+          }
+        }
+      } else {
+        if (Rc::P1 && a < 4) o[Rc::RP0 + a] = N.rp;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) o[Rc::R0 + 3 * a + i] = N.r[i];
+      }
+    }
+    __syncthreads();
+    copy_out(0, EPB, Rc::TN / 2, Rc::T0);
   }
 }
 
@@ -335,10 +544,6 @@ __device__ __forceinline__ void wave_sort(int32_t* key, int n, int lane) {
 constexpr int kItemCap = 1024;   // kMaxAdj * NPE rounded up to a power of two (Tet10: 640 -> 1024)
 constexpr int kGroupNodes = 8;   // nodes per layout group (consecutive in Morton order)
 
-// Block ownership.  K is symmetric (K_e(a, b) = K_e(b, a)^T for every element: the Neo-Hookean
-// tangent and the u-p couplings alike), so the pair of blocks (n, m), (m, n) is summed once, by its
-// owner, which writes K_nm into n's rows and its transpose into m's rows.  n owns (n, m) if m is n,
-// or m has no rows, or n < m.  Only nodes with rows own anything.
 template <bool MIXED>
 __device__ __forceinline__ bool has_rows(int info) {
   return (info & 7) || (MIXED && ((info >> 3) & 1));
@@ -346,12 +551,11 @@ __device__ __forceinline__ bool has_rows(int info) {
 
 // Build step 1 (one wavefront per node n):
 //   nelA[nptr[n] + s]       = e * 16 + a: the elements around n in ascending id, a = local index of n in e
-//   keys[nptr[n] * NPE + t] = (s0 << 23) | (j << 16) | (s << 4) | b for every element s around n and
-//                             node b of it such that n owns the block pair (n, conn[e][b]), sorted:
-//                             j = position of node conn[e][b] in the sorted coupled-node list of n (the
-//                             column block of n's rows the (s, b) block lands in), s0 = first element of
-//                             column j's run
+//   keys[nptr[n] * NPE + t] = (j << 16) | (s << 4) | b for every element s around n and node b of it that
+//                             has rows (and so columns), sorted: j = position of node conn[e][b] in the sorted
+//                             coupled-node list of n (the column block of n's rows the item adds to)
 //   cnt[n]                  = number of those items (0 for a node without rows)
+// overflow: 1 too many elements or coupled nodes, 2 inconsistent tables, 4 a node with rows in no element.
 template <int NPE, bool MIXED>
 __global__ void __launch_bounds__(64) k_node_items(int32_t nNode, const int32_t* __restrict__ nptr,
                                                    const int32_t* __restrict__ nel, const int32_t* __restrict__ nbptr,
@@ -382,6 +586,7 @@ __global__ void __launch_bounds__(64) k_node_items(int32_t nNode, const int32_t*
     nelA[e0 + lane] = sE[lane] * 16 + a;
   }
   const bool rows = has_rows<MIXED>(nodeinfo[n]);
+  if (rows && m == 0 && lane == 0) atomicOr(overflow, 4);
   const int nall = rows ? m * NPE : 0;
   int P2 = 64;
   while (P2 < nall) P2 <<= 1;
@@ -391,7 +596,7 @@ __global__ void __launch_bounds__(64) k_node_items(int32_t nNode, const int32_t*
     if (t < nall) {
       const int s = t / NPE, b = t % NPE;
       const int vb = conn[(size_t)sE[s] * NPE + b];
-      if (vb == n || !has_rows<MIXED>(nodeinfo[vb]) || n < vb) {
+      if (has_rows<MIXED>(nodeinfo[vb])) {
         int lo = 0, hi = nnb;
         while (lo < hi) {
           const int mid = (lo + hi) >> 1;
@@ -405,22 +610,10 @@ __global__ void __launch_bounds__(64) k_node_items(int32_t nNode, const int32_t*
     sK[t] = key;
   }
   for (int off = 32; off > 0; off >>= 1) own += __shfl_xor(own, off, 64);
-  const int nitems = own;
   __syncthreads();
   wave_sort(sK, P2, lane);
-  // Runs (columns) are laid out in order of their first element, so a wavefront's items come from
-  // few elements; within a run, items stay in element order.  key |= (first element of the run) << 23.
-  if (lane == 0) {
-    int first = 0;
-    for (int t = 0; t < nitems; ++t) {
-      if (t == 0 || ((sK[t] >> 16) & 127) != ((sK[t - 1] >> 16) & 127)) first = (sK[t] >> 4) & 63;
-      sK[t] |= first << 23;
-    }
-  }
-  __syncthreads();
-  wave_sort(sK, P2, lane);
-  for (int t = lane; t < nitems; t += 64) keys[(size_t)e0 * NPE + t] = sK[t];
-  if (lane == 0) cnt[n] = nitems;
+  for (int t = lane; t < own; t += 64) keys[(size_t)e0 * NPE + t] = sK[t];
+  if (lane == 0) cnt[n] = own;
 }
 
 // Layout walk over layout group g (nodes order[8g .. 8g+7]) and each node's sorted items: items are
@@ -466,97 +659,26 @@ __global__ void k_group_len(int64_t ngroups, int32_t nNode, const int32_t* __res
 
 // Build step 2b (one lane per layout group): the laid-out items,
 //   fitem[goff[g] + q] = {e * 16 + a, (blk << 4) | b}  (element e around node n, a = n's local index
-//   in e, blk = nbptr[n] + j the column block of n's rows node b of e lands in),
-//   fnode[goff[g] + q] = n; padding slots keep {-1, -1} and -1.
+//   in e, blk = nbptr[n] + j the column block of n's rows node b of e lands in), for step 4;
+//   padding slots, always at the end of a wavefront, keep {-1, -1}.
 template <int NPE>
 __global__ void k_group_fill(int64_t ngroups, int32_t nNode, const int32_t* __restrict__ order,
                              const int32_t* __restrict__ nptr, const int32_t* __restrict__ nbptr,
                              const int32_t* __restrict__ keys, const int64_t* __restrict__ cnt,
                              const int32_t* __restrict__ nelA, const int64_t* __restrict__ goff,
-                             int2* __restrict__ fitem, int32_t* __restrict__ fnode) {
+                             int2* __restrict__ fitem) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= ngroups) return;
   const int64_t base = goff[g];
   group_walk<NPE>(g, nNode, order, nptr, keys, cnt, [&](int64_t pos, int n, int, int32_t key) {
     const int blk = nbptr[n] + ((key >> 16) & 127);
     fitem[base + pos] = make_int2(nelA[nptr[n] + ((key >> 4) & 63)], (blk << 4) | (key & 15));
-    fnode[base + pos] = n;
   });
 }
 
-// Build step 2c (one lane per layout group): the group's wavefronts split into chunks of at most CW
-// (the chunked matrix kernel's workgroups); with count, only the number of chunks.
-__global__ void k_group_chunks(int64_t ngroups, int32_t CW, const int64_t* __restrict__ glen,
-                               const int64_t* __restrict__ goff, const int64_t* __restrict__ coff,
-                               int64_t* __restrict__ ccount, int32_t* __restrict__ cwave, int32_t* __restrict__ cnw) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ngroups) return;
-  const int64_t waves = glen[g] / 64;
-  const int64_t nch = (waves + CW - 1) / CW;
-  if (ccount) { ccount[g] = nch; return; }
-  for (int64_t k = 0; k < nch; ++k) {
-    cwave[coff[g] + k] = (int32_t)(goff[g] / 64 + k * CW);
-    cnw[coff[g] + k] = (int32_t)(waves - k * CW < CW ? waves - k * CW : CW);
-  }
-}
-
-// Build step 2d (one wavefront per laid-out wavefront): the order in which the lanes compute the
-// wavefront's items.  Lane L computes the item at run-order position fperm[64 w + L]; positions are
-// ranked by (element, local index of the row node, local index of the column node), padding last.
-// The run sums stay in run order; only which lane forms which block changes.  A vector load's
-// address processing takes one pass per distinct 128-byte line among each four consecutive lanes
-// (measured on MI355X: 16-byte loads take 64 cycles per wavefront when the four lanes of every quad
-// hit four lines, 16 when each quad stays in one line); in run order the lanes of a quad read four
-// different elements' records, in this order mostly the same element's.
-__global__ void __launch_bounds__(64) k_wave_perm(int64_t nwaves, const int2* __restrict__ fitem,
-                                                  uint8_t* __restrict__ fperm) {
-  const int64_t w = blockIdx.x;
-  if (w >= nwaves) return;
-  const int lane = threadIdx.x;
-  const int2 it = fitem[w * 64 + lane];
-  const long long key = it.x >= 0 ? ((long long)(it.x >> 4) << 8) | ((it.x & 15) << 4) | (it.y & 15)
-                                   : 0x7fffffffffffffffLL;
-  int rank = 0;
-  for (int j = 0; j < 64; ++j) {
-    const long long kj = __shfl(key, j, 64);
-    rank += (kj < key || (kj == key && j < lane)) ? 1 : 0;
-  }
-  fperm[w * 64 + rank] = (uint8_t)lane;
-}
-
-// Build step 3b (one wavefront per node n): for each column block (n, j) with coupled node m, the
-// entry of block (m, n) of m's rows, which receives its transpose when n owns the pair, is copied
-// next to (n, j)'s own entry, so that a run's head reads both with one load; {-1, 0, ..} when the
-// pair has no mirror (m is n, or m has no rows).  btab holds 2 BT ints per block.
-template <bool MIXED>
-__global__ void __launch_bounds__(64) k_mirror(int32_t nNode, const int32_t* __restrict__ nbptr,
-                                               const int32_t* __restrict__ nb, const int32_t* __restrict__ nodeinfo,
-                                               int32_t* __restrict__ btab) {
-  constexpr int BT = MIXED ? 4 : 2;
-  const int n = blockIdx.x;
-  if (n >= nNode) return;
-  const int b0 = nbptr[n], nnb = nbptr[n + 1] - b0;
-  for (int j = threadIdx.x; j < nnb; j += 64) {
-    const int mnode = nb[b0 + j];
-    int out = -1;
-    if (mnode != n && has_rows<MIXED>(nodeinfo[mnode])) {
-      int lo = nbptr[mnode], hi = nbptr[mnode + 1];
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (nb[mid] < n) lo = mid + 1; else hi = mid;
-      }
-      out = (lo < nbptr[mnode + 1] && nb[lo] == n) ? lo : -1;
-    }
-    int32_t* dst = btab + 2 * BT * (size_t)(b0 + j) + BT;
-#pragma unroll
-    for (int q = 0; q < BT; ++q) dst[q] = out >= 0 ? btab[2 * BT * (size_t)out + q] : (q == 0 ? -1 : 0);
-  }
-}
-
 // Build step 3 (one wavefront per node n): where each column block (n, j) of n's rows lives in the CSR,
-// the first BT of the block's 2 BT ints (the mirror's entry follows, step 3b).
-//   Hex8:      {A, (La << 9) | flags}                         (BT = 2)
-//   Tet10/P1:  {A, Bp, (D << 16) | La, flags}                 (BT = 4)
+//   displacement elements:  {A, (La << 9) | flags}
+//   Tet10/P1:               {A, Bp, (D << 16) | La, flags}
 //   flags = (self << 8) | (isPn << 7) | (isPb << 6) | (mn << 3) | mb
 // A = start of n's first free u row + column offset of j's u dofs (-1 if n has no free u dof),
 // Bp = the same in n's pressure row (-1 if n carries no pressure), D = offset of j's pressure column
@@ -607,13 +729,13 @@ __global__ void __launch_bounds__(64) k_block_table(int32_t nNode, const int32_t
       const int self = nb[b0 + j] == n;
       if (MIXED) {
         const int isPb = (inf >> 3) & 1;
-        btab[8 * blk] = RU >= 0 ? RU + upos : -1;
-        btab[8 * blk + 1] = RP >= 0 ? RP + upos : -1;
-        btab[8 * blk + 2] = ((Ucols + ppos - upos) << 16) | La;
-        btab[8 * blk + 3] = (self << 8) | ((int)isPn << 7) | (isPb << 6) | (mn << 3) | mb;
-      } else {
         btab[4 * blk] = RU >= 0 ? RU + upos : -1;
-        btab[4 * blk + 1] = (La << 9) | (self << 8) | (mn << 3) | mb;
+        btab[4 * blk + 1] = RP >= 0 ? RP + upos : -1;
+        btab[4 * blk + 2] = ((Ucols + ppos - upos) << 16) | La;
+        btab[4 * blk + 3] = (self << 8) | ((int)isPn << 7) | (isPb << 6) | (mn << 3) | mb;
+      } else {
+        btab[2 * blk] = RU >= 0 ? RU + upos : -1;
+        btab[2 * blk + 1] = (La << 9) | (self << 8) | (mn << 3) | mb;
       }
     }
     cu0 += __shfl(iu, 63, 64);
@@ -621,516 +743,289 @@ __global__ void __launch_bounds__(64) k_block_table(int32_t nNode, const int32_t
   }
 }
 
-// Build step 4: near[n] = 1 if an element around n has a node with a prescribed dof (the first-
-// iteration lift of n's rows is non-zero only there).
-template <int NPE>
-__global__ void k_near(int32_t nNode, const int32_t* __restrict__ nptr, const int32_t* __restrict__ nel,
-                       const int32_t* __restrict__ conn, const int32_t* __restrict__ nodeinfo,
-                       int32_t* __restrict__ near) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= nNode) return;
-  int f = 0;
-  for (int s = nptr[n]; s < nptr[n + 1] && !f; ++s) {
-    const int32_t* c = conn + (size_t)nel[s] * NPE;
-    for (int b = 0; b < NPE; ++b)
-      if ((nodeinfo[c[b]] & 7) != 7) f = 1;
+// Build step 4 (one wavefront per laid-out wavefront w): its runs (columns) and self runs (the column of the
+// node itself) are counted (COUNT), then tabled in their order in the wavefront:
+//   rtab[whead[w].x + r]  = the block table entry of run r
+//   stab[whead[w].y + q]  = {n's first free row, n's pressure row or -1, first item | items << 8 | free mask << 16, n}
+//   whead[w].zw           = the positions that start a run, as a 64-bit mask
+//   mtab[mhead[w] + q]    = Tet10/P1, the q-th run whose column node m carries a pressure: where n's u columns
+//                           start in m's pressure row (Kpu(m, n) is the transpose of the run's Kup(n, m))
+//   fitem                 = {offset of the item's block in the records (unsigned), slot | a << 10 | b << 14 |
+//                            transposed << 18 | self << 19 | first of its run << 20 | position << 21}, padding {0, -1},
+//                            in the order of the offsets
+// so that the row kernel reads its tables with consecutive lanes and does no index arithmetic.  A vector load's
+// address processing takes one pass per distinct 128-byte line among each four consecutive lanes (measured on
+// MI355X), and the kernel is bound by it: in record order a node's neighbouring blocks of an element are
+// neighbouring lanes.
+template <int NPE, bool MIXED, bool COUNT>
+__global__ void __launch_bounds__(64) k_wave_table(int64_t nwaves, int2* __restrict__ fitem,
+                                                   const int32_t* __restrict__ btab, const int32_t* __restrict__ conn,
+                                                   const int32_t* __restrict__ nodeinfo,
+                                                   const int32_t* __restrict__ nda, const int32_t* __restrict__ idp,
+                                                   const int32_t* __restrict__ nbptr, const int32_t* __restrict__ nb,
+                                                   int32_t dispDOF, int64_t* __restrict__ nrun,
+                                                   int64_t* __restrict__ nself, const int64_t* __restrict__ roff,
+                                                   const int64_t* __restrict__ soff, int4* __restrict__ whead,
+                                                   int32_t* __restrict__ rtab, int4* __restrict__ stab,
+                                                   int64_t* __restrict__ npres, const int64_t* __restrict__ poff,
+                                                   int32_t* __restrict__ mhead, int32_t* __restrict__ mtab) {
+  using Rc = Rec<NPE, MIXED>;
+  constexpr int BT = Rc::P1 ? 4 : 2;
+  const int64_t w = blockIdx.x;
+  if (w >= nwaves) return;
+  const int lane = threadIdx.x;
+  const int2 it = fitem[w * 64 + lane];
+  const bool on = it.x >= 0;
+  const int blk = on ? (it.y >> 4) : -1;
+  const int pblk = __shfl_up(blk, 1, 64);
+  const bool head = on && (lane == 0 || pblk != blk);
+  const int e = it.x >> 4, a = it.x & 15, b = it.y & 15;
+  const bool self = on && a == b;
+  const unsigned long long hm = __ballot(head), sm = __ballot(head && self), am = __ballot(self);
+  const bool pcol = Rc::P1 && head && ((btab[BT * (size_t)blk + (BT - 1)] >> 6) & 1);
+  const unsigned long long pm = __ballot(pcol);
+  if (COUNT) {
+    if (lane == 0) {
+      nrun[w] = __popcll(hm);
+      nself[w] = __popcll(sm);
+      if (Rc::P1) npres[w] = __popcll(pm);
+    }
+    return;
   }
-  near[n] = f;
-}
-
-// Gauss points gp0 .. gp0 + NG - 1 of one (element, node b) item of node n's rows, added to v: the
-// 3x3 block K_{n b} (v[0..8]) and, for the mixed element, Kup(n, b) (v[9..11]), Kpu(n, b)
-// (v[12..14]) and Kpp(n, b) (v[15]).  G, Bv, S point at the first of those Gauss points' g data
-// (stride NPE * GW; FROM_J: the inverse Jacobians of a Hex8 record, stride 9, g formed here), b
-// components (stride 6; compact records) and scalars (stride SS), in a staging record in global
-// memory or in a copy in LDS.
-template <int NPE, int NGP, bool MIXED, int NV, int NG, int UNROLL, bool FROM_J = false>
-__device__ __forceinline__ void item_gps(const double* G, const double* Bv, const double* S0p, int gp0, int a, int b,
-                                         double v[NV]) {
-  using St = Stage<NPE, NGP, MIXED>;
-#pragma unroll UNROLL
-  for (int gp = 0; gp < NG; ++gp) {
-    const double* Gp = G + gp * (FROM_J ? 9 : NPE * St::GW);
-    const double* S = S0p + gp * St::SS;
-    double ga[3], ba[3], gb[3], bb[3];
-    if (St::COMPACT && FROM_J) {  // g from the record's inverse Jacobian
-      double da[3], db[3];
-      hex8_dN_node(gp0 + gp, a, da);
-      hex8_dN_node(gp0 + gp, b, db);
-      grad_jinv(Gp, da, ga);
-      grad_jinv(Gp, db, gb);
-    } else if (St::COMPACT) {  // g formed in LDS, 3 doubles per node
+  const unsigned long long below = (1ull << lane) - 1;
+  if (lane == 0) whead[w] = make_int4((int)roff[w], (int)soff[w], (int)(uint32_t)hm, (int)(uint32_t)(hm >> 32));
+  if (head) {
+    int32_t* d = rtab + BT * (size_t)(roff[w] + __popcll(hm & below));
 #pragma unroll
-      for (int i = 0; i < 3; ++i) { ga[i] = Gp[a * 3 + i]; gb[i] = Gp[b * 3 + i]; }
-    } else {  // Tet10 records: g padded to 4 doubles, two 16-byte loads per node
-      const double2* ga2 = reinterpret_cast<const double2*>(Gp + a * 4);
-      const double2* gb2 = reinterpret_cast<const double2*>(Gp + b * 4);
-      const double2 p0 = ga2[0], p1 = ga2[1];
-      const double2 q0 = gb2[0], q1 = gb2[1];
-      ga[0] = p0.x; ga[1] = p0.y; ga[2] = p1.x;
-      gb[0] = q0.x; gb[1] = q0.y; gb[2] = q1.x;
-    }
-    {
-      const double2* B2 = reinterpret_cast<const double2*>(Bv + gp * 6);
-      const double2 c0 = B2[0], c1 = B2[1], c2 = B2[2];
-      const double B6[6] = {c0.x, c0.y, c1.x, c1.y, c2.x, c2.y};
-      bsym_times(B6, ga, ba);
-      bsym_times(B6, gb, bb);
-    }
-    tangent_gp<!MIXED>(ga, ba, gb, bb, S[0], S[1], S[2], S[3], MIXED ? 0.0 : S[4], v);
-    if (St::P1) {
-      double Np[4];
-      tet_Np(gp0 + gp, Np);
-      const double dv = S[4], dv0 = S[5], th = S[6];
-      const double Nb = b == 0 ? Np[0] : b == 1 ? Np[1] : b == 2 ? Np[2] : Np[3];
-      const double Na = a == 0 ? Np[0] : a == 1 ? Np[1] : a == 2 ? Np[2] : Np[3];
-      if (b < 4) {  // Kup(3a+i, b) += (dv g_a,i) Np_b   (ElementBase2.cpp:500-505)
-        v[9] += (dv * ga[0]) * Nb; v[10] += (dv * ga[1]) * Nb; v[11] += (dv * ga[2]) * Nb;
+    for (int q = 0; q < BT; ++q) d[q] = btab[BT * (size_t)blk + q];
+  }
+  if constexpr (Rc::P1) {
+    if (lane == 0) mhead[w] = (int)poff[w];
+    if (pcol) {
+      const int n = conn[(size_t)e * NPE + a], m = nb[blk];
+      int lo = nbptr[m], hi = nbptr[m + 1];
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (nb[mid] < n) lo = mid + 1; else hi = mid;
       }
-      if (a < 4) {  // Kpu(a, 3b+k) += (dv Np_a) g_b,k ; Kpp(a, b) -= (dv0 Np_a thetahat) Np_b (:524-539)
-        const double bb4 = dv * Na;
-        v[12] += bb4 * gb[0]; v[13] += bb4 * gb[1]; v[14] += bb4 * gb[2];
-        if (b < 4) v[15] -= ((dv0 * Na) * th) * Nb;
-      }
+      mtab[poff[w] + __popcll(pm & below)] = lo < nbptr[m + 1] && nb[lo] == n ? btab[BT * (size_t)lo + 1] : -1;
     }
   }
-}
-
-// One (element, node b) item of node n's rows over all Gauss points, from the element's staging
-// record at rec, UNROLL Gauss points at a time.
-template <int NPE, int NGP, bool MIXED, int NV, int UNROLL = 2>
-__device__ __forceinline__ void item_block(const double* rec, int a, int b, double v[NV]) {
-  using St = Stage<NPE, NGP, MIXED>;
-#pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] = 0.0;
-  item_gps<NPE, NGP, MIXED, NV, NGP, UNROLL, St::COMPACT>(rec + St::G0, rec + St::B0, rec + St::S0, 0, a, b, v);
-  if (St::P0) add_condensed(rec + St::W0, a, b, v);
-}
-
-// Node a's residual rows of one element (v[0..2]) and, for the mixed element, its pressure row (v[3])
-template <int NPE, int NGP, bool MIXED>
-__device__ __forceinline__ void item_residual(const double* rec, int a, double* v) {
-  using St = Stage<NPE, NGP, MIXED>;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) v[i] = rec[St::R0 + a * 3 + i];
-  if (St::P1 && a < 4) {
-    double fp = 0.0;  // Fp_a -= (dv0 Np_a) resip   (ElementBase2.cpp:510, 522)
-#pragma unroll
-    for (int gp = 0; gp < NGP; ++gp) {
-      double Np[4];
-      tet_Np(gp, Np);
-      const double Na = a == 0 ? Np[0] : a == 1 ? Np[1] : a == 2 ? Np[2] : Np[3];
-      fp -= (rec[St::S0 + gp * St::SS + 5] * Na) * rec[St::S0 + gp * St::SS + 7];
-    }
-    v[3] = fp;
+  if (head && self) {
+    const size_t n = (size_t)conn[(size_t)e * NPE + a];
+    const int mn = nodeinfo[n] & 7;
+    const int fr = (mn & 1) ? 0 : (mn & 2) ? 1 : 2;
+    const unsigned long long mine = am >> lane;  // the run's items are consecutive self items
+    int cnt = 1;
+    while (lane + cnt < 64 && ((mine >> cnt) & 1) && !((hm >> (lane + cnt)) & 1)) ++cnt;
+    stab[soff[w] + __popcll(sm & below)] =
+        make_int4(mn ? nda[3 * n + fr] : -1, Rc::P1 && idp[n] >= 0 ? dispDOF + idp[n] : -1,
+                  lane | (cnt << 8) | (mn << 16), (int)n);
   }
+  bool tr = false;
+  const int slot = on ? pair_slot<NPE, MIXED>(a, b, tr) : 0;
+  const uint32_t off = on ? (uint32_t)e * (uint32_t)Rc::TS + (uint32_t)slot : 0xffffffffu;
+  int rank = 0;
+  for (int j = 0; j < 64; ++j) {
+    const uint32_t oj = (uint32_t)__shfl((int)off, j, 64);
+    rank += (oj < off || (oj == off && j < lane)) ? 1 : 0;
+  }
+  fitem[w * 64 + rank] = on ? make_int2((int)off, slot | (a << 10) | (b << 14) | ((int)tr << 18) | ((int)self << 19) |
+                                                      ((int)head << 20) | (lane << 21))
+                            : make_int2(0, -1);
 }
 
-struct FlatArgs {
+struct RowArgs {
   int64_t nwaves;
-  const int2* fitem;        // {e * 16 + a, (j << 10) | (s << 4) | b}, {-1, -1} in padding slots
-  const int32_t* fnode;     // node whose rows each laid-out item belongs to (-1 in padding slots)
-  const uint8_t* fperm;     // per wavefront, lane L computes the item at run-order position fperm[L]
-  const int32_t* nbptr;
-  const int32_t* btab;      // per column block: its CSR location, then its mirror's (2 BT ints)
-  const int32_t* nda;
-  const int32_t* idp;
-  int32_t dispDOF;
-  const double* GS;
+  const int2* fitem;
+  const int4* whead;
+  const int32_t* rtab;
+  const int4* stab;
+  const int32_t* mhead;   // Tet10/P1
+  const int32_t* mtab;
+  const double* KE;
   double* vals;
   double* rhs;
-  // chunks of at most CW wavefronts of one layout group (chunked matrix kernel): first wavefront and
-  // count, distinct elements of the chunk's items in ascending order (ECAP slots per chunk), their
-  // number, and each item's slot
-  int64_t nchunks;
-  int32_t ecap;             // chunks with at most ecap (<= ECAP) distinct elements are staged
-  const int32_t* cwave;
-  const int32_t* cnw;
-  const int32_t* ctab;
-  const int32_t* ccnt;
-  const uint8_t* fslot;
+  const double* fext;     // unit-load external force per node dof, or null; rhs += lam fext
+  double lam;
+  const double* lam_dev;  // when given, the load factor in device memory (captured graphs)
 };
 
-// Three consecutive CSR values x0 x1 x2 at row[0..2] (the three free dofs of one column node) as one
-// 16-byte store on the 16-byte-aligned pair and one 8-byte store: two memory requests instead of
-// three.  row is 8-byte aligned (an offset into the value array).
-__device__ __forceinline__ void store3(double* row, double x0, double x1, double x2) {
-  const bool odd = (reinterpret_cast<uintptr_t>(row) & 8) != 0;
-  double2* pair = reinterpret_cast<double2*>(row + (odd ? 1 : 0));
-  *pair = odd ? make_double2(x1, x2) : make_double2(x0, x1);
-  row[odd ? 0 : 2] = odd ? x0 : x2;
+typedef double double2_u __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte load at an 8-byte address
+
+// The LDS writes of a wavefront are read by the same wavefront below: they execute in order, the fences
+// keep the compiler from moving them.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Writes a summed column block: K_nm (acc) into node n's rows at block blk and, through the mirror
-// table, its transpose into m's rows.  For the mixed element, acc[9..11] = Kup(n, m) (n's u rows,
-// m's pressure column), acc[12..14] = Kpu(n, m), acc[15] = Kpp(n, m); m's rows receive
-// Kup(m, n) = Kpu(n, m)^T, Kpu(m, n) = Kup(n, m)^T, Kpp(m, n) = Kpp(n, m).
-template <bool MIXED>
-__device__ __forceinline__ void write_block(const FlatArgs& F, const int* bt, const double* acc) {
-  constexpr int BT = MIXED ? 4 : 2;
+// Row kernel: kRowWaves independent wavefronts a workgroup, each on 64 laid-out items.  A lane reads its
+// item's block (72 contiguous bytes of the element's record) and stores it at its item's position in LDS, where runs
+// of equal column are consecutive items in element order.  Lane (run, column dof) then sums the run for the
+// (up to) three rows of the node and writes the values: consecutive lanes write consecutive values of a
+// row, and a wavefront that holds a whole node writes its rows entirely.
+// Bound by the vector loads' address processing (2.0 of the 3.0 ms on Hex8 128^3 with every record in cache; a
+// block is 72 scattered bytes) and by memory: 9 GB read and 4.1 GB written, exactly the values.
+// The two kernels replace Gauss-point records from which every item formed its block (Hex8: eight-wavefront chunks
+// with their elements in LDS, symmetric pairs written to both rows from one sum; Tet10: every item from global
+// memory).  Whole assembly, before -> now: Hex8 10^3 54 -> 40 us, 128^3 8.00 -> 6.07 ms; Q1/P0 45 x 31 x 52
+// 358 -> 251 us, 80^3 2.28 -> 1.54 ms; Tet10 30^3 x 6 830 -> 659 us; Tet10/P1 60^3 x 6 7.33 -> 7.06 ms.  Measured and
+// not taken (Hex8 128^3 / Tet10/P1 60^3 x 6, row kernel): non-temporal value stores 3.82 / 5.73 against 3.57 / 5.39 ms;
+// 1, 2, 8 wavefronts a workgroup 4.11, 3.93, 4.04 against 3.57 with 4; block offsets by distance before node 3.28 /
+// 4.94 against 2.97 / 4.66 by node.
+constexpr int kRowWaves = 4;
+template <int NPE, bool MIXED>
+__global__ void __launch_bounds__(64 * kRowWaves) k_rows(RowArgs F) {
+  using Rc = Rec<NPE, MIXED>;
+  constexpr bool P1 = Rc::P1;
+  constexpr int BT = P1 ? 4 : 2;  // ints of a run's table entry
+  constexpr int NR = P1 ? 4 : 3;  // right-hand-side rows of a node
+  __shared__ double sPartA[kRowWaves][64 * 9];
+  __shared__ int32_t sStartA[kRowWaves][65];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t nwg = (F.nwaves + kRowWaves - 1) / kRowWaves;
+  const int64_t w = xcd_chunk(blockIdx.x, nwg) * kRowWaves + wid;
+  if (w >= F.nwaves) return;  // no workgroup barrier below
+  double* const part = sPartA[wid];
+  int32_t* const start = sStartA[wid];
+  const int2 it = F.fitem[w * 64 + lane];
+  const int4 hd = F.whead[w];
+  const bool on = it.y >= 0;
+  const bool head = on && ((it.y >> 20) & 1);
+  const int a = (it.y >> 10) & 15, b = (it.y >> 14) & 15;
+  const double* blkp = F.KE + (uint32_t)it.x;
+  double v[9];
+  if (on) {
+    const double2_u* p2 = reinterpret_cast<const double2_u*>(blkp);
+    const double2_u x0 = p2[0], x1 = p2[1], x2 = p2[2], x3 = p2[3];
+    v[0] = x0.x; v[1] = x0.y; v[2] = x1.x; v[3] = x1.y; v[4] = x2.x; v[5] = x2.y; v[6] = x3.x; v[7] = x3.y;
+    v[8] = blkp[8];
+  }
+  const double* rec = blkp - (it.y & 1023);
+  double q4[P1 ? 4 : 1];  // Kup(n's u rows, b's pressure column), Kpp
+  if constexpr (P1) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) q4[t] = 0.0;
+    if (on && b < 4) {
+      const double* q = rec + Rc::Q0 + (a * 4 + b) * 3;
+      const double2_u x0 = *reinterpret_cast<const double2_u*>(q);
+      q4[0] = x0.x; q4[1] = x0.y; q4[2] = q[2];
+      if (a < 4) q4[3] = rec[Rc::P0f + 4 * (a < b ? a : b) + (a < b ? b : a)];
+    }
+  }
+  const bool self = on && ((it.y >> 19) & 1);
+  double rr[NR];
+  if (self) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rr[i] = rec[Rc::R0 + 3 * a + i];
+    if constexpr (P1) rr[3] = a < 4 ? rec[Rc::RP0 + a] : 0.0;
+  }
+  const unsigned long long hm = (uint32_t)hd.z | ((unsigned long long)(uint32_t)hd.w << 32);
+  const int pos = (it.y >> 21) & 63;
+  const int nruns = __popcll(hm), nself = __popcll(__ballot(head && self)), nitems = __popcll(__ballot(on));
+  if ((hm >> lane) & 1) start[__popcll(hm & ((1ull << lane) - 1))] = lane;
+  if (lane == 0) start[nruns] = nitems;
+  if (on) {
+    double* o = part + pos * 9;
+    const bool tr = (it.y >> 18) & 1;
+    o[0] = v[0];
+    o[4] = v[4];
+    o[8] = v[8];
+    const int t1 = tr ? 3 : 1, t2 = tr ? 6 : 2, t5 = tr ? 7 : 5;  // the stored block or its transpose
+    o[t1] = v[1];
+    o[4 - t1] = v[3];
+    o[t2] = v[2];
+    o[8 - t2] = v[6];
+    o[t5] = v[5];
+    o[12 - t5] = v[7];
+  }
+  wave_lds_fence();
   double* __restrict__ V = F.vals;
-  {
-    const int masks = MIXED ? bt[3] : (bt[1] & 0x1ff);
-    const int La = MIXED ? (bt[2] & 0xffff) : (bt[1] >> 9);
-    const int mn = (masks >> 3) & 7, mb = masks & 7;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      if (!((mn >> i) & 1)) continue;
-      double* row = V + bt[0] + rank3(mn, i) * La;
-      if (mb == 7) {
-        store3(row, acc[3 * i], acc[3 * i + 1], acc[3 * i + 2]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if ((mb >> k) & 1) row[rank3(mb, k)] = acc[3 * i + k];
-      }
-      if (MIXED && ((masks >> 6) & 1)) row[bt[2] >> 16] = acc[9 + i];
+  const int c = lane % 3;
+  for (int r = lane / 3, r0 = 0; r0 < nruns; r += 21, r0 += 21) {  // 21 runs at a time, lane 63 idle
+    if (lane == 63 || r >= nruns) continue;
+    int A0, La, masks;
+    if constexpr (P1) {
+      const int4 x = reinterpret_cast<const int4*>(F.rtab)[hd.x + r];
+      A0 = x.x; La = x.z & 0xffff; masks = x.w;
+    } else {
+      const int2 x = reinterpret_cast<const int2*>(F.rtab)[hd.x + r];
+      A0 = x.x; La = x.y >> 9; masks = x.y & 0x1ff;
     }
-    if (MIXED && ((masks >> 7) & 1)) {
-      double* row = V + bt[1];
-      if (mb == 7) {
-        store3(row, acc[12], acc[13], acc[14]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if ((mb >> k) & 1) row[rank3(mb, k)] = acc[12 + k];
+    int s = start[r];
+    const int s1 = start[r + 1];
+    const double* q = part + s * 9 + c;
+    double y0 = q[0], y1 = q[3], y2 = q[6];
+    for (++s; s < s1; ++s) {
+      q += 9;
+      y0 += q[0];
+      y1 += q[3];
+      y2 += q[6];
+    }
+    if ((masks & 0x3f) == 0x3f) {  // free node, free column
+      double* row = V + A0 + c;
+      row[0] = y0;
+      row[La] = y1;
+      row[2 * La] = y2;
+    } else {
+      const int mn = (masks >> 3) & 7, mb = masks & 7;
+      if ((mb >> c) & 1) {
+        double* row = V + A0 + rank3(mb, c);
+        if (mn & 1) row[0] = y0;
+        if (mn & 2) row[rank3(mn, 1) * La] = y1;
+        if (mn & 4) row[rank3(mn, 2) * La] = y2;
       }
-      if ((masks >> 6) & 1) row[bt[2] >> 16] = acc[15];
     }
   }
-  const int* mt = bt + BT;  // the mirror block (m, n): rows of m, columns of n (all masks 0 if none)
-  const int masks = MIXED ? mt[3] : (mt[1] & 0x1ff);
-  const int La = MIXED ? (mt[2] & 0xffff) : (mt[1] >> 9);
-  const int mm = (masks >> 3) & 7, mnn = masks & 7;  // free masks of m (rows) and n (columns)
+  if constexpr (P1) {  // couplings: Kup and Kpp of every item in the same LDS, the pressure column of run lane
+    wave_lds_fence();
+    if (on) {
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    if (!((mm >> k) & 1)) continue;
-    double* row = V + mt[0] + rank3(mm, k) * La;
-    if (mnn == 7) {
-      store3(row, acc[k], acc[3 + k], acc[6 + k]);
-    } else {
+      for (int i = 0; i < 4; ++i) part[pos * 4 + i] = q4[i];
+    }
+    wave_lds_fence();
+    const int4 x = lane < nruns ? reinterpret_cast<const int4*>(F.rtab)[hd.x + lane] : make_int4(0, 0, 0, 0);
+    const bool pcol = (x.w >> 6) & 1;
+    const unsigned long long pm = __ballot(pcol);
+    if (pcol) {
+      const int M = F.mtab[F.mhead[w] + __popcll(pm & ((1ull << lane) - 1))];
+      double y[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int s = start[lane]; s < start[lane + 1]; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] += part[s * 4 + i];
+      const int mn = (x.w >> 3) & 7, D = x.z >> 16, La = x.z & 0xffff;
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        if ((mnn >> i) & 1) row[rank3(mnn, i)] = acc[3 * i + k];
-    }
-    if (MIXED && ((masks >> 6) & 1)) row[mt[2] >> 16] = acc[12 + k];
-  }
-  if (MIXED && ((masks >> 7) & 1)) {
-    double* row = V + mt[1];
-    if (mnn == 7) {
-      store3(row, acc[9], acc[10], acc[11]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        if ((mnn >> i) & 1) row[rank3(mnn, i)] = acc[9 + i];
-    }
-    if ((masks >> 6) & 1) row[mt[2] >> 16] = acc[15];
-  }
-}
-
-// Column runs of one wavefront's items, after every item lane has stored its values at part[t * NT]
-// and its block index (nbptr[n] + j, unique per node and column) at col[t]: the first lane of each
-// run (its head) sums the run in lane order, which is element order, and writes the block and its
-// mirror; the self column's head also writes n's right-hand-side rows.  Every CSR value is written
-// exactly once.
-// An item lane's column-block table entry (its block's CSR location and its mirror's), loaded
-// before the lane's block is computed so that the run head has it at hand.
-template <bool MIXED>
-struct BlockEntry {
-  int v[MIXED ? 8 : 4];
-  __device__ __forceinline__ void load(const int32_t* btab, int blk) {
-    const int4* p = reinterpret_cast<const int4*>(btab) + (MIXED ? 2 : 1) * (size_t)blk;
-    const int4 x = p[0];
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-    if (MIXED) {
-      const int4 y = p[MIXED ? 1 : 0];
-      v[MIXED ? 4 : 0] = y.x; v[MIXED ? 5 : 1] = y.y; v[MIXED ? 6 : 2] = y.z; v[MIXED ? 7 : 3] = y.w;
+        if ((mn >> i) & 1) {
+          V[x.x + rank3(mn, i) * La + D] = y[i];
+          V[M + rank3(mn, i)] = y[i];
+        }
+      if ((x.w >> 7) & 1) V[x.y + D] = y[3];
     }
   }
-  __device__ __forceinline__ int flags() const { return MIXED ? v[3] : (v[1] & 0x1ff); }
-};
-
-// Column runs of one wavefront's items, after every item lane has stored its values at part[t * NT]
-// and its block index (nbptr[n] + j, unique per node and column) at col[t]: the first lane of each
-// run (its head) sums the run in lane order, which is element order, and writes the block and its
-// mirror (bt: the head's table entry); the self column's head also writes n's right-hand-side rows
-// (n: the head's node).  Every CSR value is written exactly once.
-template <bool MIXED, int NV, int NT>
-__device__ __forceinline__ void run_heads(const FlatArgs& F, int n, int lane, int blk, const double v[NT],
-                                          const int32_t* col, const double* part, const BlockEntry<MIXED>& bt) {
-  if (lane > 0 && col[lane - 1] == blk) return;
-  double acc[NT];
+  // right-hand side: lane (self run, row) sums the run's residual rows
+  if (nself == 0) return;
+  wave_lds_fence();
+  if (self) {
 #pragma unroll
-  for (int q = 0; q < NT; ++q) acc[q] = v[q];
-  for (int t2 = lane + 1; t2 < 64 && col[t2] == blk; ++t2)
-#pragma unroll
-    for (int q = 0; q < NT; ++q) acc[q] += part[t2 * NT + q];
-  const int flags = bt.flags();
-  if ((flags >> 8) & 1) {
-    // self block K_nn: its (i, k) and (k, i) entries (and n's u-p and p-u couplings) agree to
-    // rounding; their mean makes the assembled matrix exactly symmetric
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int k = i + 1; k < 3; ++k) acc[3 * i + k] = acc[3 * k + i] = 0.5 * (acc[3 * i + k] + acc[3 * k + i]);
-    if (MIXED)
-#pragma unroll
-      for (int i = 0; i < 3; ++i) acc[9 + i] = acc[12 + i] = 0.5 * (acc[9 + i] + acc[12 + i]);
-    // n's right-hand side, its elements' residuals in element order
-    const int mn = (flags >> 3) & 7;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      if ((mn >> i) & 1) F.rhs[F.nda[3 * (size_t)n + i]] = acc[NV + i];
-    if (MIXED && ((flags >> 7) & 1)) F.rhs[F.dispDOF + F.idp[n]] = acc[NT - 1];
+    for (int i = 0; i < NR; ++i) part[pos * NR + i] = rr[i];
   }
-  write_block<MIXED>(F, bt.v, acc);
-}
-
-// Matrix kernel, one wavefront per 64 laid-out items, every item reading its element's staging record
-// from global memory.  Lane L forms the block of the item at run-order position fperm[L] (items of
-// one element on consecutive lanes) and stores it at that position in LDS.  The runs are then summed
-// and written by lanes 0 .. nruns - 1, lane r taking the r-th run: the stores of a wavefront come
-// from consecutive lanes rather than from run heads spread over the wavefront (a store's address
-// processing, like a load's, takes one pass per distinct line among each four consecutive active
-// lanes).  The sums are those of the run heads, in run order, so the values are the same bits.
-template <int NPE, int NGP, bool MIXED>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) k_flat(FlatArgs F) {
-  using St = Stage<NPE, NGP, MIXED>;
-  constexpr bool P1 = St::P1;        // pressure rows (Tet10/P1)
-  constexpr int NV = P1 ? 16 : 9;    // uu 9 | up 3 | pu 3 | pp 1
-  constexpr int NR = P1 ? 4 : 3;     // right-hand-side rows of a node (self items)
-  constexpr int NT = NV + NR;
-  constexpr int BN = P1 ? 8 : 4;     // ints of a column-block table entry
-  __shared__ int32_t sCol[64];
-  __shared__ int32_t sStart[64];
-  __shared__ double sPart[64 * NT];
-  const int lane = threadIdx.x;
-  const int64_t w = xcd_chunk(blockIdx.x, F.nwaves);
-  if (w >= F.nwaves) return;
-  const int2 it = F.fitem[w * 64 + lane];  // run-order position lane
-  const int pc = F.fperm ? (int)F.fperm[w * 64 + lane] : lane;
-  const int2 ic = make_int2(__shfl(it.x, pc, 64), __shfl(it.y, pc, 64));  // the item this lane forms
-  const bool live = it.x >= 0;
-  const int blk = live ? (it.y >> 4) : -1;
-  const int pblk = __shfl_up(blk, 1, 64);
-  const bool head = live && (lane == 0 || pblk != blk);  // first position of its run
-  const bool self = head && (it.x & 15) == (it.y & 15);
-  const bool clive = ic.x >= 0;
-  const int e = ic.x >> 4, a = ic.x & 15, b = ic.y & 15;
-  const bool cself = clive && a == b;  // the element's own item of n carries its residual rows
-  double v[NT];
-#pragma unroll
-  for (int q = 0; q < NT; ++q) v[q] = 0.0;
-  const double* rec = F.GS + (size_t)(clive ? e : 0) * St::TS;
-  if (clive) item_block<NPE, NGP, MIXED, NV>(rec, a, b, v);
-  if (cself) item_residual<NPE, NGP, MIXED>(rec, a, v + NV);
-  // each run's table entry and node, loaded by its head before the barrier (registers are the
-  // limit during the block computation)
-  BlockEntry<P1> bt{};
-  if (head) bt.load(F.btab, blk);
-  const int n = self ? F.fnode[w * 64 + lane] : 0;
-  sCol[lane] = blk;
-#pragma unroll
-  for (int q = 0; q < NT; ++q) sPart[pc * NT + q] = v[q];
-  const unsigned long long hm = __ballot(head);
-  if (head) sStart[__popcll(hm & ((1ull << lane) - 1))] = lane;
-  __syncthreads();
-  const int nruns = __popcll(hm);
-  const int st = lane < nruns ? sStart[lane] : 0;
-  BlockEntry<P1> hb;
-#pragma unroll
-  for (int k = 0; k < BN; ++k) hb.v[k] = __shfl(bt.v[k], st, 64);
-  const int hn = __shfl(n, st, 64);
-  if (lane < nruns) run_heads<P1, NV, NT>(F, hn, st, sCol[st], sPart + st * NT, sCol, sPart, hb);
-}
-
-// Chunked matrix kernel: one workgroup per chunk (the wavefronts of one layout group of 8 nodes in
-// Morton order; for Hex8 on a structured grid an aligned 2x2x2 block of nodes and its 27 elements).
-// The chunk's distinct elements' Gauss-point data (g, b, scalars) is put in LDS — the verbatim part
-// of the records with coalesced 16-byte loads, g formed from the records' inverse Jacobians — and
-// every item then reads LDS: each record is read from L2 once per chunk rather than once per item
-// lane, and the per-lane gathers that bound the per-wavefront kernel on address processing become
-// LDS reads.  A chunk with more than ECAP distinct elements (or more than the problem's cap) reads
-// the records directly.  Workgroups of 8 wavefronts although a Hex8 group fills 5: measured per
-// Hex8 128^3 assembly, the kernel takes 13.6, 13.7, 8.3 and 7.0 ms with workgroups of 5, 6, 7 and 8
-// wavefronts for the same chunks.
-#ifndef MPF_CHUNK_WAVES
-#define MPF_CHUNK_WAVES 8
-#endif
-#ifndef MPF_CHUNK_ELEMS
-#define MPF_CHUNK_ELEMS 32
-#endif
-// LDS slot stride padded by 6 doubles (Hex8: 286 doubles, 2288 bytes per slot) so that the slots'
-// rows spread over the LDS banks: measured per Hex8 128^3 assembly, 10.24 ms unpadded, 9.97 ms
-// with 2, 9.93 ms with 6, 9.98 ms with 10
-#ifndef MPF_LDS_PAD
-#define MPF_LDS_PAD 6
-#endif
-// ECAP: the chunk table's slots per chunk; SCAP (<= ECAP): the most distinct elements staged in LDS
-// (Q1/P0 records are longer, so fewer fit where two workgroups share a CU's LDS).
-template <int NPE, int NGP, bool MIXED, int CW, int ECAP, int SCAP = ECAP>
-__global__ void __launch_bounds__(64 * CW) k_flat_chunk(FlatArgs F) {
-  using St = Stage<NPE, NGP, MIXED>;
-  constexpr bool P1 = St::P1;
-  constexpr int NV = P1 ? 16 : 9;
-  constexpr int NR = P1 ? 4 : 3;
-  constexpr int NT = NV + NR;
-  // LDS slot: g of every node and Gauss point (Hex8: formed here from the record's inverse
-  // Jacobians), then the record's B and S copied verbatim (Tet10/P1: the record's G and S verbatim)
-  constexpr int GX = St::COMPACT ? NGP * NPE * 3 : 0;   // g formed in LDS (doubles per slot)
-  constexpr int CP0 = St::COMPACT ? St::B0 : 0;          // record part copied verbatim: [CP0, SL)
-  constexpr int CP2 = (St::SL - CP0) / 2;                // its 16-byte groups
-  constexpr int SLP = GX + (St::SL - CP0) + MPF_LDS_PAD; // LDS stride per element slot (doubles)
-  static_assert(SLP % 2 == 0 && GX % 2 == 0 && CP0 % 2 == 0, "16-byte slots");
-  static_assert(SCAP <= ECAP, "staged elements fit the chunk table");
-  constexpr int STG = SCAP * SLP, PART = CW * 64 * NT;
-  constexpr int LDSD = STG > PART ? STG : PART;  // record copies, then the run sums
-  static_assert(ECAP <= 255, "slot tables");
-  __shared__ double2 sMem[LDSD / 2];
-  __shared__ int32_t sCol[CW * 64];
-  __shared__ double sdN[St::COMPACT ? NGP * NPE * 3 : 1];
-  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
-  const int64_t c = xcd_chunk(blockIdx.x, F.nchunks);
-  if (c >= F.nchunks) return;  // whole workgroup, before any barrier
-  const int cnt = F.ccnt[c];
-  const bool staged = cnt <= SCAP && cnt <= F.ecap;
-  // per-lane loads that need nothing from LDS, issued before the staging so that their latency
-  // overlaps it: the item, its slot, its block's table entry, and (self items) the node and the
-  // element's residual rows
-  const int64_t w = (int64_t)F.cwave[c] + wid;
-  const bool wv = wid < F.cnw[c];
-  const int2 it = wv ? F.fitem[w * 64 + lane] : make_int2(-1, -1);
-  const bool live = it.x >= 0;
-  const int blk = live ? (it.y >> 4) : 0;
-  const int e = it.x >> 4, a = it.x & 15, b = it.y & 15;
-  const bool self = live && a == b;
-  const int slot = live && staged ? F.fslot[w * 64 + lane] : 0;
-  BlockEntry<P1> bt;
-  bt.load(F.btab, blk);
-  const int n = self ? F.fnode[w * 64 + lane] : 0;
-  const double* rec = F.GS + (size_t)(live ? e : 0) * St::TS;
-  double v[NT];
-#pragma unroll
-  for (int q = 0; q < NT; ++q) v[q] = 0.0;
-  if (self) item_residual<NPE, NGP, MIXED>(rec, a, v + NV);
-  if (St::COMPACT && tid < NGP * NPE) hex8_dN_node(tid / NPE, tid % NPE, &sdN[3 * tid]);
-  __syncthreads();
-  if (staged) {
-    const int32_t* ct = F.ctab + c * ECAP;
-    constexpr int BS = 64 * CW;
-    // Hex8: one lane per (element slot, Gauss point) forms g of the 8 nodes from the record's inverse
-    // Jacobian; its loads are issued before the verbatim copy, so both share one memory latency
-    static_assert(!St::COMPACT || SCAP * NGP <= BS, "one (slot, Gauss point) per lane");
-    const bool jl = St::COMPACT && tid < cnt * NGP;
-    double Jr[9];
-    if (St::COMPACT) {
-      const double* J = F.GS + (size_t)ct[jl ? tid / NGP : 0] * St::TS + St::G0 + (tid % NGP) * 9;
-#pragma unroll
-      for (int i = 0; i < 9; ++i) Jr[i] = jl ? J[i] : 0.0;
-    }
-    // verbatim part: four 16-byte loads in flight per lane; indices past the end re-read the last group
-    const int tot = cnt * CP2;
-    auto ld = [&](int t) {
-      t = t < tot ? t : tot - 1;
-      const int k = t / CP2;
-      return reinterpret_cast<const double2*>(F.GS + (size_t)ct[k] * St::TS + CP0)[t - k * CP2];
-    };
-    auto dst = [&](int t) {
-      const int k = t / CP2;
-      return k * (SLP / 2) + GX / 2 + (t - k * CP2);
-    };
-    for (int t0 = tid; t0 < tot; t0 += 4 * BS) {
-      const double2 r0 = ld(t0), r1 = ld(t0 + BS), r2 = ld(t0 + 2 * BS), r3 = ld(t0 + 3 * BS);
-      sMem[dst(t0)] = r0;
-      if (t0 + BS < tot) sMem[dst(t0 + BS)] = r1;
-      if (t0 + 2 * BS < tot) sMem[dst(t0 + 2 * BS)] = r2;
-      if (t0 + 3 * BS < tot) sMem[dst(t0 + 3 * BS)] = r3;
-    }
-    if (jl) {
-      const int k = tid / NGP, gp = tid % NGP;
-      double* o = reinterpret_cast<double*>(sMem) + k * SLP + gp * NPE * 3;
-#pragma unroll
-      for (int a = 0; a < NPE; ++a) {
-        double g[3];
-        grad_jinv(Jr, &sdN[3 * (gp * NPE + a)], g);
-        o[3 * a] = g[0]; o[3 * a + 1] = g[1]; o[3 * a + 2] = g[2];
-      }
+  wave_lds_fence();
+  for (int t = lane; t < nself * NR; t += 64) {
+    const int q = t / NR, i = t - q * NR;
+    const int4 x = F.stab[hd.y + q];
+    const int s0 = x.z & 255, cnt = (x.z >> 8) & 255, mn = x.z >> 16;
+    double y = part[s0 * NR + i];
+    for (int s = s0 + 1; s < s0 + cnt; ++s) y += part[s * NR + i];
+    if (i == 3) {
+      if (x.y >= 0) F.rhs[x.y] = y;
+    } else if ((mn >> i) & 1) {
+      if (F.fext) y += (F.lam_dev ? *F.lam_dev : F.lam) * F.fext[3 * (size_t)x.w + i];
+      F.rhs[x.x + rank3(mn, i)] = y;
     }
   }
-  __syncthreads();
-  if (live) {
-    // one Gauss point at a time: LDS latency needs no unrolling to hide, and registers are the limit
-    if (staged) {
-      const double* sl = reinterpret_cast<const double*>(sMem) + slot * SLP;
-      item_gps<NPE, NGP, MIXED, NV, NGP, 1>(sl, sl + GX + (St::B0 - CP0), sl + GX + (St::S0 - CP0), 0, a, b, v);
-      if (St::P0) add_condensed(sl + GX + (St::W0 - CP0), a, b, v);
-    } else {
-      item_gps<NPE, NGP, MIXED, NV, NGP, 1, St::COMPACT>(rec + St::G0, rec + St::B0, rec + St::S0, 0, a, b, v);
-      if (St::P0) add_condensed(rec + St::W0, a, b, v);
-    }
-  }
-  __syncthreads();  // the record copies become the run-sum area
-  double* const part = reinterpret_cast<double*>(sMem) + wid * 64 * NT;
-  sCol[tid] = live ? blk : -1;
-#pragma unroll
-  for (int q = 0; q < NT; ++q) part[lane * NT + q] = v[q];
-  __syncthreads();
-  if (live) run_heads<P1, NV, NT>(F, n, lane, blk, v, sCol + wid * 64, part, bt);
-}
-
-// Chunk tables (once per pattern), one workgroup of 512 lanes per chunk of at most 8 wavefronts: the
-// chunk's distinct element ids in ascending order (bitonic sort of its items' elements in LDS, then a
-// compaction), their number, and each item's slot among them.
-template <int ECAP>
-__global__ void __launch_bounds__(512) k_chunk_table(int64_t nchunks, const int32_t* __restrict__ cwave,
-                                                     const int32_t* __restrict__ cnw, const int2* __restrict__ fitem,
-                                                     int32_t* __restrict__ ctab, int32_t* __restrict__ ccnt,
-                                                     uint8_t* __restrict__ fslot) {
-  constexpr int N = 512, NW = N / 64;
-  __shared__ int32_t key[N], uq[N], wsum[NW];
-  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
-  const int64_t c = blockIdx.x;
-  if (c >= nchunks) return;
-  const bool valid = wid < cnw[c];
-  const int64_t i = ((int64_t)cwave[c] + wid) * 64 + lane;
-  const int2 it = valid ? fitem[i] : make_int2(-1, -1);
-  const int32_t none = 0x7fffffff;
-  const int32_t e = it.x >= 0 ? (it.x >> 4) : none;
-  key[tid] = e;
-  __syncthreads();
-  for (int k = 2; k <= N; k <<= 1)
-    for (int h = k >> 1; h > 0; h >>= 1) {
-      const int p = tid ^ h;
-      if (p > tid) {
-        const int32_t x = key[tid], y = key[p];
-        if ((x > y) == ((tid & k) == 0)) { key[tid] = y; key[p] = x; }
-      }
-      __syncthreads();
-    }
-  const int32_t x = key[tid];
-  const bool u = x != none && (tid == 0 || key[tid - 1] != x);
-  const uint64_t bal = __ballot(u);
-  if (lane == 0) wsum[wid] = __popcll(bal);
-  __syncthreads();
-  int off = 0, tot = 0;
-  for (int q = 0; q < NW; ++q) {
-    if (q < wid) off += wsum[q];
-    tot += wsum[q];
-  }
-  if (u) uq[off + __popcll(bal & ((1ull << lane) - 1ull))] = x;
-  __syncthreads();
-  int slot = 0;
-  if (e != none && tot <= ECAP) {
-    int lo = 0, hi = tot - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (uq[mid] < e) lo = mid + 1; else hi = mid;
-    }
-    slot = lo;
-  }
-  if (valid) fslot[i] = (uint8_t)slot;
-  if (tid < ECAP) ctab[c * ECAP + tid] = tid < tot ? uq[tid] : 0;
-  if (tid == 0) ccnt[c] = tot;
 }
 
 struct RhsArgs {
@@ -1141,120 +1036,48 @@ struct RhsArgs {
   const int32_t* nda;
   const int32_t* idp;
   int32_t dispDOF;
-  const double* GS;
+  const double* KE;
   double* rhs;
-  int32_t lift_only;          // the residual sums are already in rhs (written by the matrix kernel)
+  const double* fext;
+  double lam;
+  const double* lam_dev;
+  int32_t isolated_only;      // the row kernel has written every node with an element
 };
 
 // Right-hand-side kernel (one lane per node): n's rows of the element residuals, summed in element
-// order.  With lift_only the matrix kernel has written them and only nodes in no element (whose rows
-// no item wrote) get their zeros here.
-template <int NPE, int NGP, bool MIXED>
+// order.  With isolated_only, the nodes in no element (zeros, and their external force).
+template <int NPE, bool MIXED>
 __global__ void __launch_bounds__(256) k_rhs(RhsArgs R) {
-  using St = Stage<NPE, NGP, MIXED>;
+  using Rc = Rec<NPE, MIXED>;
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= R.nNode) return;
   const int info = R.nodeinfo[n];
   const int mn = info & 7;
-  const bool isPn = St::P1 && ((info >> 3) & 1);
+  const bool isPn = Rc::P1 && ((info >> 3) & 1);
   if (!mn && !isPn) return;
   const int e0 = R.nptr[n], m = R.nptr[n + 1] - e0;
-  if (R.lift_only && m > 0) return;
+  if (R.isolated_only && m > 0) return;
   double r[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
   for (int s = 0; s < m; ++s) {
-    const int ea = R.nelA[e0 + s];
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    item_residual<NPE, NGP, MIXED>(R.GS + (size_t)(ea >> 4) * St::TS, ea & 15, t);
+    const int ea = R.nelA[e0 + s], a = ea & 15;
+    const double* rec = R.KE + (size_t)(ea >> 4) * Rc::TS;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) r[i] += t[i];
-    if (isPn) r[3] += t[3];
+    for (int i = 0; i < 3; ++i) r[i] += rec[Rc::R0 + 3 * a + i];
+    if (isPn && a < 4) r[3] += rec[Rc::RP0 + a];
   }
+  const double l = R.lam_dev ? *R.lam_dev : R.lam;
 #pragma unroll
   for (int i = 0; i < 3; ++i)
-    if ((mn >> i) & 1) R.rhs[R.nda[3 * (size_t)n + i]] = r[i];
+    if ((mn >> i) & 1) R.rhs[R.nda[3 * (size_t)n + i]] = R.fext ? r[i] + l * R.fext[3 * (size_t)n + i] : r[i];
   if (isPn) R.rhs[R.dispDOF + R.idp[n]] = r[3];
-}
-
-struct LiftArgs {
-  int32_t nnear;
-  const int32_t* list;        // nodes with a prescribed dof in an element around them
-  const int32_t* nptr;
-  const int32_t* nelA;
-  const int32_t* conn;
-  const int32_t* nodeinfo;
-  const int32_t* nda;
-  const int32_t* idp;
-  int32_t dispDOF;
-  const double* GS;
-  const double* dispApplied;
-  double* rhs;
-};
-
-// First-iteration lift (applyDirichletBCs / applyDirichletBCs2field, ElementBase.cpp:567-594,
-// 717-782): n's right-hand side loses  sum_e K_e(n, b) dubar_b  over the prescribed dofs of the
-// nodes b of n's elements.  One wavefront per listed node; its lanes take the (element, node b)
-// pairs and the wavefront sums their products in a fixed butterfly order.
-template <int NPE, int NGP, bool MIXED>
-__global__ void __launch_bounds__(64) k_lift(LiftArgs L) {
-  using St = Stage<NPE, NGP, MIXED>;
-  __shared__ double sdN[St::COMPACT ? NGP * NPE * 3 : 1];
-  const int q = blockIdx.x;
-  if (q >= L.nnear) return;
-  const int n = L.list[q], lane = threadIdx.x;
-  static_assert(!St::COMPACT || NGP * NPE <= 64, "one table entry per lane");
-  if (St::COMPACT && lane < NGP * NPE) hex8_dN_node(lane / NPE, lane % NPE, &sdN[3 * lane]);
-  __syncthreads();
-  const int info = L.nodeinfo[n];
-  const int mn = info & 7;
-  const bool isPn = St::P1 && ((info >> 3) & 1);
-  if (!mn && !isPn) return;
-  const int e0 = L.nptr[n], m = L.nptr[n + 1] - e0;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int t = lane; t < m * NPE; t += 64) {
-    const int s = t / NPE, b = t - s * NPE;
-    const int ea = L.nelA[e0 + s];
-    const int e = ea >> 4, a = ea & 15;
-    const int vb = L.conn[(size_t)e * NPE + b];
-    const int mb = L.nodeinfo[vb] & 7;
-    if (mb == 7) continue;
-    double db[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) db[k] = ((mb >> k) & 1) ? 0.0 : L.dispApplied[3 * (size_t)vb + k];
-    const double* rec = L.GS + (size_t)e * St::TS;
-    double Kb[9];
-    record_block<NPE, NGP, MIXED>(rec, a, b, Kb, St::COMPACT ? sdN : nullptr);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) acc[i] += Kb[3 * i] * db[0] + Kb[3 * i + 1] * db[1] + Kb[3 * i + 2] * db[2];
-    if (St::P1 && isPn && a < 4) {
-      double pu[3] = {0.0, 0.0, 0.0};  // Kpu(a, 3b+k) = sum (dv Np_a) g_b,k
-      for (int gp = 0; gp < NGP; ++gp) {
-        double Np[4];
-        tet_Np(gp, Np);
-        const double Na = a == 0 ? Np[0] : a == 1 ? Np[1] : a == 2 ? Np[2] : Np[3];
-        const double bb4 = rec[St::S0 + gp * St::SS + 4] * Na;
-        const double* gb = rec + St::G0 + (gp * NPE + b) * St::GW;
-        pu[0] += bb4 * gb[0]; pu[1] += bb4 * gb[1]; pu[2] += bb4 * gb[2];
-      }
-      acc[3] += pu[0] * db[0] + pu[1] * db[1] + pu[2] * db[2];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc[i] += shfl_xor_d(acc[i], off);
-  if (lane != 0) return;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-    if ((mn >> i) & 1) L.rhs[L.nda[3 * (size_t)n + i]] -= acc[i];
-  if (isPn) L.rhs[L.dispDOF + L.idp[n]] -= acc[3];
 }
 
 }  // namespace
 
-size_t stage_doubles_per_elem(int etype, bool p0) {
-  if (etype == MPF_HEX8) return p0 ? (size_t)Stage<8, 8, true>::TS : (size_t)Stage<8, 8, false>::TS;
-  if (etype == MPF_TET10) return (size_t)Stage<10, 4, false>::TS;
-  return (size_t)Stage<10, 4, true>::TS;
+size_t elem_record_doubles(int etype) {
+  if (etype == MPF_HEX8) return (size_t)Rec<8, false>::TS;
+  return etype == MPF_TET10 ? (size_t)Rec<10, false>::TS : (size_t)Rec<10, true>::TS;
 }
 
 static mpf_status gather_unsupported(mpf_problem* p, const char* why) {
@@ -1263,19 +1086,12 @@ static mpf_status gather_unsupported(mpf_problem* p, const char* why) {
   P.g_order.release();
   P.g_nelA.release();
   P.g_fitem.release();
-  P.g_fnode.release();
-  P.g_fperm.release();
-  P.g_cwave.release();
-  P.g_cnw.release();
-  P.g_btab.release();
-  P.g_near.release();
-  P.g_nearlist.release();
-  P.g_nnear = 0;
-  P.g_ctab.release();
-  P.g_ccnt.release();
-  P.g_fslot.release();
-  P.g_nchunks = 0;
-  p->GS.release();
+  P.g_whead.release();
+  P.g_rtab.release();
+  P.g_stab.release();
+  P.g_mhead.release();
+  P.g_mtab.release();
+  p->KE.release();
   p->asm_mode = MPF_ASSEMBLY_COLORED_SCATTER;
   return MPF_OK;
 }
@@ -1297,6 +1113,8 @@ mpf_status ensure_gather_tables(mpf_problem* p) {
   if (p->nElem >= (1 << 27)) return gather_unsupported(p, "more than 2^27 elements");
   if (nbtot >= (1 << 27)) return gather_unsupported(p, "more than 2^27 node-pair blocks");
   if (nNode == 0 || p->nElem == 0) return gather_unsupported(p, "empty mesh");
+  if ((uint64_t)p->nElem * elem_record_doubles(p->etype) >= (1ull << 32))
+    return gather_unsupported(p, "element records past 2^32 doubles");
 
   // processing order: Morton order of the node coordinates
   MPF_TRY(P.g_order.alloc(nNode));
@@ -1363,7 +1181,7 @@ mpf_status ensure_gather_tables(mpf_problem* p) {
     MPF_HIP(hipStreamSynchronize(s));
   }
 
-  // step 1: sorted owned items per node
+  // step 1: sorted items per node
   DevBuf<int32_t> keys, ovf;
   DevBuf<int64_t> cnt;
   MPF_TRY(P.g_nelA.alloc(nadj));
@@ -1386,6 +1204,7 @@ mpf_status ensure_gather_tables(mpf_problem* p) {
   MPF_HIP(hipStreamSynchronize(s));
   if (o & 1) return gather_unsupported(p, "a node has more than 64 elements or 128 coupled nodes");
   if (o & 2) return MPF_ERR_STATE;
+  P.g_isolated = (o & 4) != 0;
 
   // step 2: layout groups of 8 nodes in Morton order, their padded lengths and offsets
   const int64_t ngroups = ((int64_t)nNode + kGroupNodes - 1) / kGroupNodes;
@@ -1417,171 +1236,125 @@ mpf_status ensure_gather_tables(mpf_problem* p) {
 
   // laid-out items
   MPF_TRY(P.g_fitem.alloc(total > 0 ? (size_t)total : 64));
-  MPF_TRY(P.g_fnode.alloc(total > 0 ? (size_t)total : 64));
   MPF_HIP(hipMemsetAsync(P.g_fitem.ptr, 0xff, (total > 0 ? (size_t)total : 64) * sizeof(int2), s));
-  MPF_HIP(hipMemsetAsync(P.g_fnode.ptr, 0xff, (total > 0 ? (size_t)total : 64) * sizeof(int32_t), s));
   if (npe == 10)
     hipLaunchKernelGGL(k_group_fill<10>, dim3(ggrid), dim3(256), 0, s, ngroups, nNode, P.g_order.ptr, P.nptr.ptr,
-                       P.nbptr.ptr, keys.ptr, cnt.ptr, P.g_nelA.ptr, goff.ptr, P.g_fitem.ptr, P.g_fnode.ptr);
+                       P.nbptr.ptr, keys.ptr, cnt.ptr, P.g_nelA.ptr, goff.ptr, P.g_fitem.ptr);
   else
     hipLaunchKernelGGL(k_group_fill<8>, dim3(ggrid), dim3(256), 0, s, ngroups, nNode, P.g_order.ptr, P.nptr.ptr,
-                       P.nbptr.ptr, keys.ptr, cnt.ptr, P.g_nelA.ptr, goff.ptr, P.g_fitem.ptr, P.g_fnode.ptr);
+                       P.nbptr.ptr, keys.ptr, cnt.ptr, P.g_nelA.ptr, goff.ptr, P.g_fitem.ptr);
   MPF_HIP(hipGetLastError());
   P.g_nwaves = total / 64;
-  MPF_TRY(P.g_fperm.alloc(total > 0 ? (size_t)total : 64));
-  if (P.g_nwaves > 0)
-    hipLaunchKernelGGL(k_wave_perm, dim3((unsigned)P.g_nwaves), dim3(64), 0, s, P.g_nwaves, P.g_fitem.ptr,
-                       P.g_fperm.ptr);
-  MPF_HIP(hipGetLastError());
 
-  // chunk tables of the chunked matrix kernel (Hex8): each group's wavefronts in chunks of <= CW
-  if (p->etype == MPF_HEX8 && P.g_nwaves > 0) {
-    constexpr int CW = MPF_CHUNK_WAVES, ECAP = MPF_CHUNK_ELEMS;
-    static_assert(ECAP == 32, "mpf_set_chunk_stage_cap documents a cap of 32");
-    static_assert(CW >= 1 && CW <= 8, "k_chunk_table covers 8 wavefronts");
-    DevBuf<int64_t> ccount, coff;
-    MPF_TRY(ccount.alloc(ngroups + 1));
-    MPF_TRY(coff.alloc(ngroups + 1));
-    hipLaunchKernelGGL(k_group_chunks, dim3(ggrid), dim3(256), 0, s, ngroups, CW, glen.ptr, goff.ptr, nullptr,
-                       ccount.ptr, nullptr, nullptr);
-    MPF_HIP(hipMemsetAsync(ccount.ptr + ngroups, 0, sizeof(int64_t), s));
-    MPF_TRY(exclusive_sum(ccount.ptr, coff.ptr, ngroups + 1));
-    int64_t nch = 0;
-    MPF_HIP(hipMemcpyAsync(&nch, coff.ptr + ngroups, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+  // step 3: column-block table; step 4: the row kernel's tables
+  DevBuf<int32_t> btab;
+  MPF_TRY(btab.alloc((size_t)(nbtot > 0 ? nbtot : 1) * (mixed ? 4 : 2)));
+  if (mixed)
+    hipLaunchKernelGGL(k_block_table<true>, dim3(nNode), dim3(64), 0, s, nNode, P.nbptr.ptr, P.nb.ptr, P.nodeinfo.ptr,
+                       P.nda.ptr, P.idp.ptr, P.dispDOF, P.rowptr.ptr, btab.ptr);
+  else
+    hipLaunchKernelGGL(k_block_table<false>, dim3(nNode), dim3(64), 0, s, nNode, P.nbptr.ptr, P.nb.ptr, P.nodeinfo.ptr,
+                       P.nda.ptr, nullptr, P.dispDOF, P.rowptr.ptr, btab.ptr);
+  MPF_HIP(hipGetLastError());
+  if (P.g_nwaves > 0) {
+    DevBuf<int64_t> nrun, nself, roff, soff, npres, poff;
+    const int64_t nw = P.g_nwaves;
+    MPF_TRY(nrun.alloc(nw + 1));
+    MPF_TRY(nself.alloc(nw + 1));
+    MPF_TRY(roff.alloc(nw + 1));
+    MPF_TRY(soff.alloc(nw + 1));
+    MPF_HIP(hipMemsetAsync(nrun.ptr + nw, 0, sizeof(int64_t), s));
+    MPF_HIP(hipMemsetAsync(nself.ptr + nw, 0, sizeof(int64_t), s));
+    MPF_TRY(P.g_whead.alloc(nw));
+    if (mixed) {
+      MPF_TRY(npres.alloc(nw + 1));
+      MPF_TRY(poff.alloc(nw + 1));
+      MPF_TRY(P.g_mhead.alloc(nw));
+      MPF_HIP(hipMemsetAsync(npres.ptr + nw, 0, sizeof(int64_t), s));
+    }
+    const auto table = [&](bool count) {
+#define MPF_WT(NPE, MX, C)                                                                                           \
+  hipLaunchKernelGGL((k_wave_table<NPE, MX, C>), dim3((unsigned)nw), dim3(64), 0, s, nw, P.g_fitem.ptr, btab.ptr, \
+                     p->conn.ptr, P.nodeinfo.ptr, P.nda.ptr, P.idp.ptr, P.nbptr.ptr, P.nb.ptr, P.dispDOF, nrun.ptr,  \
+                     nself.ptr, roff.ptr, soff.ptr, P.g_whead.ptr, P.g_rtab.ptr, P.g_stab.ptr, npres.ptr, poff.ptr,   \
+                     P.g_mhead.ptr, P.g_mtab.ptr)
+      if (mixed) { if (count) MPF_WT(10, true, true); else MPF_WT(10, true, false); }
+      else if (npe == 10) { if (count) MPF_WT(10, false, true); else MPF_WT(10, false, false); }
+      else { if (count) MPF_WT(8, false, true); else MPF_WT(8, false, false); }
+#undef MPF_WT
+    };
+    table(true);
+    MPF_TRY(exclusive_sum(nrun.ptr, roff.ptr, nw + 1));
+    MPF_TRY(exclusive_sum(nself.ptr, soff.ptr, nw + 1));
+    if (mixed) MPF_TRY(exclusive_sum(npres.ptr, poff.ptr, nw + 1));
+    int64_t tot[3] = {0, 0, 0};
+    if (mixed) MPF_HIP(hipMemcpyAsync(&tot[2], poff.ptr + nw, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    MPF_HIP(hipMemcpyAsync(&tot[0], roff.ptr + nw, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    MPF_HIP(hipMemcpyAsync(&tot[1], soff.ptr + nw, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     MPF_HIP(hipStreamSynchronize(s));
-    P.g_nchunks = nch;
-    MPF_TRY(P.g_cwave.alloc((size_t)nch));
-    MPF_TRY(P.g_cnw.alloc((size_t)nch));
-    MPF_TRY(P.g_ctab.alloc((size_t)nch * ECAP));
-    MPF_TRY(P.g_ccnt.alloc((size_t)nch));
-    MPF_TRY(P.g_fslot.alloc((size_t)P.g_nwaves * 64));
-    hipLaunchKernelGGL(k_group_chunks, dim3(ggrid), dim3(256), 0, s, ngroups, CW, glen.ptr, goff.ptr, coff.ptr,
-                       nullptr, P.g_cwave.ptr, P.g_cnw.ptr);
-    hipLaunchKernelGGL((k_chunk_table<ECAP>), dim3((unsigned)nch), dim3(512), 0, s, nch, P.g_cwave.ptr, P.g_cnw.ptr,
-                       P.g_fitem.ptr, P.g_ctab.ptr, P.g_ccnt.ptr, P.g_fslot.ptr);
+    MPF_TRY(P.g_rtab.alloc((size_t)tot[0] * (mixed ? 4 : 2)));
+    MPF_TRY(P.g_stab.alloc((size_t)tot[1]));
+    if (mixed) MPF_TRY(P.g_mtab.alloc((size_t)std::max<int64_t>(tot[2], 1)));
+    table(false);
     MPF_HIP(hipGetLastError());
     MPF_HIP(hipStreamSynchronize(s));
   }
-
-  // step 3: column-block table; step 4: near-Dirichlet flags
-  MPF_TRY(P.g_btab.alloc((size_t)(nbtot > 0 ? nbtot : 1) * (mixed ? 8 : 4)));
-  if (mixed)
-    hipLaunchKernelGGL(k_block_table<true>, dim3(nNode), dim3(64), 0, s, nNode, P.nbptr.ptr, P.nb.ptr, P.nodeinfo.ptr,
-                       P.nda.ptr, P.idp.ptr, P.dispDOF, P.rowptr.ptr, P.g_btab.ptr);
-  else
-    hipLaunchKernelGGL(k_block_table<false>, dim3(nNode), dim3(64), 0, s, nNode, P.nbptr.ptr, P.nb.ptr, P.nodeinfo.ptr,
-                       P.nda.ptr, nullptr, P.dispDOF, P.rowptr.ptr, P.g_btab.ptr);
-  if (mixed)
-    hipLaunchKernelGGL(k_mirror<true>, dim3(nNode), dim3(64), 0, s, nNode, P.nbptr.ptr, P.nb.ptr, P.nodeinfo.ptr,
-                       P.g_btab.ptr);
-  else
-    hipLaunchKernelGGL(k_mirror<false>, dim3(nNode), dim3(64), 0, s, nNode, P.nbptr.ptr, P.nb.ptr, P.nodeinfo.ptr,
-                       P.g_btab.ptr);
-  MPF_HIP(hipGetLastError());
-  MPF_TRY(P.g_near.alloc(nNode));
-  if (npe == 10)
-    hipLaunchKernelGGL(k_near<10>, dim3(grid_for(nNode, 256)), dim3(256), 0, s, nNode, P.nptr.ptr, P.nel.ptr,
-                       p->conn.ptr, P.nodeinfo.ptr, P.g_near.ptr);
-  else
-    hipLaunchKernelGGL(k_near<8>, dim3(grid_for(nNode, 256)), dim3(256), 0, s, nNode, P.nptr.ptr, P.nel.ptr,
-                       p->conn.ptr, P.nodeinfo.ptr, P.g_near.ptr);
-  MPF_HIP(hipGetLastError());
-  // list of the flagged nodes (the lift kernel's wavefronts)
-  {
-    MPF_TRY(P.g_nearlist.alloc(nNode));
-    DevBuf<int32_t> nsel;
-    MPF_TRY(nsel.alloc(1));
-    hipcub::CountingInputIterator<int32_t> ids(0);
-    size_t tmp = 0;
-    MPF_HIP(hipcub::DeviceSelect::Flagged(nullptr, tmp, ids, P.g_near.ptr, P.g_nearlist.ptr, nsel.ptr, nNode, s));
-    DevBuf<char> t;
-    MPF_TRY(t.alloc(tmp > 0 ? tmp : 1));
-    MPF_HIP(hipcub::DeviceSelect::Flagged(t.ptr, tmp, ids, P.g_near.ptr, P.g_nearlist.ptr, nsel.ptr, nNode, s));
-    MPF_HIP(hipMemcpyAsync(&P.g_nnear, nsel.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    MPF_HIP(hipStreamSynchronize(s));
-  }
-  MPF_TRY(p->GS.alloc((size_t)p->nElem * stage_doubles_per_elem(p->etype, p->p0)));
+  MPF_TRY(p->KE.alloc((size_t)p->nElem * elem_record_doubles(p->etype)));
   MPF_HIP(hipStreamSynchronize(s));
   P.gather_ready = true;
   return MPF_OK;
 }
 
-mpf_status launch_gather_assembly(mpf_problem* p, const ElemArgs& A, const double* dispApplied, int writeK,
-                                  hipStream_t s) {
+// The two kernels of one element type.  Elements a workgroup: Hex8, 8 (64 Gauss-point lanes and 64 node lanes);
+// Tet10, 12 (48 and 120 lanes of 128).
+template <int NPE, int NGP, bool MIXED, int EPB>
+static void launch_type(const ElemArgs& A, mpf_problem* p, const double* dispApplied, const RowArgs& F,
+                        const RhsArgs& R, bool flat, hipStream_t s) {
+  const int32_t nElem = p->nElem;
+  const dim3 grid(grid_for(nElem, EPB));
+  const int block = (EPB * NPE + 63) / 64 * 64;
+  const int32_t* info = p->pat.nodeinfo.ptr;
+  double *KE = p->KE.ptr, *qu = p->q_Kup.ptr, *qp = p->q_Kpp.ptr, *qf = p->q_Fp.ptr;
+#define MPF_ELEM(BLOCKS, LIFT)                                                                                   \
+  hipLaunchKernelGGL((k_elem_records<NPE, NGP, MIXED, EPB, BLOCKS, LIFT>), grid, dim3(block *(BLOCKS ? 2 : 1)), 0, \
+                     s, A, nElem, dispApplied, info, KE, qu, qp, qf)
+  if (flat && dispApplied) MPF_ELEM(true, true);
+  else if (flat) MPF_ELEM(true, false);
+  else if (dispApplied) MPF_ELEM(false, true);
+  else MPF_ELEM(false, false);
+#undef MPF_ELEM
+  if (flat) {
+    const int64_t nwg = (F.nwaves + kRowWaves - 1) / kRowWaves;
+    hipLaunchKernelGGL((k_rows<NPE, MIXED>), dim3((unsigned)((nwg + 7) / 8 * 8)), dim3(64 * kRowWaves), 0, s, F);
+  }
+  if (!flat || R.isolated_only)
+    hipLaunchKernelGGL((k_rhs<NPE, MIXED>), dim3(grid_for(p->nNode, 256)), dim3(256), 0, s, R);
+}
+
+mpf_status launch_gather_assembly(mpf_problem* p, const ElemArgs& A, const double* dispApplied, int writeK, double lam,
+                                  const double* lam_dev, hipStream_t s) {
   const PatternBufs& P = p->pat;
   if (!P.gather_ready) return MPF_ERR_STATE;
-  const int32_t nElem = p->nElem, nNode = p->nNode;
-  if (nElem <= 0 || nNode <= 0) return MPF_OK;
-  const bool mixed = p->etype == MPF_TET10P1;
-  FlatArgs F{};
+  if (p->nElem <= 0 || p->nNode <= 0) return MPF_OK;
+  if (p->bc_dof_h.empty()) dispApplied = nullptr;  // nothing prescribed: no lift
+  const double* fext = p->has_fext && P.dispDOF > 0 ? p->fext_unit.ptr : nullptr;
+  RowArgs F{};
   F.nwaves = P.g_nwaves;
-  F.fitem = P.g_fitem.ptr;
-  F.fnode = P.g_fnode.ptr;
-  F.fperm = P.g_fperm.ptr;
-  F.nbptr = P.nbptr.ptr;
-  F.btab = P.g_btab.ptr;
-  F.nda = P.nda.ptr;
-  F.idp = P.idp.ptr;
-  F.dispDOF = P.dispDOF;
-  F.GS = p->GS.ptr;
-  F.vals = p->vals.ptr;
-  F.rhs = p->rhs.ptr;
-  F.nchunks = P.g_nchunks;
-  F.ecap = p->chunk_cap;
-  F.cwave = P.g_cwave.ptr;
-  F.cnw = P.g_cnw.ptr;
-  F.ctab = P.g_ctab.ptr;
-  F.ccnt = P.g_ccnt.ptr;
-  F.fslot = P.g_fslot.ptr;
-  RhsArgs R{};
-  R.nNode = nNode;
-  R.nptr = P.nptr.ptr; R.nelA = P.g_nelA.ptr; R.nodeinfo = P.nodeinfo.ptr; R.nda = P.nda.ptr;
-  R.idp = P.idp.ptr; R.dispDOF = P.dispDOF; R.GS = p->GS.ptr; R.rhs = p->rhs.ptr;
-  LiftArgs L{};
-  L.nnear = P.g_nnear; L.list = P.g_nearlist.ptr;
-  L.nptr = P.nptr.ptr; L.nelA = P.g_nelA.ptr; L.conn = p->conn.ptr; L.nodeinfo = P.nodeinfo.ptr;
-  L.nda = P.nda.ptr; L.idp = P.idp.ptr; L.dispDOF = P.dispDOF; L.GS = p->GS.ptr; L.dispApplied = dispApplied;
-  L.rhs = p->rhs.ptr;
-  const bool lift = dispApplied != nullptr && L.nnear > 0;
-  // with the matrix the residual sums come from the matrix kernel; k_rhs then only lifts
+  F.fitem = P.g_fitem.ptr; F.whead = P.g_whead.ptr; F.rtab = P.g_rtab.ptr; F.stab = P.g_stab.ptr;
+  F.mhead = P.g_mhead.ptr; F.mtab = P.g_mtab.ptr;
+  F.KE = p->KE.ptr; F.vals = p->vals.ptr; F.rhs = p->rhs.ptr;
+  F.fext = fext; F.lam = lam; F.lam_dev = lam_dev;
   const bool flat = writeK && F.nwaves > 0;
-  R.lift_only = flat ? 1 : 0;
-  const unsigned flat_grid = (unsigned)(((F.nwaves + 7) / 8) * 8);
-  const unsigned chunk_grid = (unsigned)(((F.nchunks + 7) / 8) * 8);
-  const bool chunked = p->asm_mode != MPF_ASSEMBLY_GATHER_DIRECT && F.nchunks > 0;
-  if (p->etype == MPF_TET10) {
-    hipLaunchKernelGGL((k_stage<10, 4, false, 16, MPF_STAGE_LDS_TET>), dim3(grid_for(nElem, 16)), dim3(64), 0, s, A,
-                       nElem, p->GS.ptr, nullptr, nullptr, nullptr);
-    if (flat) hipLaunchKernelGGL((k_flat<10, 4, false>), dim3(flat_grid), dim3(64), 0, s, F);
-    hipLaunchKernelGGL((k_rhs<10, 4, false>), dim3(grid_for(nNode, 256)), dim3(256), 0, s, R);
-    if (lift) hipLaunchKernelGGL((k_lift<10, 4, false>), dim3(L.nnear), dim3(64), 0, s, L);
-  } else if (p->p0) {  // Hex8 Q1/P0: condensed records, displacement rows only
-    hipLaunchKernelGGL((k_stage<8, 8, true, 8, MPF_STAGE_LDS_HEX>), dim3(grid_for(nElem, 8)), dim3(64), 0, s, A,
-                       nElem, p->GS.ptr, p->q_Kup.ptr, p->q_Kpp.ptr, p->q_Fp.ptr);
-    if (flat && chunked)
-      hipLaunchKernelGGL((k_flat_chunk<8, 8, true, MPF_CHUNK_WAVES, MPF_CHUNK_ELEMS, 28>),
-                         dim3(chunk_grid), dim3(64 * MPF_CHUNK_WAVES), 0, s, F);
-    else if (flat)
-      hipLaunchKernelGGL((k_flat<8, 8, true>), dim3(flat_grid), dim3(64), 0, s, F);
-    hipLaunchKernelGGL((k_rhs<8, 8, true>), dim3(grid_for(nNode, 256)), dim3(256), 0, s, R);
-    if (lift) hipLaunchKernelGGL((k_lift<8, 8, true>), dim3(L.nnear), dim3(64), 0, s, L);
-  } else if (!mixed) {
-    hipLaunchKernelGGL((k_stage<8, 8, false, 8, MPF_STAGE_LDS_HEX>), dim3(grid_for(nElem, 8)), dim3(64), 0, s, A,
-                       nElem, p->GS.ptr, nullptr, nullptr, nullptr);
-    if (flat && chunked)
-      hipLaunchKernelGGL((k_flat_chunk<8, 8, false, MPF_CHUNK_WAVES, MPF_CHUNK_ELEMS>),
-                         dim3(chunk_grid), dim3(64 * MPF_CHUNK_WAVES), 0, s, F);
-    else if (flat)
-      hipLaunchKernelGGL((k_flat<8, 8, false>), dim3(flat_grid), dim3(64), 0, s, F);
-    hipLaunchKernelGGL((k_rhs<8, 8, false>), dim3(grid_for(nNode, 256)), dim3(256), 0, s, R);
-    if (lift) hipLaunchKernelGGL((k_lift<8, 8, false>), dim3(L.nnear), dim3(64), 0, s, L);
-  } else {
-    hipLaunchKernelGGL((k_stage<10, 4, true, 16, MPF_STAGE_LDS_TET>), dim3(grid_for(nElem, 16)), dim3(64), 0, s, A,
-                       nElem, p->GS.ptr, nullptr, nullptr, nullptr);
-    if (flat) hipLaunchKernelGGL((k_flat<10, 4, true>), dim3(flat_grid), dim3(64), 0, s, F);
-    hipLaunchKernelGGL((k_rhs<10, 4, true>), dim3(grid_for(nNode, 256)), dim3(256), 0, s, R);
-    if (lift) hipLaunchKernelGGL((k_lift<10, 4, true>), dim3(L.nnear), dim3(64), 0, s, L);
-  }
+  RhsArgs R{};
+  R.nNode = p->nNode;
+  R.nptr = P.nptr.ptr; R.nelA = P.g_nelA.ptr; R.nodeinfo = P.nodeinfo.ptr; R.nda = P.nda.ptr;
+  R.idp = P.idp.ptr; R.dispDOF = P.dispDOF; R.KE = p->KE.ptr; R.rhs = p->rhs.ptr;
+  R.fext = fext; R.lam = lam; R.lam_dev = lam_dev;
+  R.isolated_only = flat && P.g_isolated ? 1 : 0;
+  if (p->etype == MPF_TET10) launch_type<10, 4, false, 12>(A, p, dispApplied, F, R, flat, s);
+  else if (p->etype == MPF_TET10P1) launch_type<10, 4, true, 12>(A, p, dispApplied, F, R, flat, s);
+  else if (p->p0) launch_type<8, 8, true, 8>(A, p, dispApplied, F, R, flat, s);
+  else launch_type<8, 8, false, 8>(A, p, dispApplied, F, R, flat, s);
   MPF_HIP(hipGetLastError());
   return MPF_OK;
 }

@@ -143,20 +143,13 @@ struct PatternBufs {
   // gather-assembly tables (gather.hip)
   DevBuf<int32_t> g_order;    // nodes in Morton (Z-curve) order of their coordinates
   DevBuf<int32_t> g_nelA;     // elements around each node (ascending), with the node's local index
-  DevBuf<int2> g_fitem;       // laid-out (element, node) items of the owned blocks, 64 per wavefront
-  DevBuf<int32_t> g_fnode;    // node whose rows each laid-out item belongs to
-  DevBuf<uint8_t> g_fperm;    // per wavefront: the run-order position of the item each lane computes
-  DevBuf<int32_t> g_btab;     // CSR location of every column block (n, j) and of its mirror (m, n)
-  DevBuf<int32_t> g_near;     // node has a prescribed dof in an element around it
-  DevBuf<int32_t> g_nearlist; // the flagged nodes
-  int32_t g_nnear = 0;
+  DevBuf<int2> g_fitem;       // laid-out (element, node) items of every node, 64 per wavefront
+  DevBuf<int4> g_whead;       // per wavefront of items: its first entries in the two tables below, run starts
+  DevBuf<int32_t> g_rtab;     // CSR location of every column block, in the wavefronts' order
+  DevBuf<int4> g_stab;        // rows and residual items of every node, in the wavefronts' order
+  DevBuf<int32_t> g_mhead, g_mtab;  // Tet10/P1: where a run's transpose goes in the pressure rows
   int64_t g_nwaves = 0;
-  mpf::DevBuf<int32_t> g_cwave;  // chunked matrix kernel: first wavefront of each chunk
-  mpf::DevBuf<int32_t> g_cnw;    // its number of wavefronts
-  mpf::DevBuf<int32_t> g_ctab;   // distinct elements per chunk
-  mpf::DevBuf<int32_t> g_ccnt;   // their number per chunk
-  mpf::DevBuf<uint8_t> g_fslot;  // each laid-out item's element slot in its chunk
-  int64_t g_nchunks = 0;
+  bool g_isolated = false;    // some node with rows lies in no element
   bool gather_ready = false;
   std::vector<int32_t> color_off;  // host: [ncolors + 1] offsets into perm
   int32_t dispDOF = 0, presDOF = 0, ncolors = 0;
@@ -205,11 +198,11 @@ struct mpf_problem {
   bool assembled = false;
   bool solved = false;
   mpf::KrylovWork* kw = nullptr;
-  // assembly algorithm (MPF_ASSEMBLY_*) and the gather path's staging records
+  // assembly algorithm (MPF_ASSEMBLY_*) and the gather path's element records
   int32_t asm_mode = MPF_ASSEMBLY_GATHER;
   int32_t band_split = 1;  // banded direct solve: cut long blocks at a separator (band.hip)
-  int32_t chunk_cap = 32;  // Hex8 chunked matrix kernel: most distinct elements staged in LDS
-  mpf::DevBuf<double> GS;
+  int32_t chunk_cap = 32;  // mpf_set_chunk_stage_cap's value (kept for the autotuner's report)
+  mpf::DevBuf<double> KE;
   mpf::DevBuf<double> scratch;  // reductions (norms)
   mpf::BatchWork* batch = nullptr;  // independent meshes solved together (batch.hip)
   mpf::BandWork* band = nullptr;    // banded LDL^T direct solver (band.hip)
@@ -219,10 +212,10 @@ struct mpf_problem {
 
 namespace mpf {
 uint64_t next_problem_uid();                        // problem.hip: unique per process
-size_t stage_doubles_per_elem(int etype, bool p0);  // gather.hip
+size_t elem_record_doubles(int etype);              // gather.hip
 mpf_status ensure_gather_tables(mpf_problem* p);   // gather.hip (falls back to the scatter when unsupported)
-mpf_status launch_gather_assembly(mpf_problem* p, const ElemArgs& A, const double* dispApplied, int writeK,
-                                  hipStream_t s);
+mpf_status launch_gather_assembly(mpf_problem* p, const ElemArgs& A, const double* dispApplied, int writeK, double lam,
+                                  const double* lam_dev, hipStream_t s);
 mpf_status build_pattern(mpf_problem* p);          // pattern.hip
 // batch.hip
 ElemArgs batch_elem_args(mpf_problem* p, ElemArgs a);

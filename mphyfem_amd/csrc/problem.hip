@@ -230,14 +230,16 @@ ElemArgs elem_args(mpf_problem* p) {
 
 
 
-// Enqueue the element kernels of one assembly (no zero fill, no external forces).
-mpf_status enqueue_element_kernels(mpf_problem* p, bool first_iter, int scatterK) {
+bool gathers(const mpf_problem* p) { return p->asm_mode != MPF_ASSEMBLY_COLORED_SCATTER; }
+
+// Enqueue the kernels of one assembly: of the gather, everything; of the coloured scatter, the element
+// kernels (no zero fill, no external forces).
+mpf_status enqueue_element_kernels(mpf_problem* p, bool first_iter, int scatterK, double lam, const double* lam_dev) {
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
   ElemArgs A = elem_args(p);
-  if (p->asm_mode == MPF_ASSEMBLY_GATHER || p->asm_mode == MPF_ASSEMBLY_GATHER_DIRECT) {
-    return launch_gather_assembly(p, A, first_iter ? p->dispApplied.ptr : nullptr, scatterK, s);
-  }
+  if (gathers(p))
+    return launch_gather_assembly(p, A, first_iter ? p->dispApplied.ptr : nullptr, scatterK, lam, lam_dev, s);
   ScatterArgs sc{};
   sc.slot = P.slot.ptr;
   sc.nodeinfo = P.nodeinfo.ptr;
@@ -261,17 +263,18 @@ mpf_status enqueue_element_kernels(mpf_problem* p, bool first_iter, int scatterK
 }
 
 // Enqueue one full assembly (no synchronisation).  scatterK = 0 assembles the residual only.
-// zeroMtx (SolverPetsc.cpp:145-163) is only needed by the scatter, which accumulates.
+// zeroMtx (SolverPetsc.cpp:145-163) is only needed by the scatter, which accumulates; the gather adds
+// the external forces where it writes the right-hand side.
 mpf_status enqueue_assembly(mpf_problem* p, bool first_iter, double lam, int scatterK, const double* lam_dev = nullptr) {
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
   const int64_t n = (int64_t)P.dispDOF + P.presDOF;
-  if (p->asm_mode == MPF_ASSEMBLY_COLORED_SCATTER) {
+  if (!gathers(p)) {
     if (scatterK) hipLaunchKernelGGL(k_fill_d, dim3(g256(P.nnz)), dim3(256), 0, s, p->vals.ptr, P.nnz, 0.0);
     hipLaunchKernelGGL(k_fill_d, dim3(g256(n)), dim3(256), 0, s, p->rhs.ptr, n, 0.0);
   }
-  MPF_TRY(enqueue_element_kernels(p, first_iter, scatterK));
-  if (p->has_fext && P.dispDOF > 0)
+  MPF_TRY(enqueue_element_kernels(p, first_iter, scatterK, lam, lam_dev));
+  if (!gathers(p) && p->has_fext && P.dispDOF > 0)
     hipLaunchKernelGGL(k_add_fext, dim3(grid_for(P.dispDOF, 256)), dim3(256), 0, s, P.dispDOF, P.assy.ptr,
                        p->fext_unit.ptr, lam, lam_dev, p->rhs.ptr);
   MPF_HIP(hipGetLastError());
@@ -866,9 +869,9 @@ mpf_status mpf_time_assembly(mpf_problem* p, int32_t reps, int32_t first_iter, d
   MPF_HIP(hipEventElapsedTime(&ms, e0, e1));
   if (ms_per_assembly) *ms_per_assembly = ms / reps;
   if (ms_scatter_kernels) {
-    // element kernels only (no zero fill / external forces)
+    // the scatter's element kernels only (no zero fill / external forces); the gather's are the assembly
     MPF_HIP(hipEventRecord(e0, s));
-    for (int r = 0; r < reps; ++r) MPF_TRY(enqueue_element_kernels(p, first_iter != 0, 1));
+    for (int r = 0; r < reps; ++r) MPF_TRY(enqueue_element_kernels(p, first_iter != 0, 1, lam, nullptr));
     MPF_HIP(hipEventRecord(e1, s));
     MPF_HIP(hipEventSynchronize(e1));
     MPF_HIP(hipEventElapsedTime(&ms, e0, e1));

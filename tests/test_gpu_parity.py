@@ -766,3 +766,69 @@ def test_newton_tet10_vs_oracle(mpf, orc, gpu, ksp):
     assert st == 0
     assert np.array_equal(iters, oit), (iters, oit)
     assert normwise_rel(P.state()[0], O.state()[0]) < 1e-9
+
+
+@pytest.mark.parametrize("first", [True, False], ids=["lift", "no_lift"])
+@pytest.mark.parametrize("etype,dims", [("hex8", (1, 1, 1)), ("hex8", (9, 1, 1)), ("hex8", (3, 5, 7)), ("hex8p0", (2, 1, 1)),
+                                        ("hex8p0", (5, 3, 3)), ("tet10", 1), ("tet10", 3), ("tet10p1", 1),
+                                        ("tet10p1", 3)])
+def test_gather_workgroup_remainders_vs_oracle(mpf, orc, gpu, etype, dims, first):
+    """Element counts that leave part of a workgroup's elements empty (8 a workgroup for Hex8, 12 for Tet10), one
+    element alone, wavefronts of items shared by several boundary nodes, nodes split over wavefronts (Tet10 vertices),
+    prescribed single components, and a dead load: K and R against the oracle within TOL_K, the assembled matrix
+    bitwise repeatable.  1e-12 is some 100 rounding errors of a sum of at most 24 elements' blocks."""
+    code = {"hex8": mpf.HEX8, "hex8p0": mpf.HEX8P0, "tet10": mpf.TET10, "tet10p1": mpf.TET10P1}[etype]
+    hexa = etype.startswith("hex8")
+    if hexa:
+        nx, ny, nz = dims
+        X, conn = mpf.mesh_hex(nx, ny, nz, jitter=0.1, seed=8)
+        faces = mpf.hex_face_quads(nx, ny, nz, 5)
+        h = 1.0 / max(dims)
+    else:
+        X, conn = mpf.mesh_tet10(dims, jitter=0.1, seed=8)
+        nx = ny = nz = dims
+        faces, h = None, 0.5 / dims
+    m = mpf.matl(1.0, 1e-2, 3, mixed=etype in ("hex8p0", "tet10p1"))
+    P = mpf.Problem(code, X, conn, m)
+    O = orc.Problem({mpf.HEX8: 8, mpf.HEX8P0: 9, mpf.TET10: 11, mpf.TET10P1: 10}[code], X, conn, 1.0, 1e-2, 3)
+    rng = np.random.default_rng(81)
+    u = rng.uniform(-0.01 * h, 0.01 * h, 3 * len(X))
+    p = rng.uniform(-0.2, 0.2, len(conn) if etype == "hex8p0" else len(X))
+    low = mpf.face_nodes(code, nx, ny, nz, 4)
+    for Q in (P, O):
+        Q.add_dirichlet(low, -1)
+        Q.add_dirichlet(mpf.face_nodes(code, nx, ny, nz, 1), 0, 0.02)
+        Q.add_dirichlet(low[:1], 1, -0.01)
+        if faces is not None:
+            Q.add_traction(faces, -0.05, 0.02)
+        Q.prepare_matrix_pattern()
+        Q.set_state(disp=u, disp_prev=0.5 * u, pres=p, pres_prev=p)
+        Q.set_boundary_conditions(0.8)
+    assert P.assembly_mode() == mpf.ASSEMBLY_GATHER
+    P.calc_stiffness_and_residual(first, 0.8)
+    vals, rhs = P.system()
+    P.calc_stiffness_and_residual(first, 0.8)
+    v2, r2 = P.system()
+    assert np.array_equal(vals, v2) and np.array_equal(rhs, r2)
+    ov, orhs, st = O.assemble(first, 0.8)
+    assert st == 0
+    assert normwise_rel(vals, ov) < TOL_K and normwise_rel(rhs, orhs) < TOL_K
+
+
+def test_gather_node_in_no_element(mpf, orc, gpu):
+    """A free node that no element holds: empty rows, a right-hand side of zero at every assembly (not what the last
+    solve or assembly left there), the other rows as without it."""
+    X, conn = cube_hex(3)
+    P = mpf.Problem(mpf.HEX8, X, conn, mpf.matl_from_E_nu(1e3, 0.3))
+    Q = mpf.Problem(mpf.HEX8, np.vstack([X, [[2.0, 2.0, 2.0]]]), conn, mpf.matl_from_E_nu(1e3, 0.3))
+    out = []
+    for R in (P, Q):
+        apply_bcs(R, hex_stretch_bcs(3))
+        R.prepare_matrix_pattern()
+        R.set_boundary_conditions(1.0)
+        for _ in range(2):
+            R.calc_stiffness_and_residual(True, 1.0)
+        out.append(R.system())
+    n = len(out[0][1])
+    assert len(out[1][1]) == n + 3 and not out[1][1][n:].any()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1][:n])
