@@ -6,7 +6,7 @@
 // renumbered node by node (reverse Cuthill-McKee or slices across an axis, whichever gives the
 // smaller half-bandwidth b), which makes the block banded; the block is then factored as L D L^T
 // without pivoting (K is the symmetric tangent of the consistent mode; a zero or non-finite pivot is
-// reported) and solved, one workgroup per segment and kernel.
+// reported) and solved, the solve and the separator's steps by one workgroup per segment.
 //
 // Segments: a block long enough (n >= 3 b + 64 rows) is cut in two at a separator S of s rows
 // (b <= s < b + 16) in its middle, and eliminated in the order [A1, A2 reversed, S]: segment 0
@@ -17,10 +17,12 @@
 // serial chain of panels of a long block is halved, and the segments (longest first) fill more of
 // the GPU's compute units than one workgroup per block.  Shorter blocks are one segment.
 //
-//   k_band_factor: right-looking in panels of kW columns -- the panel factored column by column
-//   (bands up to 176 wide: by one wavefront in registers, three rows per lane; wider: one thread
-//   per panel row and one barrier per column), the rank-kW update of the b x b trailing triangle
-//   on the matrix cores (FP64 MFMA);
+//   k_band_panel / k_band_trail: right-looking in panels of kP columns on several workgroups per
+//   segment, one launch pair per panel (few segments, or wide bands: band_panels);
+//   k_band_factor: right-looking in panels of kW columns by one workgroup per segment -- the panel
+//   factored column by column (bands up to 176 wide: by one wavefront in registers, three rows per
+//   lane; wider: one thread per panel row and one barrier per column), the rank-kW update of the
+//   b x b trailing triangle on the matrix cores (FP64 MFMA);
 //   k_band_solve: forward and backward substitution in blocks of kW rows, the unit triangle in one
 //   wavefront's registers, the coupling to the next b rows by the whole workgroup.
 //
@@ -70,6 +72,7 @@ struct BandArgs {
   double* band;
   double* y;     // permuted right-hand side, then the solution, per segment
   int32_t* bad;  // set on a zero or non-finite pivot
+  double* diag;  // the current panel's factored diagonal block per segment (kP x kP, column-major)
 };
 
 // Band of every active segment from the CSR rows, zeros included, and its right-hand side, in one
@@ -409,6 +412,268 @@ __global__ void __launch_bounds__(kFBS) k_band_factor(BandArgs A, int32_t bmax, 
   if (tid == 0 && phase == 0) factored[S.blk] = 1;  // the band holds this block's factors once the launches end
 }
 
+// ---- factorisation by panels of kP columns over several workgroups per segment ----
+//
+// Launch pair p (all segments at once) factors the segments' p-th panels of kP columns: k_band_panel the panel
+// itself, k_band_trail the rank-kP update of the trailing window.  One workgroup per segment (k_band_factor) is a serial
+// chain of panels and of the window's tiles on one compute unit; here the tiles leave the chain, which is then the
+// diagonal block's 64 pivots (divide, multiply, broadcast, multiply-add: 280 cycles each, 8.5 of the panel's 22 us),
+// the panel's load, the last 16 columns of the rows below and two launches.  Measured, a whole direct solve, one workgroup per
+// segment -> panels: 8 x 8 x 8 elements (half-bandwidth 235, 2 segments) 2.44 -> 0.89 ms, 60 blocks of 11 to 19 x 11 x 11
+// (473) 30.8 -> 13.2 ms, one beam of 64 x 4 x 8 (167) 4.77 -> 3.39 ms, 40 of them 5.75 -> 4.84 ms.
+// Not kept: 192 or 128 rows below the diagonal block per workgroup (its loads then wait on one compute unit:
+// 32 / 31 us a panel against 22), 32 x 32 window tiles per wavefront (11.3 us an update against 7.5), window loads in
+// one branch per entry (a lane's 64 loads one after the other: 25 us a panel's load against 2).
+constexpr int kP = 64;      // panel width
+constexpr int kLdP = 80;    // LDS column stride of 64 rows: two columns of 16 rows fall on different halves of the banks
+constexpr int kRW = 32;     // rows below the diagonal block per wavefront
+constexpr int kStrip = 64;  // such rows per workgroup: two wavefronts
+
+// Dynamic LDS of k_band_panel: the diagonal block (column-major: L below, the pivots on the diagonal, their
+// reciprocals in row 64), the strip.
+constexpr size_t kPanelLds = 2 * kP * kLdP * sizeof(double);
+
+// Keeps a load where it stands: without it the compiler moves a load whose value is selected by a condition
+// under a branch on that condition, and a lane's loads then run one after the other.
+__device__ __forceinline__ void keep(double& v) { asm("" : "+v"(v)); }
+
+__device__ __forceinline__ void wave_order() {  // LDS of one wavefront: in order, not reordered by the compiler
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Columns q .. q + 15 (q a multiple of 16, above 0) of NT 16-row tiles at X (column-major, stride kLdP) less their products
+// with the q columns before: X(r, q + c) -= sum_k X(r, k) D(k, k) D(q + c, k), by one wavefront on the matrix
+// cores, the operands of 16 columns loaded ahead of their products.
+template <int NT>
+__device__ __forceinline__ void panel_update16(double* X, const double* D, int q, int i16, int k4) {
+  double4_t acc[NT];
+  double av[4], pv[4], xv[4][NT];
+  const auto load = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 + 4 * u + k4;
+      av[u] = D[k * kLdP + q + i16];
+      pv[u] = D[k * (kLdP + 1)];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) xv[u][t] = X[k * kLdP + 16 * t + i16];
+    }
+  };
+  load(0);
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[t][v] = X[(q + 4 * v + k4) * kLdP + 16 * t + i16];
+#pragma unroll 1
+  for (int k0 = 0; k0 < q; k0 += 16) {
+    double a[4], x[4][NT];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a[u] = -(av[u] * pv[u]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) x[u][t] = xv[u][t];
+    }
+    if (k0 + 16 < q) load(k0 + 16);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], x[u][t], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) X[(q + 4 * v + k4) * kLdP + 16 * t + i16] = acc[t][v];
+}
+
+// Panel p: columns [j0, j0 + w) of the segment's [c0, c1).  Wavefront 0 factors the w x w diagonal block (padded
+// with the identity to kP) in LDS, 16 columns at a time: their update by the columns before on the matrix cores, then
+// the 16 in registers, one row per lane, the pivot and the rows' entries read across lanes.  The other wavefronts
+// follow one step of 16 columns behind with kRW rows each below the block: the same update, then substitution against
+// the unit triangle in LDS, a row on two lanes.  Workgroups of one segment (blockIdx.y) factor the diagonal
+// block alike; the first puts it out.
+__global__ void __launch_bounds__(192) k_band_panel(BandArgs A, int32_t phase, int32_t p,
+                                                   const int32_t* __restrict__ active, int32_t astride,
+                                                   int32_t* __restrict__ factored) {
+  extern __shared__ double sPanel[];
+  double* D = sPanel;
+  const BandSeg S = A.seg[blockIdx.x];
+  if (active && !active[(size_t)S.blk * astride]) return;
+  const int c1 = phase ? S.nend : S.nf, j0 = (phase ? S.nf : 0) + p * kP;
+  if (j0 >= c1) return;  // whole workgroup
+  const int w = min(kP, c1 - j0);
+  const int n = S.n, b = S.b, B1 = b + 1;
+  double* L = A.band + S.boff + (size_t)j0 * B1;        // entry (j0 + r, j0 + c) at c B1 + r - c
+  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63, i16 = lane & 15, k4 = lane >> 4;
+  const int rs0 = w + blockIdx.y * kStrip;              // panel-relative first strip row
+  const int rend = min(n - j0, w + b);                  // rows the panel reaches
+  if (blockIdx.y > 0 && rs0 >= rend) return;
+  const int sw = (wid - 1) * kRW;                       // wavefronts from 1: first strip row, this lane's row
+  const int half = lane / kRW, rl = lane % kRW, r = rs0 + sw + rl;
+  const bool strip = wid > 0 && rs0 + sw < rend;        // uniform per wavefront
+  double* X = D + kP * kLdP + sw;
+  // rows of the wavefront that all lie in the band in all kP columns take no test per entry
+  const bool whole = w == kP && (wid == 0 ? b >= kP - 1 : rs0 + sw + kRW <= min(rend, b + 1));
+  // all columns in one round trip; above the diagonal and past the band: any entry
+  if (wid == 0) {
+    const uint32_t at = (uint32_t)min(lane, w - 1);
+    double v[kP];
+#pragma unroll
+    for (int c = 0; c < kP; ++c) v[c] = (L + (size_t)c * (B1 - 1))[at];  // entry (lane, c)
+#pragma unroll
+    for (int c = 0; c < kP; ++c) keep(v[c]);
+    if (!whole) {
+#pragma unroll
+      for (int c = 0; c < kP; ++c)
+        if (c >= w || lane < c || lane >= w || lane - c > b) v[c] = c >= w && lane == c ? 1.0 : 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < kP; ++c) D[c * kLdP + lane] = v[c];
+    wave_order();
+  } else if (strip) {  // the lanes' halves take every other column
+    const uint32_t at = (uint32_t)(half * (B1 - 1) + min(r, rend - 1));
+    double v[kP / 2];
+#pragma unroll
+    for (int c = 0; c < kP / 2; ++c) v[c] = (L + (size_t)(2 * c) * (B1 - 1))[at];  // entry (r, 2 c + half)
+#pragma unroll
+    for (int c = 0; c < kP / 2; ++c) keep(v[c]);
+    if (!whole) {
+#pragma unroll
+      for (int c = 0; c < kP / 2; ++c) {
+        if (2 * c + half >= w || r >= rend || r - (2 * c + half) > b) v[c] = 0.0;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kP / 2; ++c) X[(2 * c + half) * kLdP + rl] = v[c];
+    wave_order();
+  }
+  const int nq = (w + 15) / 16;
+#pragma unroll 1
+  for (int s = 0; s <= nq; ++s) {
+    if (wid == 0 && s < nq) {
+      const int q = 16 * s;
+      if (s == 1) panel_update16<3>(D + 16, D, q, i16, k4);  // rows q .. 63
+      if (s == 2) panel_update16<2>(D + 32, D, q, i16, k4);
+      if (s == 3) panel_update16<1>(D + 48, D, q, i16, k4);
+      wave_order();
+      double a[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) a[c] = D[(q + c) * kLdP + lane];
+      double dl = 1.0;  // lane q + c: its pivot
+#pragma unroll
+      for (int c = 0; c < 16; ++c) {
+        const double d = lane_value(a[c], q + c);
+        const double t = a[c] * (1.0 / d);  // L(r, c)
+#pragma unroll
+        for (int cc = c + 1; cc < 16; ++cc) a[cc] -= a[c] * lane_value(t, q + cc);
+        dl = lane == q + c ? d : dl;
+        a[c] = lane > q + c ? t : a[c];
+      }
+      if (dl == 0.0 || !isfinite(dl)) *A.bad = 1;
+#pragma unroll
+      for (int c = 0; c < 16; ++c)
+        if (lane >= q + c) D[(q + c) * kLdP + lane] = a[c];
+      if (lane >= q && lane < q + 16) D[lane * kLdP + 64] = 1.0 / dl;
+    }
+    if (strip && s > 0) {
+      const int q = 16 * (s - 1);
+      if (q > 0) panel_update16<kRW / 16>(X, D, q, i16, k4);
+      wave_order();
+      double x[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) x[c] = X[(q + c) * kLdP + rl];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) {
+        const double* col = D + (q + c) * kLdP + q;
+#pragma unroll
+        for (int cc = c + 1; cc < 16; ++cc) x[cc] -= x[c] * col[cc];
+        x[c] *= D[(q + c) * kLdP + 64];
+      }
+      double* out = L + (size_t)q * (B1 - 1);
+#pragma unroll
+      for (int c = 0; c < 16; c += 2) {  // the lanes' halves write every other column
+        keep(x[c]);  // or the pair becomes an array in memory, indexed by half
+        keep(x[c + 1]);
+        const double xc = half ? x[c + 1] : x[c];
+        X[(q + c + half) * kLdP + rl] = xc;
+        if (whole || (q + c + half < w && r < rend && r - (q + c + half) <= b))
+          (out + (size_t)c * (B1 - 1))[(uint32_t)(half * (B1 - 1) + r)] = xc;
+      }
+      wave_order();
+    }
+    __syncthreads();
+  }
+  if (wid == 0 && blockIdx.y == 0) {  // not into the band: the segment's other workgroups may still read it there
+    double* out = A.diag + (size_t)blockIdx.x * kP * kP;
+#pragma unroll 16
+    for (int c = 0; c < kP; ++c) out[c * kP + lane] = D[c * kLdP + lane];
+  }
+  // the band holds this block's factors once the launches end
+  if (phase == 0 && blockIdx.y == 0 && tid == 0 && j0 + w >= c1) factored[S.blk] = 1;
+}
+
+// Trailing update of panel p: A(r, c) -= sum over the panel's columns of L(r, k) d_k L(c, k), r >= c, for the
+// rows and columns past the panel that it reaches: one tile of kTile rows and columns of the lower triangle per workgroup, a
+// quarter per wavefront, operands read from the band (L2) as the matrix cores take them, all loads in flight together.
+constexpr int kTile = 32;
+__global__ void __launch_bounds__(256) k_band_trail(BandArgs A, int32_t phase, int32_t p,
+                                                   const int32_t* __restrict__ active, int32_t astride) {
+  const BandSeg S = A.seg[blockIdx.x];
+  if (active && !active[(size_t)S.blk * astride]) return;
+  const int c1 = phase ? S.nend : S.nf, j0 = (phase ? S.nf : 0) + p * kP;
+  if (j0 >= c1) return;
+  const int w = min(kP, c1 - j0);
+  const int b = S.b, B1 = b + 1;
+  const int rend = min(S.n - j0, w + b);  // panel-relative
+  int t = 0;
+  while ((t + 1) * (t + 2) / 2 <= (int)blockIdx.y) ++t;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+  double* L = A.band + S.boff + (size_t)j0 * B1;
+  const double* D = A.diag + (size_t)blockIdx.x * kP * kP;
+  if (blockIdx.y == 0)  // the diagonal block's factors into the band (no entry of it is read here)
+    for (int c = wid; c < w; c += 4)
+      if (lane >= c && lane < w && lane - c <= b) L[(size_t)c * B1 + (lane - c)] = D[c * kP + lane];
+  const int R0 = w + kTile * t + 16 * (wid >> 1);
+  const int C0 = w + kTile * ((int)blockIdx.y - t * (t + 1) / 2) + 16 * (wid & 1);
+  if (R0 >= rend || C0 >= rend || R0 + 15 < C0) return;  // uniform per wavefront, no barrier below
+  // Entry (r, c) lies at c (B1 - 1) + r: the columns of a lane are 4 apart, one 32-bit offset per lane and a uniform
+  // base.  A quarter inside the band takes no test per entry; elsewhere what is loaded past the band is replaced.
+  const bool whole = w == kP && R0 + 15 < rend && R0 + 15 <= b && R0 >= C0 + 15;
+  const int r = R0 + i16, ca = C0 + i16;  // this lane's row, and its column's row as an operand
+  const uint32_t ro = (uint32_t)(k4 * (B1 - 1) + min(r, rend - 1)), co = (uint32_t)(k4 * (B1 - 1) + min(ca, rend - 1));
+  double old[4], rv[kP / 4], cv[kP / 4], dk[kP / 4];
+#pragma unroll
+  for (int u = 0; u < kP / 4; ++u) {
+    dk[u] = (D + 4 * u * (kP + 1))[k4 * (kP + 1)];
+    const double* col = L + (size_t)(4 * u) * (B1 - 1);
+    rv[u] = col[ro];
+    cv[u] = col[co];
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) old[v] = (L + (size_t)min(C0 + 4 * v, rend - 1) * (B1 - 1))[ro];
+#pragma unroll
+  for (int u = 0; u < kP / 4; ++u) { keep(dk[u]); keep(rv[u]); keep(cv[u]); }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) keep(old[v]);
+  if (!whole) {
+#pragma unroll
+    for (int u = 0; u < kP / 4; ++u) {
+      const int k = 4 * u + k4;
+      if (k >= w || r >= rend || r - k > b) rv[u] = 0.0;
+      if (k >= w || ca >= rend || ca - k > b) cv[u] = 0.0;
+      if (k >= w) dk[u] = 0.0;
+    }
+  }
+  double4_t acc = {};
+#pragma unroll
+  for (int u = 0; u < kP / 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[u] * dk[u], rv[u], acc, 0, 0, 0);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {  // entry (r, C0 + 4 v + k4)
+    const int c = C0 + 4 * v + k4;
+    if (whole || (r >= c && r < rend && r - c <= b)) (L + (size_t)(C0 + 4 * v) * (B1 - 1))[ro] = old[v] - acc[v];
+  }
+}
+
 // Solve L D L^T x = y in place for one segment per workgroup (skipped like the factorisation), in
 // blocks of kW rows: the kW x kW unit triangle by wavefront 0 with the segment's L in registers and
 // the solved values read across lanes; the coupling to the next b rows by the workgroup (forward)
@@ -680,11 +945,13 @@ struct BandWork {
   uint64_t key = 0;       // problem uid, block layout and cut setting it was built for
   int32_t nblk = 0, n = 0, bmax = 0;
   int32_t nseg = 0, ncut = 0, ncols = 0;  // segments, blocks cut in two, band columns of all segments
+  int32_t most[2] = {0, 0};               // most columns of a segment factored in phase 0 and 1
   int64_t nband = 0;
   std::vector<int32_t> bw_h, bstart_h;
   DevBuf<int32_t> perm, iperm, cseg;
   DevBuf<BandSeg> seg;
   DevBuf<double> band, y;
+  DevBuf<double> diag;    // per segment: the factored diagonal block of the panel being eliminated
   DevBuf<int32_t> bad;
   DevBuf<int32_t> bok;    // per block: 1 once the band holds its factors
   bool factored = false;  // a factorisation has been enqueued since the layout was built
@@ -888,6 +1155,11 @@ mpf_status band_prepare(mpf_problem* p, const std::vector<int32_t>& node_off) {
   W.nseg = (int32_t)sorted.size();
   W.ncut = ncut;
   W.ncols = ncols;
+  W.most[0] = W.most[1] = 0;
+  for (const BandSeg& g : sorted) {
+    W.most[0] = std::max(W.most[0], g.nf);
+    W.most[1] = std::max(W.most[1], g.nend - g.nf);
+  }
   W.bmax = nblk > 0 ? *std::max_element(bw.begin(), bw.end()) : 0;
   W.nband = nband;
   W.bw_h = bw;
@@ -900,16 +1172,35 @@ mpf_status band_prepare(mpf_problem* p, const std::vector<int32_t>& node_off) {
   MPF_TRY(W.iperm.upload(iperm.data(), iperm.size(), s));
   MPF_TRY(W.cseg.upload(cseg.data(), cseg.size(), s));
   if (!sorted.empty()) MPF_TRY(W.seg.upload(sorted.data(), sorted.size(), s));
-  MPF_TRY(W.band.alloc(W.nband > 0 ? (size_t)W.nband : 1));
+  // a panel's loads take kP columns also where the block has fewer left: in bounds past the last segment's end
+  MPF_TRY(W.band.alloc((size_t)W.nband + (size_t)kP * (W.bmax + 1)));
   MPF_TRY(W.y.alloc(ncols > 0 ? (size_t)ncols : 1));
   MPF_TRY(W.bad.alloc(1));
+  MPF_TRY(W.diag.alloc(std::max<size_t>(sorted.size(), 1) * kP * kP));
   {
     const std::vector<int32_t> zero(std::max(nblk, 1), 0);
     MPF_TRY(W.bok.upload(zero.data(), zero.size(), s));
   }
+  MPF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_band_panel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)kPanelLds));
   MPF_HIP(hipStreamSynchronize(s));
   W.key = key;
   return MPF_OK;
+}
+
+// Factorisation by panels over several workgroups per segment, or by one workgroup per segment?  The panels' workgroups
+// (one per 64 rows of the band) take a compute unit each, so what counts is how often they fill the 256 of the
+// GPU.  Whole direct solves, one workgroup per segment -> panels:
+//   64 x 4 x 8 beams (b 167, three a segment): 80 segments 5.75 -> 4.84 ms, 128 segments 5.93 -> 7.03 ms
+//   64 x 3 x 5 beams (b 95, two): 80 segments 2.65 -> 2.20 ms, 200 segments 2.81 -> 3.34 ms
+//   64 x 2 x 2 beams (b 41, one): 80 segments 0.94 -> 0.82 ms, 400 segments 1.82 -> 1.58 ms
+//   32 x 5 x 8 beams (b 194, four): 80 segments 6.67 -> 4.19 ms, 200 segments 7.15 -> 7.50 ms
+//   8 to 16 x 8 x 8 blocks (b 275, five): 80 segments 6.03 -> 2.75 ms, 400 segments 10.0 -> 9.4 ms
+// so: bands up to 64 and above 255 always, up to 176 (where one workgroup per segment looks ahead) if one round of the
+// compute units holds them, between if two do.
+static bool band_panels(int32_t nseg, int32_t bmax) {
+  const int64_t rounds = ((int64_t)nseg * ((bmax + kStrip - 1) / kStrip) + 255) / 256;
+  return bmax <= kStrip || bmax > 255 || rounds <= (bmax + kW <= 3 * 64 ? 1 : 2);
 }
 
 // Solve phases of every segment with the factors in the band (active as for the factorisation).
@@ -933,7 +1224,7 @@ mpf_status band_enqueue_solve(mpf_problem* p, const int32_t* active, int32_t ast
   if (W->nseg == 0) return MPF_OK;  // no free dofs
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
-  const BandArgs A{W->seg.ptr, W->band.ptr, W->y.ptr, W->bad.ptr};
+  const BandArgs A{W->seg.ptr, W->band.ptr, W->y.ptr, W->bad.ptr, W->diag.ptr};
   static_assert(kFillCols * 494 * sizeof(double) <= 64 * 1024, "the fill's LDS holds columns of b <= 493");
   hipLaunchKernelGGL(k_band_fill, dim3(std::max((W->ncols + kFillCols - 1) / kFillCols, 1)), dim3(256),
                      (size_t)kFillCols * (W->bmax + 1) * sizeof(double), s, W->ncols, W->bmax + 1, W->cseg.ptr,
@@ -942,10 +1233,24 @@ mpf_status band_enqueue_solve(mpf_problem* p, const int32_t* active, int32_t ast
   const size_t lds = (kW + W->bmax <= 3 * 64 ? 2 * ((size_t)(kW + W->bmax) * kW + kW)
                                              : (size_t)(kW + W->bmax) * kW + 3 * kW) * sizeof(double);
   const dim3 g(std::max(W->nseg, 1));
-  hipLaunchKernelGGL(k_band_factor, g, dim3(kFBS), lds, s, A, W->bmax, 0, active, astride, W->bok.ptr);
+  const bool panels = band_panels(W->nseg, W->bmax);
+  const auto factor = [&](int phase) {
+    if (!panels) {
+      hipLaunchKernelGGL(k_band_factor, g, dim3(kFBS), lds, s, A, W->bmax, phase, active, astride, W->bok.ptr);
+      return;
+    }
+    const int tiles = std::max((W->bmax + kTile - 1) / kTile, 1);
+    const dim3 gp(W->nseg, std::max((W->bmax + kStrip - 1) / kStrip, 1)), gt(W->nseg, tiles * (tiles + 1) / 2);
+    for (int q = 0; q * kP < W->most[phase]; ++q) {
+      hipLaunchKernelGGL(k_band_panel, gp, dim3(192), kPanelLds, s, A, phase, q, active, astride,
+                         W->bok.ptr);
+      hipLaunchKernelGGL(k_band_trail, gt, dim3(256), 0, s, A, phase, q, active, astride);
+    }
+  };
+  factor(0);
   if (W->ncut > 0) {
     hipLaunchKernelGGL(k_band_schur, g, dim3(1024), 0, s, A, active, astride);
-    hipLaunchKernelGGL(k_band_factor, g, dim3(kFBS), lds, s, A, W->bmax, 1, active, astride, W->bok.ptr);
+    factor(1);
   }
   enqueue_band_solves(W, A, active, astride, s);
   hipLaunchKernelGGL(k_band_scatter, dim3(grid_for(std::max(W->ncols, 1), 256)), dim3(256), 0, s, W->ncols,
@@ -963,7 +1268,7 @@ mpf_status band_enqueue_resolve(mpf_problem* p) {
   if (!W || !W->factored) return MPF_ERR_STATE;
   if (W->nseg == 0) return MPF_OK;  // no free dofs
   hipStream_t s = p->stream;
-  const BandArgs A{W->seg.ptr, W->band.ptr, W->y.ptr, W->bad.ptr};
+  const BandArgs A{W->seg.ptr, W->band.ptr, W->y.ptr, W->bad.ptr, W->diag.ptr};
   hipLaunchKernelGGL(k_band_rhs, dim3(grid_for(std::max(W->ncols, 1), 256)), dim3(256), 0, s, W->ncols,
                      W->cseg.ptr, W->perm.ptr, p->rhs.ptr, A);
   enqueue_band_solves(W, A, W->bok.ptr, 1, s);

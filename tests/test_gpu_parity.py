@@ -582,6 +582,39 @@ def test_band_cut_block_vs_oracle(mpf, orc, gpu, shape):
     assert normwise_rel(cut, whole) < 1e-12 and not np.array_equal(cut, whole)
 
 
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 1, 1), (16, 1, 1), (9, 2, 3), (6, 3, 3), (13, 4, 3), (7, 5, 5)])
+def test_band_panel_edges_vs_oracle(mpf, orc, gpu, dims):
+    """Factorisation by panels of 64 columns where it can go wrong: fewer rows than a panel, bands
+    narrower than one (1 x 1 and 2 x 3 sections), one strip of 64 rows and a few rows of the next, last panels of any
+    width, separators shorter than a panel; whole and cut blocks.  Bounds as for the other direct solves: an L D L^T
+    of n <= 600 rows leaves a residual of order n eps = 1e-13 relative to the right-hand side (the largest entries
+    are near the diagonal's), the solution within that times the condition number, below 1e3."""
+    size = tuple(0.1 * d for d in dims)
+    m = mpf.matl_from_E_nu(1e3, 0.3, tangent=1)
+    X, conn = mpf.mesh_hex(*dims, L=size, jitter=0.05, seed=3)
+    bcs = [(mpf.face_nodes(mpf.HEX8, *dims, 0), -1, None), (mpf.face_nodes(mpf.HEX8, *dims, 1), 0, 0.005)]
+    P = mpf.Problem(mpf.HEX8, X, conn, m)
+    O = orc.Problem(8, X, conn, m.mu, m.Kinv, m.Utype)
+    O.set_tangent(True)
+    for Q in (P, O):
+        apply_bcs(Q, bcs)
+        Q.prepare_matrix_pattern()
+        Q.set_boundary_conditions(1.0)
+    P.calc_stiffness_and_residual(True, 1.0)
+    vals, rhs = P.system()
+    x_ref, st = O.direct_solve(vals, rhs)
+    assert st == 0
+    for split in (True, False):
+        P.set_band_split(split)
+        assert P.factorise_and_solve(ksp=mpf.KSP_BAND).converged
+        du = P.solution()
+        print(dims, P.band_stats()[1:3], P.band_segments(), flush=True)
+        assert normwise_rel(du, x_ref) < 1e-10
+        assert np.linalg.norm(O.spmv(vals, du) - rhs) / np.linalg.norm(rhs) < 1e-12
+        P.factorise_and_solve(ksp=mpf.KSP_BAND)
+        assert np.array_equal(P.solution(), du)
+
+
 def test_band_rejects_mixed_system(mpf, gpu):
     X, conn = mpf.mesh_tet10(2, jitter=0.1, seed=2)
     P = mpf.Problem(mpf.TET10P1, X, conn, mpf.matl(1.0, 1e-3, 3, mixed=True))
