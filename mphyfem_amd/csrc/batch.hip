@@ -56,7 +56,7 @@ struct BatchWork {
   bool grp_spmv = false;  // every group's rows share one column list (checked once)
   // CG vectors (x is the problem's du)
   DevBuf<double> dinv, r, z, pv, q;
-  DevBuf<double> part;  // [ntiles][2]
+  DevBuf<double> part;  // [ntiles][2], then [ntiles] (p.q of a CG iteration)
   // per-mesh scalars: see the k_b_* kernels for the slots
   DevBuf<double> ms;    // [nmesh][kMS]
   DevBuf<int32_t> mf;   // [nmesh][kMF]
@@ -90,7 +90,7 @@ constexpr int kKs[BatchWork::kNK] = {0, 32, 64, 128, 256, 512, 1024, 2048, 4096}
 
 // per-mesh double slots
 //   kETA forcing term of the last solve, kRNP residual norm before the last solve
-enum { kRZ = 0, kPQ, kRR, kRR0, kAL, kBE, kTOL2, kR0, kRN, kREL, kETA, kRNP, kMS };
+enum { kRZ = 0, kRR0, kTOL2, kR0, kRN, kREL, kETA, kRNP, kMS };
 // per-mesh int slots
 //   kCGA CG running, kNA Newton running, kCGIT CG iterations of the current solve, kNIT Newton
 //   iterations (solves) of the current load step, kDIV diverged, kCGT CG iterations of the load step
@@ -110,6 +110,46 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += sh[w];
   __syncthreads();
   return s;  // valid in thread 0
+}
+
+// Sum of v[0], v[stride], .. v[(n - 1) stride] by the workgroup in a fixed order, in every thread.
+__device__ __forceinline__ double tile_sum(const double* __restrict__ v, int n, int stride, double* sh) {
+  double s = 0.0;
+  for (int t = threadIdx.x; t < n; t += kB) s += v[(size_t)t * stride];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  static_assert(kB == 256, "four wavefronts");
+  __syncthreads();
+  return s;
+}
+
+// A CG iteration is three launches: k_b_spmv (q = A p), k_b_xrz (x, r, z) and k_b_p (p).  The scalars of a mesh are
+// sums over its tiles that every tile's workgroup takes for itself from the launch before, in one fixed order, so
+// that no launch of its own stands between (measured on 24 meshes of 8 to 32 cubed, 136 us an iteration: 34 us were
+// two one-workgroup launches with a serial sum per mesh).  What a launch reads of the mesh's state no workgroup
+// of the same launch changes: the mesh's first tile moves on r.z and the iteration count in k_b_spmv, which reads
+// neither, and clears the running flag in k_b_p, where a workgroup that already sees it cleared stops as it would have.
+struct MeshState {
+  const int32_t* tmesh;  // tile -> mesh
+  const int32_t* mtile;  // mesh -> first tile
+  double* ms;
+  int32_t* mf;
+  double* part;          // per tile r.r, r.z
+  double* pq;            // per tile p.q
+};
+
+// k_b_spmv's share of the mesh's state (tile b of mesh m, p.q of the tile in thread 0)
+__device__ __forceinline__ void spmv_state(const MeshState& M, int b, int m, double dot, double* sh) {
+  if (threadIdx.x == 0) M.pq[b] = dot;
+  const int t0 = M.mtile[m];
+  if (b != t0) return;
+  const double rz = tile_sum(M.part + 2 * t0 + 1, M.mtile[m + 1] - t0, 2, sh);
+  if (threadIdx.x == 0) {
+    M.ms[m * kMS + kRZ] = rz;
+    M.mf[m * kMF + kCGIT] += 1;
+  }
 }
 
 // Jacobi: inverse of the diagonal of every row.
@@ -140,20 +180,18 @@ __global__ void __launch_bounds__(kB) k_b_dot(const int32_t* __restrict__ tlo, c
   if (threadIdx.x == 0) part[2 * b + comp] = v;
 }
 
-// y = A x on the tile's rows (LPR lanes per row) and partial[tile][0] = x . y; skipped for meshes
-// whose CG has stopped.
+// y = A x on the tile's rows (LPR lanes per row) and the tile's x . y; skipped for meshes whose CG has
+// stopped.
 template <int LPR>
 __global__ void __launch_bounds__(kB) k_b_spmv(const int32_t* __restrict__ tlo, const int32_t* __restrict__ thi,
-                                               const int32_t* __restrict__ tmesh, const int32_t* __restrict__ mf,
+                                               MeshState M,
                                                const int32_t* __restrict__ rowptr, const int32_t* __restrict__ colidx,
                                                const double* __restrict__ vals, const double* __restrict__ x,
-                                               double* __restrict__ y, double* __restrict__ part) {
+                                               double* __restrict__ y) {
   __shared__ double sh[kB / 64];
   const int b = blockIdx.x;
-  if (!mf[tmesh[b] * kMF + kCGA]) {
-    if (threadIdx.x == 0) part[2 * b] = 0.0;
-    return;
-  }
+  const int mesh = M.tmesh[b];
+  if (!M.mf[mesh * kMF + kCGA]) return;
   const int g = threadIdx.x / LPR, l = threadIdx.x % LPR;
   double dot = 0.0;
   for (int row = tlo[b] + g; row < thi[b]; row += kB / LPR) {
@@ -166,23 +204,21 @@ __global__ void __launch_bounds__(kB) k_b_spmv(const int32_t* __restrict__ tlo, 
     }
   }
   dot = block_sum(dot, sh);
-  if (threadIdx.x == 0) part[2 * b] = dot;
+  spmv_state(M, b, mesh, dot, sh);
 }
 
 // q = A p over the tile's row groups (a node's free rows share one column list, so each column
 // index and p value is read once for up to three rows); same per-row summation order as k_b_spmv.
 template <int LPR>
 __global__ void __launch_bounds__(kB) k_b_spmv_grp(const int32_t* __restrict__ tg, const int32_t* __restrict__ gs,
-                                                   const int32_t* __restrict__ tmesh, const int32_t* __restrict__ mf,
+                                                   MeshState M,
                                                    const int32_t* __restrict__ rowptr, const int32_t* __restrict__ colidx,
                                                    const double* __restrict__ vals, const double* __restrict__ x,
-                                                   double* __restrict__ y, double* __restrict__ part) {
+                                                   double* __restrict__ y) {
   __shared__ double sh[kB / 64];
   const int b = blockIdx.x;
-  if (!mf[tmesh[b] * kMF + kCGA]) {
-    if (threadIdx.x == 0) part[2 * b] = 0.0;
-    return;
-  }
+  const int mesh = M.tmesh[b];
+  if (!M.mf[mesh * kMF + kCGA]) return;
   const int gi = threadIdx.x / LPR, l = threadIdx.x % LPR;
   double dot = 0.0;
   for (int g = tg[b] + gi; g < tg[b + 1]; g += kB / LPR) {
@@ -210,7 +246,7 @@ __global__ void __launch_bounds__(kB) k_b_spmv_grp(const int32_t* __restrict__ t
     }
   }
   dot = block_sum(dot, sh);
-  if (threadIdx.x == 0) part[2 * b] = dot;
+  spmv_state(M, b, mesh, dot, sh);
 }
 
 // bad[0] = 1 if some group's rows do not share one column list, or a group has more than 3 rows
@@ -255,21 +291,18 @@ __global__ void __launch_bounds__(kB) k_b_start(const int32_t* __restrict__ tlo,
   if (threadIdx.x == 0) { part[2 * b] = rr; part[2 * b + 1] = rz; }
 }
 
-// x += a p, r -= a q, z = D^-1 r; partials r.r and r.z.
+// x += a p, r -= a q, z = D^-1 r, a = r.z / p.q; partials r.r and r.z.
 __global__ void __launch_bounds__(kB) k_b_xrz(const int32_t* __restrict__ tlo, const int32_t* __restrict__ thi,
-                                              const int32_t* __restrict__ tmesh, const int32_t* __restrict__ mf,
-                                              const double* __restrict__ ms, const double* __restrict__ dinv,
-                                              double* __restrict__ x, double* __restrict__ r, double* __restrict__ z,
-                                              const double* __restrict__ p, const double* __restrict__ q,
-                                              double* __restrict__ part) {
+                                              MeshState M, const double* __restrict__ dinv, double* __restrict__ x,
+                                              double* __restrict__ r, double* __restrict__ z,
+                                              const double* __restrict__ p, const double* __restrict__ q) {
   __shared__ double sh[kB / 64];
   const int b = blockIdx.x;
-  const int m = tmesh[b];
-  if (!mf[m * kMF + kCGA]) {
-    if (threadIdx.x == 0) { part[2 * b] = 0.0; part[2 * b + 1] = 0.0; }
-    return;
-  }
-  const double a = ms[m * kMS + kAL];
+  const int m = M.tmesh[b];
+  if (!M.mf[m * kMF + kCGA]) return;
+  const int t0 = M.mtile[m];
+  const double pq = tile_sum(M.pq + t0, M.mtile[m + 1] - t0, 1, sh);
+  const double a = pq != 0.0 ? M.ms[m * kMS + kRZ] / pq : 0.0;
   double rr = 0.0, rz = 0.0;
   for (int i = tlo[b] + threadIdx.x; i < thi[b]; i += kB) {
     x[i] += a * p[i];
@@ -282,17 +315,30 @@ __global__ void __launch_bounds__(kB) k_b_xrz(const int32_t* __restrict__ tlo, c
   }
   rr = block_sum(rr, sh);
   rz = block_sum(rz, sh);
-  if (threadIdx.x == 0) { part[2 * b] = rr; part[2 * b + 1] = rz; }
+  if (threadIdx.x == 0) { M.part[2 * b] = rr; M.part[2 * b + 1] = rz; }
 }
 
+// The mesh's CG test, and p = z + b p, b = r.z / r.z before, where it goes on.
 __global__ void __launch_bounds__(kB) k_b_p(const int32_t* __restrict__ tlo, const int32_t* __restrict__ thi,
-                                            const int32_t* __restrict__ tmesh, const int32_t* __restrict__ mf,
-                                            const double* __restrict__ ms, const double* __restrict__ z,
+                                            MeshState M, int32_t maxit, const double* __restrict__ z,
                                             double* __restrict__ p) {
+  __shared__ double sh[kB / 64];
   const int b = blockIdx.x;
-  const int m = tmesh[b];
-  if (!mf[m * kMF + kCGA]) return;
-  const double be = ms[m * kMS + kBE];
+  const int m = M.tmesh[b];
+  int32_t* F = M.mf + m * kMF;
+  const double* S = M.ms + m * kMS;
+  // the flag may be cleared while the workgroup starts: all its threads take the value that one of them read
+  __shared__ int32_t on;
+  if (threadIdx.x == 0) on = F[kCGA];
+  __syncthreads();
+  if (!on) return;
+  const int t0 = M.mtile[m], nt = M.mtile[m + 1] - t0;
+  const double rr = tile_sum(M.part + 2 * t0, nt, 2, sh), rz = tile_sum(M.part + 2 * t0 + 1, nt, 2, sh);
+  if (rr <= S[kTOL2] * S[kRR0] || F[kCGIT] >= maxit || rr != rr) {
+    if (b == t0 && threadIdx.x == 0) F[kCGA] = 0;
+    return;
+  }
+  const double be = S[kRZ] != 0.0 ? rz / S[kRZ] : 0.0;
   for (int i = tlo[b] + threadIdx.x; i < thi[b]; i += kB) p[i] = z[i] + be * p[i];
 }
 
@@ -382,7 +428,6 @@ __global__ void __launch_bounds__(kB) k_b_start_scalars(int32_t nmesh, const int
     int32_t* F = mf + m * kMF;
     const double rr = mesh_sum(part, mtile, m, 0), rz = mesh_sum(part, mtile, m, 1);
     S[kRR0] = rr;
-    S[kRR] = rr;
     S[kRZ] = rz;
     F[kCGT] += F[kCGIT];
     F[kCGIT] = 0;
@@ -393,32 +438,12 @@ __global__ void __launch_bounds__(kB) k_b_start_scalars(int32_t nmesh, const int
   if (threadIdx.x == 0) cnt[3] = 0;
 }
 
-__global__ void __launch_bounds__(kB) k_b_alpha(int32_t nmesh, const int32_t* __restrict__ mtile,
-                                                const double* __restrict__ part, double* __restrict__ ms,
-                                                const int32_t* __restrict__ mf) {
-  for (int m = threadIdx.x; m < nmesh; m += blockDim.x) {
-    double* S = ms + m * kMS;
-    const double pq = mesh_sum(part, mtile, m, 0);
-    S[kPQ] = pq;
-    S[kAL] = (mf[m * kMF + kCGA] && pq != 0.0) ? S[kRZ] / pq : 0.0;
-  }
-}
-
-__global__ void __launch_bounds__(kB) k_b_beta(int32_t nmesh, const int32_t* __restrict__ mtile,
-                                               const double* __restrict__ part, double* __restrict__ ms,
-                                               int32_t* __restrict__ mf, int32_t maxit, int32_t* __restrict__ cnt) {
+// after the CG iterations of a graph: meshes still running, most iterations of one mesh
+__global__ void __launch_bounds__(kB) k_b_count(int32_t nmesh, const int32_t* __restrict__ mf,
+                                                int32_t* __restrict__ cnt) {
   int32_t act = 0, most = 0;
   for (int m = threadIdx.x; m < nmesh; m += blockDim.x) {
-    double* S = ms + m * kMS;
-    int32_t* F = mf + m * kMF;
-    if (F[kCGA]) {
-      const double rr = mesh_sum(part, mtile, m, 0), rz = mesh_sum(part, mtile, m, 1);
-      F[kCGIT] += 1;
-      S[kRR] = rr;
-      S[kBE] = S[kRZ] != 0.0 ? rz / S[kRZ] : 0.0;
-      S[kRZ] = rz;
-      if (rr <= S[kTOL2] * S[kRR0] || F[kCGIT] >= maxit || rr != rr) F[kCGA] = 0;
-    }
+    const int32_t* F = mf + m * kMF;
     act += F[kCGA];
     most = max(most, F[kNA] ? F[kCGIT] : 0);
   }
@@ -469,7 +494,7 @@ mpf_status build_tiles(BatchWork& B, int T, hipStream_t s) {
   MPF_TRY(B.thi.upload(hi.data(), hi.size(), s));
   MPF_TRY(B.tmesh.upload(tm.data(), tm.size(), s));
   MPF_TRY(B.mtile.upload(mt.data(), mt.size(), s));
-  MPF_TRY(B.part.alloc((size_t)std::max(B.ntiles, 1) * 2));
+  MPF_TRY(B.part.alloc((size_t)std::max(B.ntiles, 1) * 3));
   MPF_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
   return MPF_OK;
 }
@@ -479,41 +504,47 @@ mpf_status enqueue_cg_iter(mpf_problem* p, BatchWork& B, int32_t maxit) {
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
   const dim3 gt(std::max(B.ntiles, 1)), bt(kB);
+  const MeshState M{B.tmesh.ptr, B.mtile.ptr, B.ms.ptr, B.mf.ptr, B.part.ptr, B.part.ptr + 2 * (size_t)B.ntiles};
   if (B.grp_spmv) {
     switch (B.LPR) {
       case 4:
-        hipLaunchKernelGGL(k_b_spmv_grp<4>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, B.tmesh.ptr, B.mf.ptr, P.rowptr.ptr,
-                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
+        hipLaunchKernelGGL(k_b_spmv_grp<4>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
+                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       case 16:
-        hipLaunchKernelGGL(k_b_spmv_grp<16>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, B.tmesh.ptr, B.mf.ptr, P.rowptr.ptr,
-                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
+        hipLaunchKernelGGL(k_b_spmv_grp<16>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
+                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       default:
-        hipLaunchKernelGGL(k_b_spmv_grp<8>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, B.tmesh.ptr, B.mf.ptr, P.rowptr.ptr,
-                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
+        hipLaunchKernelGGL(k_b_spmv_grp<8>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
+                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
     }
   } else {
     switch (B.LPR) {
       case 4:
-        hipLaunchKernelGGL(k_b_spmv<4>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, B.tmesh.ptr, B.mf.ptr, P.rowptr.ptr,
-                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
+        hipLaunchKernelGGL(k_b_spmv<4>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
+                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       case 16:
-        hipLaunchKernelGGL(k_b_spmv<16>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, B.tmesh.ptr, B.mf.ptr, P.rowptr.ptr,
-                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
+        hipLaunchKernelGGL(k_b_spmv<16>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
+                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       default:
-        hipLaunchKernelGGL(k_b_spmv<8>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, B.tmesh.ptr, B.mf.ptr, P.rowptr.ptr,
-                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
+        hipLaunchKernelGGL(k_b_spmv<8>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
+                           P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
     }
   }
-  hipLaunchKernelGGL(k_b_alpha, dim3(1), bt, 0, s, B.nmesh, B.mtile.ptr, B.part.ptr, B.ms.ptr, B.mf.ptr);
-  hipLaunchKernelGGL(k_b_xrz, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, B.tmesh.ptr, B.mf.ptr, B.ms.ptr, B.dinv.ptr,
-                     p->du.ptr, B.r.ptr, B.z.ptr, B.pv.ptr, B.q.ptr, B.part.ptr);
-  hipLaunchKernelGGL(k_b_beta, dim3(1), bt, 0, s, B.nmesh, B.mtile.ptr, B.part.ptr, B.ms.ptr, B.mf.ptr, maxit,
-                     B.cnt.ptr);
-  hipLaunchKernelGGL(k_b_p, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, B.tmesh.ptr, B.mf.ptr, B.ms.ptr, B.z.ptr, B.pv.ptr);
+  hipLaunchKernelGGL(k_b_xrz, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, B.dinv.ptr, p->du.ptr, B.r.ptr, B.z.ptr,
+                     B.pv.ptr, B.q.ptr);
+  hipLaunchKernelGGL(k_b_p, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, maxit, B.z.ptr, B.pv.ptr);
+  MPF_HIP(hipGetLastError());
+  return MPF_OK;
+}
+
+// k CG iterations of every active mesh, and the counts that the host reads after them.
+mpf_status enqueue_cg_iters(mpf_problem* p, BatchWork& B, int32_t k, int32_t maxit) {
+  for (int32_t i = 0; i < k; ++i) MPF_TRY(enqueue_cg_iter(p, B, maxit));
+  hipLaunchKernelGGL(k_b_count, dim3(1), dim3(kB), 0, p->stream, B.nmesh, B.mf.ptr, B.cnt.ptr);
   MPF_HIP(hipGetLastError());
   return MPF_OK;
 }
@@ -834,15 +865,11 @@ static mpf_status batch_step(mpf_problem* p, double lam, const mpf_batch_opts* o
     MPF_TRY(enqueue_newton_head(p, B, v == 0, lam, o->rtol, o->cg_rtol, !band));
     if (kidx > 0) {
       if (band) MPF_TRY(band_enqueue_solve(p, B.mf.ptr + kNA, kMF));
-      else
-        for (int k = 0; k < kKs[kidx]; ++k) MPF_TRY(enqueue_cg_iter(p, B, o->cg_maxit));
+      else MPF_TRY(enqueue_cg_iters(p, B, kKs[kidx], o->cg_maxit));
     }
     return MPF_OK;
   };
-  auto chunk_work = [&]() -> mpf_status {
-    for (int k = 0; k < B.chunk; ++k) MPF_TRY(enqueue_cg_iter(p, B, o->cg_maxit));
-    return MPF_OK;
-  };
+  auto chunk_work = [&]() -> mpf_status { return enqueue_cg_iters(p, B, B.chunk, o->cg_maxit); };
   if (G && (B.g_solver != o->solver || B.g_rtol != o->rtol || B.g_cg_rtol != o->cg_rtol ||
             B.g_cg_maxit != o->cg_maxit)) {
     B.release_graphs();
