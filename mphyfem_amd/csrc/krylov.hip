@@ -45,7 +45,7 @@ struct KrylovWork {
 namespace {
 
 // scalar slots
-enum { S_RZ0 = 0, S_RZ1 = 1, S_PQ = 2, S_RR = 3, S_BB = 4, S_DONE = 5, S_ITS = 6, S_TOL2 = 7, S_MAXIT = 8, S_N = 16 };
+enum { S_RZ0 = 0, S_RZ1 = 1, S_RR = 3, S_BB = 4, S_DONE = 5, S_ITS = 6, S_TOL2 = 7, S_MAXIT = 8, S_N = 16 };
 static_assert(S_N == kCgScalars, "CG scalar slots");
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -62,6 +62,19 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
   double s = 0.0;
   if (threadIdx.x == 0)
     for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += sh[i];
+  __syncthreads();
+  return s;
+}
+
+// Sum of v[0 .. n) by the workgroup in a fixed order, in every thread.
+__device__ __forceinline__ double parts_sum(const double* __restrict__ v, int n, double* sh) {
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += kRB) s += v[i];
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = 0.0;
+  for (int i = 0; i < kRB / 64; ++i) s += sh[i];
   __syncthreads();
   return s;
 }
@@ -239,17 +252,18 @@ __global__ void __launch_bounds__(kRB) k_cg_start(int64_t nblk, const int32_t* _
 
 // One thread per row: x += alpha p ; r_out = r_in - alpha q ; z = M r_out with the row's 3x3 block
 // (its block's r_in and q are read, only the row itself is written, so rows of one block never
-// race); partials of r.z and r.r.   alpha = rz[par] / pq
+// race); partials of r.z and r.r.   alpha = rz[par] / pq, p.q summed from its npq partials
 __global__ void __launch_bounds__(kRB) k_cg_update_rows(int64_t n, const int32_t* __restrict__ rblk,
                                                         const int32_t* __restrict__ bs, const int32_t* __restrict__ bm,
                                                         const double* __restrict__ binv, double* __restrict__ x,
                                                         const double* __restrict__ rin, double* __restrict__ rout,
                                                         double* __restrict__ z, const double* __restrict__ p,
                                                         const double* __restrict__ q, double* __restrict__ part, int np,
+                                                        const double* __restrict__ pq, int npq,
                                                         const double* __restrict__ sc, int par) {
   if (sc[S_DONE] != 0.0) return;
   __shared__ double sh[kRB / 64];
-  const double alpha = sc[S_RZ0 + par] / sc[S_PQ];
+  const double alpha = sc[S_RZ0 + par] / parts_sum(pq, npq, sh);
   double rz = 0.0, rr = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * kRB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRB) {
     x[i] += alpha * p[i];
@@ -282,28 +296,26 @@ __global__ void k_row_blk(int64_t nblk, const int32_t* __restrict__ bs, const in
   for (int j = 0; j < bm[k]; ++j) rblk[bs[k] + j] = (int32_t)k;
 }
 
-// reduce the two partial arrays into rz[1-par], rr; convergence test
-__global__ void __launch_bounds__(kRB) k_cg_check(const double* __restrict__ part, int np, double* __restrict__ sc,
-                                                  int par, int it) {
-  if (sc[S_DONE] != 0.0) return;
-  __shared__ double sh[kRB / 64];
-  double s1 = 0.0, s2 = 0.0;
-  for (int i = threadIdx.x; i < np; i += kRB) { s1 += part[i]; s2 += part[np + i]; }
-  const double t1 = block_sum(s1, sh);
-  const double t2 = block_sum(s2, sh);
-  if (threadIdx.x == 0) {
-    sc[S_RZ0 + (1 - par)] = t1;
-    sc[S_RR] = t2;
-    sc[S_ITS] = (double)(it + 1);
-    if (t2 <= sc[S_TOL2] || (double)(it + 1) >= sc[S_MAXIT] || !(t2 == t2)) sc[S_DONE] = 1.0;
-  }
-}
-
-// p = z + beta p,  beta = rz[1-par] / rz[par]
+// Convergence test of iteration it, and where it goes on p = z + beta p, beta = rz[1-par] / rz[par].  Every
+// workgroup sums the partials of r.z and r.r itself, in one fixed order, and the first leaves them and the outcome in
+// sc: of those no other workgroup reads but S_DONE, and one that already sees it set stops as it would have.
 __global__ void __launch_bounds__(kRB) k_cg_p(int64_t n, const double* __restrict__ z, double* __restrict__ p,
-                                              const double* __restrict__ sc, int par) {
-  if (sc[S_DONE] != 0.0) return;
-  const double beta = sc[S_RZ0 + (1 - par)] / sc[S_RZ0 + par];
+                                              const double* __restrict__ part, int np, double* sc, int par, int it) {
+  __shared__ double sh[kRB / 64];
+  __shared__ int done;  // one thread's reading for all
+  if (threadIdx.x == 0) done = sc[S_DONE] != 0.0;
+  __syncthreads();
+  if (done) return;
+  const double rz = parts_sum(part, np, sh), rr = parts_sum(part + np, np, sh);
+  const bool stop = rr <= sc[S_TOL2] || (double)(it + 1) >= sc[S_MAXIT] || !(rr == rr);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[S_RZ0 + (1 - par)] = rz;
+    sc[S_RR] = rr;
+    sc[S_ITS] = (double)(it + 1);
+    if (stop) sc[S_DONE] = 1.0;
+  }
+  if (stop) return;
+  const double beta = rz / sc[S_RZ0 + par];
   for (int64_t i = (int64_t)blockIdx.x * kRB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRB)
     p[i] = z[i] + beta * p[i];
 }
@@ -741,17 +753,20 @@ mpf_status pcg_csr(const CsrView& A, const BlockPcView& B, const CgScratch& w, c
   int it = 0;
   int chunk = 8;
   double hs[S_N];
-  const unsigned nsp = spmv_parts(A, B);
+  // An iteration is three launches; k_cg_update_rows and k_cg_p take the sums they need from the partials of the launch
+  // before, which every workgroup reads: as few as still fill the GPU.  (48^3 Hex8, us a launch that runs: 2048 and 1024 partials
+  // product 57.7, update 14.2, p 6.9; 4096 and 1342: 59.0, 15.3, 8.0; 1024 and 512: 81.0, 14.6, 5.9.  As five launches with one
+  // workgroup's sums between: 91 us an iteration with the launches' gaps, now 79.)
+  const unsigned nsp = std::min(spmv_parts(A, B), 2048u), nv = std::min(nps, 1024u);
+  double* pq = w.part + 2 * (size_t)kMaxParts;  // r.z and r.r before it
   for (;;) {
     for (int c = 0; c < chunk; ++c, ++it) {
       const int par = it & 1;
-      MPF_TRY(spmv_view(A, B, w.p, w.q, w.part, nsp, sc, s));
-      hipLaunchKernelGGL(k_finish, dim3(1), dim3(kRB), 0, s, w.part, (int)nsp, (int)nsp, 1, sc + S_PQ);
+      MPF_TRY(spmv_view(A, B, w.p, w.q, pq, nsp, sc, s));
       double* rb[2] = {w.r, w.r2};
-      hipLaunchKernelGGL(k_cg_update_rows, dim3(nps), dim3(kRB), 0, s, n, B.rblk, B.bs, B.bm, B.binv, x, rb[par],
-                         rb[1 - par], w.z, w.p, w.q, w.part, (int)nps, sc, par);
-      hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(kRB), 0, s, w.part, (int)nps, sc, par, it);
-      hipLaunchKernelGGL(k_cg_p, dim3(nps), dim3(kRB), 0, s, n, w.z, w.p, sc, par);
+      hipLaunchKernelGGL(k_cg_update_rows, dim3(nv), dim3(kRB), 0, s, n, B.rblk, B.bs, B.bm, B.binv, x, rb[par],
+                         rb[1 - par], w.z, w.p, w.q, w.part, (int)nv, pq, (int)nsp, sc, par);
+      hipLaunchKernelGGL(k_cg_p, dim3(nv), dim3(kRB), 0, s, n, w.z, w.p, w.part, (int)nv, sc, par, it);
     }
     MPF_HIP(hipMemcpyAsync(hs, sc, sizeof(hs), hipMemcpyDeviceToHost, s));
     MPF_HIP(hipStreamSynchronize(s));
