@@ -452,15 +452,32 @@ __global__ void k_row_blocks(int64_t nb0, int64_t count, int32_t row0, int32_t* 
 
 // ---- GMRES helpers ----
 // h[j] partials: part[j*np + b] = sum_i V_j[i] w[i] for j <= jmax
+// kMV vectors a pass: their loads in flight together and one round of sums (16^3 Tet10/P1 cells, 1.2e5 rows, 1 to 30
+// vectors: 39.6 us at a vector a pass, 21.8 us at 8, 31 us at 16 and 35 us at 32, where the sums across lanes of vectors
+// past the last one cost more than the passes they save).
+constexpr int kMV = 8;
 __global__ void __launch_bounds__(kRB) k_multidot(int64_t n, int nv, const double* __restrict__ V,
                                                   const double* __restrict__ w, double* __restrict__ part, int np) {
-  __shared__ double sh[kRB / 64];
-  for (int j = 0; j < nv; ++j) {
-    const double* v = V + (size_t)j * n;
-    double s = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * kRB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRB) s += v[i] * w[i];
-    const double t = block_sum(s, sh);
-    if (threadIdx.x == 0) part[(size_t)j * np + blockIdx.x] = t;
+  __shared__ double sh[kMV][kRB / 64];
+  for (int j0 = 0; j0 < nv; j0 += kMV) {
+    double s[kMV] = {};
+    for (int64_t i = (int64_t)blockIdx.x * kRB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRB) {
+      const double wi = w[i];
+#pragma unroll
+      for (int u = 0; u < kMV; ++u) s[u] += V[(size_t)min(j0 + u, nv - 1) * n + i] * wi;  // past nv: not stored
+    }
+#pragma unroll
+    for (int u = 0; u < kMV; ++u) {
+      s[u] = wave_sum(s[u]);
+      if ((threadIdx.x & 63) == 0) sh[u][threadIdx.x >> 6] = s[u];
+    }
+    __syncthreads();
+    if (threadIdx.x < kMV && j0 + (int)threadIdx.x < nv) {
+      double t = 0.0;
+      for (int v = 0; v < kRB / 64; ++v) t += sh[threadIdx.x][v];
+      part[(size_t)(j0 + threadIdx.x) * np + blockIdx.x] = t;
+    }
+    __syncthreads();
   }
 }
 
@@ -469,6 +486,7 @@ __global__ void __launch_bounds__(kRB) k_multiaxpy(int64_t n, int nv, const doub
                                                    const double* __restrict__ h, double* __restrict__ w) {
   for (int64_t i = (int64_t)blockIdx.x * kRB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRB) {
     double s = w[i];
+#pragma unroll 8
     for (int j = 0; j < nv; ++j) s -= h[j] * V[(size_t)j * n + i];
     w[i] = s;
   }
@@ -739,11 +757,12 @@ static mpf_status setup_work(mpf_problem* p, int pc, int restart) {
 }
 
 mpf_status pcg_csr(const CsrView& A, const BlockPcView& B, const CgScratch& w, const double* b, double* x,
-                   double rtol, int maxit, hipStream_t s, mpf_krylov_report* rep) {
+                   double rtol, int maxit, hipStream_t s, mpf_krylov_report* rep, int first) {
   const int64_t n = A.n;
   const unsigned np = nparts_for(B.nblk);
   const unsigned nps = nparts_for(n);
   double* sc = w.sc;
+  double hs[S_N];
   hipLaunchKernelGGL(k_cg_start, dim3(np), dim3(kRB), 0, s, B.nblk, B.bs, B.bm, B.binv, b, x, w.r, w.z, w.p, w.part,
                      (int)np);
   // rz -> sc[S_RZ0], bb -> sc[S_RR]
@@ -751,8 +770,8 @@ mpf_status pcg_csr(const CsrView& A, const BlockPcView& B, const CgScratch& w, c
   hipLaunchKernelGGL(k_finish, dim3(1), dim3(kRB), 0, s, w.part + np, (int)np, (int)np, 1, sc + S_RR);
   hipLaunchKernelGGL(k_cg_init_scalars, dim3(1), dim3(64), 0, s, sc, rtol, maxit);
   int it = 0;
-  int chunk = 8;
-  double hs[S_N];
+  // launched ahead of each look at the outcome: `first` iterations, then 16, 32, 64, 64 ..; after a caller's own guess 8, 16 ..
+  int chunk = first > 0 ? first : 8, next = first > 0 ? 8 : 16;
   // An iteration is three launches; k_cg_update_rows and k_cg_p take the sums they need from the partials of the launch
   // before, which every workgroup reads: as few as still fill the GPU.  (48^3 Hex8, us a launch that runs: 2048 and 1024 partials
   // product 57.7, update 14.2, p 6.9; 4096 and 1342: 59.0, 15.3, 8.0; 1024 and 512: 81.0, 14.6, 5.9.  As five launches with one
@@ -771,7 +790,8 @@ mpf_status pcg_csr(const CsrView& A, const BlockPcView& B, const CgScratch& w, c
     MPF_HIP(hipMemcpyAsync(hs, sc, sizeof(hs), hipMemcpyDeviceToHost, s));
     MPF_HIP(hipStreamSynchronize(s));
     if (hs[S_DONE] != 0.0) break;
-    if (chunk < 64) chunk *= 2;
+    chunk = next;
+    next = std::min(64, 2 * next);
   }
   MPF_HIP(hipGetLastError());
   const double bb = hs[S_BB];

@@ -259,12 +259,13 @@ struct BlockPcView {
   bool grp = false;               // every block's rows share one column list (row-group SpMV)
 };
 constexpr int kCgScalars = 16;    // device scalars of one CG run
-struct CgScratch {                // n doubles each; part: 2 * kMaxPartials; sc: kCgScalars
+struct CgScratch {                // n doubles each; part: 3 * kMaxPartials; sc: kCgScalars
   double *r, *r2, *z, *p, *q, *part, *sc;
 };
-// Block-preconditioned CG from x = 0 to ||b - A x|| <= rtol ||b|| or maxit iterations.
+// Block-preconditioned CG from x = 0 to ||b - A x|| <= rtol ||b|| or maxit iterations.  first: iterations to launch
+// before the outcome is first looked at, where the caller can guess them (those past the last one do nothing); 0: 8.
 mpf_status pcg_csr(const CsrView& A, const BlockPcView& B, const CgScratch& w, const double* b, double* x,
-                   double rtol, int maxit, hipStream_t s, mpf_krylov_report* rep);
+                   double rtol, int maxit, hipStream_t s, mpf_krylov_report* rep, int first = 0);
 // Block structure set-up: rblk from (bs, bm); *grp = 1 when every block's rows share one column list.
 mpf_status block_pc_structure(const CsrView& A, int64_t nblk, const int32_t* bs, const int32_t* bm,
                               int32_t* rblk, bool* grp, hipStream_t s);

@@ -91,6 +91,7 @@ struct PmgWork {
   double lambda_c = 0.0;                   // largest eigenvalue of Bc^-1 Kc
   // statistics of the current solve
   int64_t vcycles = 0, coarse_its = 0;
+  int32_t coarse_last = 0;  // iterations of the last coarse solve since the set-up
   double setup_seconds = 0.0;
 };
 
@@ -923,6 +924,7 @@ mpf_status pmg_setup(mpf_problem* p, const BlockPcView& F, int64_t nub) {
     MPF_TRY(build_tables(p, W));
   W.vcycles = 0;
   W.coarse_its = 0;
+  W.coarse_last = 0;
   const CsrView A = fine_csr(p);
   int32_t hbad = 0;
   MPF_HIP(hipMemcpyAsync(W.bad.ptr, &hbad, sizeof(int32_t), hipMemcpyHostToDevice, s));
@@ -991,6 +993,9 @@ mpf_status pmg_apply(mpf_problem* p, const BlockPcView& F, int64_t nub, const do
                      W.res.ptr, W.rc.ptr);
   const CgScratch cw{W.cr.ptr, W.cr2.ptr, W.cz.ptr, W.cp.ptr, W.cq.ptr, W.cpart.ptr, W.csc.ptr};
   mpf_krylov_report cr{};
+  // the coarse solves of one Krylov run take nearly the same number of iterations: two more than the last one's are
+  // launched before the first look at the outcome (16^3 Tet10/P1 cells, 12 to 13 iterations: 24 were launched, in two looks)
+  const int guess = W.coarse_last > 0 ? std::min(W.coarse_last + 2, 64) : 0;
   if (W.levels == 3 && W.na > 0) {
     // the vertex level's own V-cycle: Chebyshev smoothing from 0, the aggregates' correction (Ka
     // by block-Jacobi CG to crtol), Chebyshev smoothing again, the result in xc
@@ -1010,7 +1015,7 @@ mpf_status pmg_apply(mpf_problem* p, const BlockPcView& F, int64_t nub, const do
     launch_sweep<2>(lc, ncb, Cb, Cv, W.cval32.ptr, W.culen.ptr, 0.0, 0.0, W.rc.ptr, xc0, W.cres.ptr, nullptr, s);
     hipLaunchKernelGGL(k_agg_restrict, dim3(grid_for(W.na, kT)), dim3(kT), 0, s, W.na, W.amptr.ptr, W.amem.ptr,
                        W.cres.ptr, W.ra.ptr);
-    MPF_TRY(pcg_csr(agg_csr(W), agg_blocks(W), cw, W.ra.ptr, W.xa3.ptr, W.crtol, W.cmaxit, s, &cr));
+    MPF_TRY(pcg_csr(agg_csr(W), agg_blocks(W), cw, W.ra.ptr, W.xa3.ptr, W.crtol, W.cmaxit, s, &cr, guess));
     hipLaunchKernelGGL(k_agg_prolong, dim3(grid_for(nc, kT)), dim3(kT), 0, s, nc, W.aoff.ptr, W.xa3.ptr, xc0);
     for (int k = 0; k < W.degree; ++k) {
       double* out = (k == W.degree - 1) ? W.xc.ptr : xc1;
@@ -1019,9 +1024,10 @@ mpf_status pmg_apply(mpf_problem* p, const BlockPcView& F, int64_t nub, const do
       xc0 = out;
     }
   } else {
-    MPF_TRY(pcg_csr(coarse_csr(W), coarse_blocks(W), cw, W.rc.ptr, W.xc.ptr, W.crtol, W.cmaxit, s, &cr));
+    MPF_TRY(pcg_csr(coarse_csr(W), coarse_blocks(W), cw, W.rc.ptr, W.xc.ptr, W.crtol, W.cmaxit, s, &cr, guess));
   }
   W.coarse_its += cr.iterations;
+  W.coarse_last = cr.iterations;
   hipLaunchKernelGGL(k_prolong, dim3(grid_for(d, kT)), dim3(kT), 0, s, d, W.pidx.ptr, W.pw.ptr, W.xc.ptr, cur);
   // post-smoothing from the corrected x, the last step into z
   for (int k = 0; k < W.degree; ++k) {
