@@ -681,19 +681,21 @@ __global__ void __launch_bounds__(256) k_band_trail(BandArgs A, int32_t phase, i
 // [c0, c1): forward L z = y, then z / d; backward L^T x = z, rows past c1 already solved.
 
 // Band entries of forward block step j0 (w rows): thread gt of a group holds coupling row
-// j0 + w + gt's entries in lc (zero outside the band), the group's wavefront 0 lane r row r of the
-// unit triangle in l.
+// j0 + w + gt's entries in lc, the group's wavefront 0 lane r row r of the unit triangle in l.  Entry (r, c) lies at
+// c (B1 - 1) + r: a uniform base and the lane's row.  Loaded without a test per entry (rows past the window: its last
+// row; past the band: any entry in the storage), tested where they are used: the tests and branches of the loads cost
+// more of a block step than its products (a launch on average, half-bandwidth 353: 202 -> 160 us; 40 beams of
+// half-bandwidth 167: 537 -> 451 us).
 __device__ __forceinline__ void fwd_entries(const double* L, int B1, int b, int n, int j0, int w, int gt, int gw,
                                             int lane, double (&lc)[kW], double (&l)[kW]) {
-  const int r = j0 + w + gt;
-  const bool crow = r < min(n, j0 + w + b);
+  const double* L0 = L + (size_t)j0 * B1;
+  const uint32_t r = (uint32_t)(min(j0 + w + gt, min(n, j0 + w + b) - 1) - j0);
 #pragma unroll
-  for (int k = 0; k < kW; ++k)
-    lc[k] = (crow && k < w && r - (j0 + k) <= b) ? L[(size_t)(j0 + k) * B1 + (r - (j0 + k))] : 0.0;
+  for (int k = 0; k < kW; ++k) lc[k] = (L0 + (size_t)k * (B1 - 1))[r];
   if (gw == 0) {
+    const uint32_t q = (uint32_t)min(lane, w - 1);
 #pragma unroll
-    for (int c = 0; c < kW; ++c)
-      l[c] = (lane < w && c < lane && lane - c <= b) ? L[(size_t)(j0 + c) * B1 + (lane - c)] : 0.0;
+    for (int c = 0; c < kW; ++c) l[c] = (L0 + (size_t)c * (B1 - 1))[q];
   }
 }
 
@@ -712,7 +714,7 @@ static_assert(kRing >= 2 * (493 + kW), "the ring holds the window and the rows l
 __device__ __forceinline__ void band_forward(const double* L, double* y, double* sy, double* ring, int n, int b,
                                              int c0, int c1, int tid, int wid, int lane) {
   const int B1 = b + 1;
-  const int g = tid / (kBS / 2), gt = tid % (kBS / 2), gw = gt >> 6;
+  const int g = wid / (kBS / 128), gt = tid % (kBS / 2), gw = wid % (kBS / 128);
   const int nsteps = (c1 - c0 + kW - 1) / kW;
   for (int i = tid; i < kRing; i += kBS) ring[(c0 + i) % kRing] = c0 + i < n ? y[c0 + i] : 0.0;
   double lc[kW], l[kW];
@@ -731,7 +733,7 @@ __device__ __forceinline__ void band_forward(const double* L, double* y, double*
       for (int c = 0; c < kW; ++c) {
         if (c < w) {
           const double zc = lane_value(z, c);
-          if (lane > c) z -= l[c] * zc;
+          if (lane > c && lane <= c + b) z -= l[c] * zc;
         }
       }
       if (lane < w) {
@@ -742,9 +744,14 @@ __device__ __forceinline__ void band_forward(const double* L, double* y, double*
     __syncthreads();
     if (crow) {
       double acc = ring[r % kRing];
+      if (w == kW && (gw + 1) * 64 - 1 + w <= b) {  // every row of the wavefront in the band in every column
 #pragma unroll
-      for (int k = 0; k < kW; ++k)
-        if (k < w) acc -= lc[k] * sy[k];  // lc is 0 beyond the band
+        for (int k = 0; k < kW; ++k) acc -= lc[k] * sy[k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < kW; ++k)
+          if (k < w && w + gt - k <= b) acc -= lc[k] * sy[k];
+      }
       ring[r % kRing] = acc;
     }
     // the last wavefront (a coupling row only in bands wider than kBS / 2 - 64, so its wait for the row
@@ -787,7 +794,8 @@ __device__ __forceinline__ void bwd_entries(const double* L, const double* y, in
 #pragma unroll
   for (int t = 0; t < kBRow; ++t) {
     const int r = j0 + w + lane + 64 * t;
-    v[t] = (wid < w && r <= min(n - 1, k + b)) ? L[(size_t)k * B1 + (r - k)] : 0.0;
+    // uniform: some lane's row is in the band; past it any entry in the storage, not used
+    if (wid < w && w + 64 * t - wid <= b) v[t] = (L + (size_t)k * (B1 - 1))[(uint32_t)min(r, n - 1)];
   }
   yk = wid < w ? y[k] : 0.0;
 }
@@ -809,9 +817,9 @@ __device__ __forceinline__ void band_backward(const double* L, double* y, double
     const int j0 = q * kW, w = min(kW, c1 - j0);
     double lt[kW];  // wavefront 0, lane r: L(c, r), c > r, loaded before the row sums
     if (wid == 0) {
+      const double* Lr = L + (size_t)(j0 + min(lane, w - 1)) * (B1 - 1) + j0;  // entry (j0 + c, j0 + lane) at c
 #pragma unroll
-      for (int c = 0; c < kW; ++c)
-        lt[c] = (lane < w && c < w && c > lane && c - lane <= b) ? L[(size_t)(j0 + lane) * B1 + (c - lane)] : 0.0;
+      for (int c = 0; c < kW; ++c) lt[c] = Lr[c];
     }
     if (q > c0 / kW) bwd_entries(L, y, B1, b, n, j0 - kW, kW, wid, lane, vn, ykn);
     if (wid < w) {  // row j0 + wid: minus the rows already solved beyond the block
@@ -832,7 +840,7 @@ __device__ __forceinline__ void band_backward(const double* L, double* y, double
       for (int c = kW - 1; c >= 0; --c) {
         if (c < w) {
           const double xc = lane_value(x, c);
-          if (lane < c) x -= lt[c] * xc;
+          if (lane < c && c <= lane + b) x -= lt[c] * xc;
         }
       }
       if (lane < w) {
@@ -857,7 +865,7 @@ __global__ void __launch_bounds__(kBS) k_band_solve(BandArgs A, int32_t mode, co
   __shared__ double ring[kRing];
   const BandSeg S = A.seg[blockIdx.x];
   if (active && !active[(size_t)S.blk * astride]) return;
-  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const double* L = A.band + S.boff;
   double* y = A.y + S.yoff;
   if (mode == 0) {
