@@ -10,8 +10,9 @@
 // Converged meshes are masked out of the remaining work.
 //
 // Vector work is organised in tiles: contiguous dof ranges inside one mesh (meshes own contiguous dof
-// ranges because free dofs are numbered node-major).  One workgroup per tile; per-tile partial dot
-// products are reduced per mesh in tile order, so every reduction is deterministic.
+// ranges because free dofs are numbered node-major).  One workgroup per tile (several
+// for the matrix product); per-tile partial dot products are reduced per mesh in a fixed order, so every
+// reduction is deterministic.
 //
 // One Newton iteration of the whole batch is one graph launch and one 16-byte read-back: the update
 // of the previous iteration's solve, the assembly, residual norms, Newton test and CG start, then K
