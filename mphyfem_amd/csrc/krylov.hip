@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(kRB) k_spmv(int64_t n, const int32_t* __restri
 // pressure row), which share one column list, so each column index and x value is read once for
 // up to three rows.  Entries go to the LPR lanes as in k_spmv (same per-row summation order);
 // part[b] = sum over the block's rows of x_r y_r (when part != null).  Bound by the values from HBM; the loads take
-// no branch on the block's number of rows, so that a lane's stay in flight together (48^3 Hex8, 9.1 M block entries,
+// no branch on the block's number of rows, so that a lane's stay in flight together (48^3 Hex8, 3.4e5 rows,
 // 61.5 -> 56.0 us, 4.7 TB/s).
 template <int LPR, typename V = double>
 __global__ void __launch_bounds__(kRB) k_spmv_grp(int64_t nblk, const int32_t* __restrict__ bs,
