@@ -55,6 +55,7 @@ struct BatchWork {
   std::vector<int32_t> gs_h;
   DevBuf<int32_t> gs, tg;
   bool grp_spmv = false;  // every group's rows share one column list (checked once)
+  int32_t tile_groups = 0, mesh_tiles = 0;  // most row groups of a tile, most tiles of a mesh
   // CG vectors (x is the problem's du)
   DevBuf<double> dinv, r, z, pv, q;
   DevBuf<double> part;  // [ntiles][2], then [ntiles][parts] (p.q of a CG iteration)
@@ -146,8 +147,15 @@ struct MeshState {
 // k_b_spmv's workgroups per tile: enough that each takes one round of the row groups that it holds at a time.  With
 // one per tile a workgroup's rounds (11 for 1024 dofs and 8 lanes a row) ran one after the other, and where few
 // meshes still iterate few workgroups were left (24 meshes of 8 to 32 cubed: 280 us with all of them, 120 us with the last
-// ones; 235 and 20 us in parts of one round, 247 and 28 us of two, 265 and 50 us of four).
-inline int32_t spmv_parts(int T, int lpr) { return T / 3 * lpr / kB + 1; }
+// ones; 235 and 20 us in parts of one round, 247 and 28 us of two, 265 and 50 us of four).  Counted from the longest
+// tile there is: the tile length that a caller gives may be far above every mesh's.  At most kMaxMeshParts partial sums a
+// mesh, since each of its tiles' workgroups sums them all (one mesh of 64 cubed: 188 us an iteration without the limit,
+// 186 with it; 96: 610 and 593; 120: 1204 and 1151; meshes up to 32 cubed stay below it).
+constexpr int64_t kMaxMeshParts = 4096;
+inline int32_t spmv_parts(const BatchWork& B, int lpr) {
+  const int64_t rounds = ((int64_t)B.tile_groups * lpr + kB - 1) / kB;
+  return (int32_t)std::max<int64_t>(1, std::min(rounds, kMaxMeshParts / std::max(B.mesh_tiles, 1)));
+}
 
 // k_b_spmv's share of the mesh's state (first part of tile b of mesh m, and p.q of the part in thread 0)
 __device__ __forceinline__ void spmv_state(const MeshState& M, int b, int m, double dot, double* sh) {
@@ -498,6 +506,9 @@ mpf_status build_tiles(BatchWork& B, int T, hipStream_t s) {
   }
   tgh.push_back(g);
   mt[B.nmesh] = (int32_t)lo.size();
+  B.tile_groups = B.mesh_tiles = 0;
+  for (size_t t = 0; t + 1 < tgh.size(); ++t) B.tile_groups = std::max(B.tile_groups, tgh[t + 1] - tgh[t]);
+  for (int m = 0; m < B.nmesh; ++m) B.mesh_tiles = std::max(B.mesh_tiles, mt[m + 1] - mt[m]);
   MPF_TRY(B.tg.upload(tgh.data(), tgh.size(), s));
   B.T = T;
   B.ntiles = (int32_t)lo.size();
@@ -505,7 +516,7 @@ mpf_status build_tiles(BatchWork& B, int T, hipStream_t s) {
   MPF_TRY(B.thi.upload(hi.data(), hi.size(), s));
   MPF_TRY(B.tmesh.upload(tm.data(), tm.size(), s));
   MPF_TRY(B.mtile.upload(mt.data(), mt.size(), s));
-  MPF_TRY(B.part.alloc((size_t)std::max(B.ntiles, 1) * (2 + spmv_parts(T, kMaxLPR))));
+  MPF_TRY(B.part.alloc((size_t)std::max(B.ntiles, 1) * (2 + spmv_parts(B, kMaxLPR))));
   MPF_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
   return MPF_OK;
 }
@@ -515,7 +526,7 @@ mpf_status enqueue_cg_iter(mpf_problem* p, BatchWork& B, int32_t maxit) {
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
   const dim3 gt(std::max(B.ntiles, 1)), bt(kB);
-  const int32_t np = spmv_parts(B.T, B.LPR);
+  const int32_t np = spmv_parts(B, B.LPR);
   const dim3 gs(gt.x, np);
   const MeshState M{B.tmesh.ptr, B.mtile.ptr, B.ms.ptr, B.mf.ptr, B.part.ptr, B.part.ptr + 2 * (size_t)B.ntiles, np};
   if (B.grp_spmv) {

@@ -204,6 +204,23 @@ def test_batch_autotune_choice_is_used(mpf, gpu):
     assert np.all(rel < 1e-9)
 
 
+@pytest.mark.parametrize("lanes", [4, 16])
+@pytest.mark.parametrize("tile", [1, 7, 100_000, 1 << 30, (1 << 31) - 1])
+def test_tile_length_far_from_the_meshes(mpf, gpu, tile, lanes):
+    """Tiles of one node's rows, and tiles far longer than every mesh (one per mesh, whatever the length asked for):
+    the same Newton path as with the default tile, up to the rounding of its corrections (the bound of the tests
+    against the oracle)."""
+    u = []
+    for t in (0, tile):
+        _, P = _batch(mpf)
+        _, rel, rep = P.batch_newton_step(1.0, itmax=25, rtol=1e-11, cg_maxit=20000, cg_rtol=1e-13, tile=t,
+                                          lanes_per_row=lanes)
+        assert np.all(rel < 1e-11), rel
+        assert t == 0 or rep.tile == t
+        u.append(P.state()[0])
+    assert normwise_rel(u[1], u[0]) < 1e-9
+
+
 def test_gather_stage_caps_give_the_same_system(mpf, gpu):
     """The element-batch candidates of the autotuner that share the row-owner gather (chunk kernel
     staging 8..32 distinct elements, or direct record reads) assemble bitwise the same K and R."""
