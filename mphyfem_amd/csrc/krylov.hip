@@ -26,7 +26,7 @@ struct KrylovWork {
   int64_t n = 0;
   DevBuf<double> r, z, p, q, w;
   DevBuf<double> r2;          // PCG residual, the other half of the pair (alternates by iteration)
-  DevBuf<double> part;        // partial sums [kMaxParts * 64]
+  DevBuf<double> part;        // partial sums (setup_work says how many)
   DevBuf<double> sc;          // device scalars
   DevBuf<double> V;           // GMRES basis [(m+1) * n]
   int vcap = 0;
@@ -678,8 +678,9 @@ static mpf_status setup_work(mpf_problem* p, int pc, int restart) {
     MPF_TRY(W.sc.alloc(S_N + kMaxRestart + 2));
     W.pc_kind = -1;
   }
-  // partial sums: 2 arrays for CG, (restart + 1) for the GMRES multi-dot, +1 slot for dev_norm2's result
-  const size_t nparts_needed = (size_t)kMaxParts * (size_t)(std::max(2, restart + 1) + 1);
+  // partial sums: CG's arrays, or the GMRES multi-dot's restart + 1 and one more (dev_norm2 takes one array and one
+  // place for its result)
+  const size_t nparts_needed = (size_t)kMaxParts * (size_t)std::max(kCgPartArrays, restart + 2);
   if (W.part.n < nparts_needed) MPF_TRY(W.part.alloc(nparts_needed));
   if (restart > 0 && W.vcap < restart + 1) {
     MPF_TRY(W.V.alloc((size_t)(restart + 1) * n));
@@ -777,7 +778,7 @@ mpf_status pcg_csr(const CsrView& A, const BlockPcView& B, const CgScratch& w, c
   // product 57.7, update 14.2, p 6.9; 4096 and 1342: 59.0, 15.3, 8.0; 1024 and 512: 81.0, 14.6, 5.9.  As five launches with one
   // workgroup's sums between: 91 us an iteration with the launches' gaps, now 79.)
   const unsigned nsp = std::min(spmv_parts(A, B), 2048u), nv = std::min(nps, 1024u);
-  double* pq = w.part + 2 * (size_t)kMaxParts;  // r.z and r.r before it
+  double* pq = w.part + (kCgPartArrays - 1) * (size_t)kMaxParts;  // r.z and r.r before it
   for (;;) {
     for (int c = 0; c < chunk; ++c, ++it) {
       const int par = it & 1;

@@ -259,7 +259,8 @@ struct BlockPcView {
   bool grp = false;               // every block's rows share one column list (row-group SpMV)
 };
 constexpr int kCgScalars = 16;    // device scalars of one CG run
-struct CgScratch {                // n doubles each; part: 3 * kMaxPartials; sc: kCgScalars
+constexpr int kCgPartArrays = 3;  // its arrays of kMaxPartials partial sums: r.z, r.r and p.q
+struct CgScratch {                // n doubles each; part: kCgPartArrays * kMaxPartials; sc: kCgScalars
   double *r, *r2, *z, *p, *q, *part, *sc;
 };
 // Block-preconditioned CG from x = 0 to ||b - A x|| <= rtol ||b|| or maxit iterations.  first: iterations to launch

@@ -821,7 +821,8 @@ mpf_status build_tables(mpf_problem* p, PmgWork& W) {
   MPF_TRY(W.kabinv.alloc(9 * (size_t)(W.nab > 0 ? W.nab : 1)));
   for (DevBuf<double>* b : {&W.cxa, &W.cxb, &W.cdd, &W.cres}) MPF_TRY(b->alloc(nc));
   for (DevBuf<double>* b : {&W.ra, &W.xa3}) MPF_TRY(b->alloc(W.na > 0 ? W.na : 1));
-  MPF_TRY(W.cpart.alloc(3 * (size_t)kMaxPartials));  // coarse CG: 2 per workgroup; power steps: 3
+  static_assert(kCgPartArrays >= 3, "the power steps' three sums");
+  MPF_TRY(W.cpart.alloc(kCgPartArrays * (size_t)kMaxPartials));  // coarse CG, power steps
   MPF_TRY(W.csc.alloc(kCgScalars));
   MPF_TRY(W.bad.alloc(1));
   CsrView C;
