@@ -642,10 +642,12 @@ constexpr int kTetEPW = MPF_TET_EPW;
 
 // Workgroups of the dense kernels: epw elements' Gauss points each and then one element's matrix after the other; where
 // that leaves compute units idle, epw workgroups share the elements' matrices, each with all the Gauss points of
-// its own (125 Hex8: 18.0 -> 8.1 us).  Up to 256 blocks, one a compute unit: from there on the shared work would wait.
+// its own.  Up to 1024 workgroups, the four that a compute unit holds at a time: further ones would wait with the shared
+// work before them.  Whole calls, apart -> sharing: Hex8 125 elements 41 -> 32 us, 800 41 -> 36, 1024 41 -> 36, but 1100 41 ->
+// 43 and 2048 43 -> 49; Tet10/P1 60 elements 47 -> 42, 1024 49 -> 46.
 static dim3 dense_grid(int32_t count, int epw) {
   const unsigned nb = (unsigned)grid_for(count, epw);
-  return dim3(nb, nb <= 256 ? epw : 1);
+  return dim3(nb, nb * epw <= 1024 ? epw : 1);
 }
 
 mpf_status launch_hex8_dense(const ElemArgs& a, int32_t first, int32_t count, double* Ke, double* Re,

@@ -63,21 +63,20 @@ def test_hex8_batch_vs_oracle(mpf, orc, gpu, tangent):
     assert np.array_equal(Ke2.cpu().numpy(), Ke[13:18])
 
 
-@pytest.mark.parametrize("etype", ["hex8", "tet10p1"])
+@pytest.mark.parametrize("etype", ["hex8", "tet10", "tet10p1"])
 @pytest.mark.parametrize("extra", [-1, 0, 1])
 def test_dense_elements_across_the_shared_block_limit(mpf, gpu, etype, extra):
-    """Calls of 256 blocks of elements, one fewer and one more (up to 256 blocks, several workgroups share a
-    block's matrices): the same bits as each element called in the middle of a small call."""
+    """Calls of 1024 elements, one fewer and one more (up to 1024 workgroups, several share a block's matrices: 8 elements
+    of Hex8, 4 of Tet10): the same bits as each element called in the middle of a small call."""
     import torch
-    hexa = etype == "hex8"
-    n = 256 * (8 if hexa else 4) + extra
-    X, conn = mpf.mesh_hex(13, 13, 13, jitter=0.05, seed=3) if hexa else mpf.mesh_tet10(6, jitter=0.05, seed=3)
+    n = 1024 + extra
+    X, conn = mpf.mesh_hex(11, 11, 11, jitter=0.05, seed=3) if etype == "hex8" else mpf.mesh_tet10(6, jitter=0.05, seed=3)
     conn = conn[:n]
     assert len(conn) == n
     u = 0.01 * np.sin(7.0 * X).ravel()
     m = mpf.matl_from_E_nu(1e3, 0.3)
-    args = [_t(gpu, X), _t(gpu, u)] + ([] if hexa else [_t(gpu, 0.5 * u), _t(gpu, np.cos(3.0 * X[:, 0]))])
-    call = mpf.elem_hex8_nh_batch if hexa else mpf.elem_tet10p1_nh_batch
+    args = [_t(gpu, X), _t(gpu, u)] + ([_t(gpu, 0.5 * u), _t(gpu, np.cos(3.0 * X[:, 0]))] if etype == "tet10p1" else [])
+    call = {"hex8": mpf.elem_hex8_nh_batch, "tet10": mpf.elem_tet10_nh_batch, "tet10p1": mpf.elem_tet10p1_nh_batch}[etype]
     out = call(*args, _t(gpu, conn, torch.int32), m)
     for first in (0, n // 2, n - 9):
         part = call(*args, _t(gpu, conn, torch.int32), m, first=first, count=9)
