@@ -109,13 +109,14 @@ def test_tangent_increment_solves_the_tangent_system(mpf, gpu):
     assert torch.equal(d, d2)
 
 
-@pytest.mark.parametrize("n", [4, 7])
-def test_batched_band_many_meshes_match_one(mpf, gpu, n):
-    """130 copies of one mesh, enough that each is factored by one workgroup per segment (half-bandwidth 77: panels looking
-    ahead; 194: a thread per panel row), against the mesh alone, factored by panels over several workgroups: the
-    Newton path is the same up to the rounding of its corrections (the bound of the tests against the oracle)."""
+@pytest.mark.parametrize("n,many", [(4, 130), (7, 130), (8, 321)])
+def test_batched_band_many_meshes_match_one(mpf, gpu, n, many):
+    """Copies of one mesh, enough that each is factored by one workgroup per segment (half-bandwidth 77: panels looking
+    ahead; 194 and, cut in two, 275: a thread per panel row), against the mesh alone, factored by panels over several
+    workgroups: the Newton path is the same up to the rounding of its corrections (the bound of the tests against the
+    oracle)."""
     u = {}
-    for copies in (1, 130):
+    for copies in (1, many):
         one = np.ones(copies)
         _, P = mpf.batch_problem([n] * copies, 1e3 * one, 0.3 * one, -30.0 * one, 10.0 * one)
         P.prepare_matrix_pattern()
@@ -124,8 +125,8 @@ def test_batched_band_many_meshes_match_one(mpf, gpu, n):
         assert P.band_segments()[0] >= copies
         u[copies] = P.state()[0].reshape(copies, -1)
         print(n, copies, P.band_stats()[1], P.band_segments(), iters[0], flush=True)
-    assert np.array_equal(u[130], np.tile(u[130][0], (130, 1)))
-    assert normwise_rel(u[130][0], u[1][0]) < 1e-9
+    assert np.array_equal(u[many], np.tile(u[many][0], (many, 1)))
+    assert normwise_rel(u[many][0], u[1][0]) < 1e-9
 
 
 def test_batched_band_cut_blocks_match_whole_blocks(mpf, gpu):
