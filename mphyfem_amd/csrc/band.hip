@@ -949,6 +949,26 @@ __global__ void k_band_rhs(int32_t ncols, const int32_t* __restrict__ cseg, cons
 
 }  // namespace
 
+// Factorisation by panels over several workgroups per segment, or by one workgroup per segment?  A segment's panel takes a
+// workgroup per 64 rows of the band (two fit on a compute unit), so what counts is how often they fill the GPU's 256
+// compute units.  Whole direct solves, one workgroup per segment -> panels:
+//   64 x 4 x 8 beams (b 167, three a segment): 80 segments 5.75 -> 4.84 ms, 128 segments 5.93 -> 7.03 ms
+//   64 x 3 x 5 beams (b 95, two): 80 segments 2.65 -> 2.20 ms, 200 segments 2.81 -> 3.34 ms
+//   64 x 2 x 2 beams (b 41, one): 80 segments 0.94 -> 0.82 ms, 400 segments 1.82 -> 1.58 ms; 32 x 2 x 2: 4000 segments 7.87 -> 6.40
+//   32 x 5 x 8 beams (b 194, four): 80 segments 6.67 -> 4.19 ms, 200 segments 7.15 -> 7.50 ms
+//   8 to 16 x 8 x 8 blocks (b 275, five): 100 segments 6.07 -> 2.96 ms, 600 segments 14.0 -> 13.8, 800 17.9 -> 18.8, 3000 41.3 -> 49.8
+//   9 to 11 x 9 x 9 blocks (b 335, six): 600 segments 18.3 -> 17.3 ms, 1200 32.6 -> 35.2
+//   10 to 12 x 10 x 10 blocks (b 401, seven): 400 segments 23.6 -> 19.6 ms, 1000 52.0 -> 50.8, 2000 101.6 -> 102.8
+//   11 to 13 x 11 x 11 blocks (b 473, eight): 200 segments 25.4 -> 15.6 ms, 1400 143 -> 119
+// so: bands up to 64 and above 383 always; up to 176 (where one workgroup per segment looks ahead) if one round of one
+// workgroup a compute unit holds them; up to 255 if two do; up to 383 for up to 640 segments.
+static bool band_panels(int32_t nseg, int32_t bmax) {
+  if (bmax <= kStrip || bmax > 383) return true;
+  if (bmax > 255) return nseg <= 640;
+  const int64_t rounds = ((int64_t)nseg * ((bmax + kStrip - 1) / kStrip) + 255) / 256;
+  return rounds <= (bmax + kW <= 3 * 64 ? 1 : 2);
+}
+
 struct BandWork {
   uint64_t key = 0;       // problem uid, block layout and cut setting it was built for
   int32_t nblk = 0, n = 0, bmax = 0;
@@ -959,7 +979,7 @@ struct BandWork {
   DevBuf<int32_t> perm, iperm, cseg;
   DevBuf<BandSeg> seg;
   DevBuf<double> band, y;
-  DevBuf<double> diag;    // per segment: the factored diagonal block of the panel being eliminated
+  DevBuf<double> diag;    // with panels, per segment: the factored diagonal block of the panel being eliminated
   DevBuf<int32_t> bad;
   DevBuf<int32_t> bok;    // per block: 1 once the band holds its factors
   bool factored = false;  // a factorisation has been enqueued since the layout was built
@@ -1184,36 +1204,18 @@ mpf_status band_prepare(mpf_problem* p, const std::vector<int32_t>& node_off) {
   MPF_TRY(W.band.alloc((size_t)W.nband + (size_t)kP * (W.bmax + 1)));
   MPF_TRY(W.y.alloc(ncols > 0 ? (size_t)ncols : 1));
   MPF_TRY(W.bad.alloc(1));
-  MPF_TRY(W.diag.alloc(std::max<size_t>(sorted.size(), 1) * kP * kP));
+  if (band_panels(W.nseg, W.bmax)) {
+    MPF_TRY(W.diag.alloc(std::max<size_t>(sorted.size(), 1) * kP * kP));
+    MPF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_band_panel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)kPanelLds));
+  }
   {
     const std::vector<int32_t> zero(std::max(nblk, 1), 0);
     MPF_TRY(W.bok.upload(zero.data(), zero.size(), s));
   }
-  MPF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_band_panel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kPanelLds));
   MPF_HIP(hipStreamSynchronize(s));
   W.key = key;
   return MPF_OK;
-}
-
-// Factorisation by panels over several workgroups per segment, or by one workgroup per segment?  A segment's panel takes a
-// workgroup per 64 rows of the band (two fit on a compute unit), so what counts is how often they fill the GPU's 256
-// compute units.  Whole direct solves, one workgroup per segment -> panels:
-//   64 x 4 x 8 beams (b 167, three a segment): 80 segments 5.75 -> 4.84 ms, 128 segments 5.93 -> 7.03 ms
-//   64 x 3 x 5 beams (b 95, two): 80 segments 2.65 -> 2.20 ms, 200 segments 2.81 -> 3.34 ms
-//   64 x 2 x 2 beams (b 41, one): 80 segments 0.94 -> 0.82 ms, 400 segments 1.82 -> 1.58 ms; 32 x 2 x 2: 4000 segments 7.87 -> 6.40
-//   32 x 5 x 8 beams (b 194, four): 80 segments 6.67 -> 4.19 ms, 200 segments 7.15 -> 7.50 ms
-//   8 to 16 x 8 x 8 blocks (b 275, five): 100 segments 6.07 -> 2.96 ms, 600 segments 14.0 -> 13.8, 800 17.9 -> 18.8, 3000 41.3 -> 49.8
-//   9 to 11 x 9 x 9 blocks (b 335, six): 600 segments 18.3 -> 17.3 ms, 1200 32.6 -> 35.2
-//   10 to 12 x 10 x 10 blocks (b 401, seven): 400 segments 23.6 -> 19.6 ms, 1000 52.0 -> 50.8, 2000 101.6 -> 102.8
-//   11 to 13 x 11 x 11 blocks (b 473, eight): 200 segments 25.4 -> 15.6 ms, 1400 143 -> 119
-// so: bands up to 64 and above 383 always; up to 176 (where one workgroup per segment looks ahead) if one round of one
-// workgroup a compute unit holds them; up to 255 if two do; up to 383 for up to 640 segments.
-static bool band_panels(int32_t nseg, int32_t bmax) {
-  if (bmax <= kStrip || bmax > 383) return true;
-  if (bmax > 255) return nseg <= 640;
-  const int64_t rounds = ((int64_t)nseg * ((bmax + kStrip - 1) / kStrip) + 255) / 256;
-  return rounds <= (bmax + kW <= 3 * 64 ? 1 : 2);
 }
 
 // Solve phases of every segment with the factors in the band (active as for the factorisation).
