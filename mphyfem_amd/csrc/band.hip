@@ -18,10 +18,10 @@
 // the GPU's compute units than one workgroup per block.  Shorter blocks are one segment.
 //
 //   k_band_panel / k_band_trail: right-looking in panels of kP columns on several workgroups per
-//   segment, one launch pair per panel (few segments, or wide bands: band_panels);
+//   segment, one launch pair per panel (few segments, or narrow or wide bands: band_panels);
 //   k_band_factor: right-looking in panels of kW columns by one workgroup per segment -- the panel
-//   factored column by column (bands up to 176 wide: by one wavefront in registers, three rows per
-//   lane; wider: one thread per panel row and one barrier per column), the rank-kW update of the
+//   factored column by column (bands of 65 to 176: by one wavefront in registers, three rows per
+//   lane; of 177 to 383: one thread per panel row and one barrier per column), the rank-kW update of the
 //   b x b trailing triangle on the matrix cores (FP64 MFMA);
 //   k_band_solve: forward and backward substitution in blocks of kW rows, the unit triangle in one
 //   wavefront's registers, the coupling to the next b rows by the whole workgroup.
@@ -46,6 +46,12 @@ constexpr int kFBS = 768;   // threads per workgroup of the factorisation: 12 wa
 #ifndef MPF_BAND_TILES
 #define MPF_BAND_TILES 2
 #endif
+// Widest half-bandwidth accepted: the substitution's ring and the band fill's columns in LDS and a lane's entries of a
+// row in the backward sums are sized for it.
+constexpr int kMaxBand = 493;
+// Widest that one workgroup per segment factors (band_panels).
+constexpr int kMaxFactorBand = 383;
+static_assert(kW + kMaxFactorBand <= kFBS, "each row of a wide panel has a thread");
 constexpr int kNH = MPF_BAND_TILES;  // trailing-update tiles per wavefront and round (old values loaded first)
 static_assert(kBS / 64 == kW, "one wavefront per panel row in the backward solve");
 
@@ -630,7 +636,7 @@ __global__ void __launch_bounds__(256) k_band_trail(BandArgs A, int32_t phase, i
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
   double* L = A.band + S.boff + (size_t)j0 * B1;
   const double* D = A.diag + (size_t)blockIdx.x * kP * kP;
-  if (blockIdx.y == 0)  // the diagonal block's factors into the band (no entry of it is read here)
+  if (blockIdx.y == 0)  // the diagonal block's factors into the band (what is read of it here, past the band, is replaced)
     for (int c = wid; c < w; c += 4)
       if (lane >= c && lane < w && lane - c <= b) L[(size_t)c * B1 + (lane - c)] = D[c * kP + lane];
   const int R0 = w + kTile * t + 16 * (wid >> 1);
@@ -703,7 +709,8 @@ __device__ __forceinline__ void fwd_entries(const double* L, int B1, int b, int 
 // (backward) the current block -- are kept in an LDS ring, row r at ring[r % kRing], so that a
 // block step reads and updates them without a round trip through global memory.
 constexpr int kRing = 1024;
-static_assert(kRing >= 2 * (493 + kW), "the ring holds the window and the rows loaded ahead of it");
+static_assert(kRing >= 2 * (kMaxBand + kW), "the ring holds the window and the rows loaded ahead of it");
+static_assert(kMaxBand < kBS / 2, "each half of the workgroup gives a coupling row one thread");
 
 // forward substitution over columns [c0, c1) and the division by the pivots.  The two halves of
 // the workgroup take the block steps in turn (b < kBS / 2 coupling rows each), and each half loads
@@ -784,7 +791,7 @@ __device__ __forceinline__ void band_forward(const double* L, double* y, double*
 }
 
 constexpr int kBRow = 8;  // band entries per lane of a backward row sum: b < 64 kBRow
-static_assert(64 * kBRow > 493, "the widest band the panel LDS allows");
+static_assert(64 * kBRow > kMaxBand, "a lane holds its share of the widest row");
 
 // backward row k's entries L(r, k), r = j0 + w + lane + 64 t <= min(n - 1, k + b), k = j0 + wid,
 // and its right-hand side
@@ -963,7 +970,7 @@ __global__ void k_band_rhs(int32_t ncols, const int32_t* __restrict__ cseg, cons
 // so: bands up to 64 and above 383 always; up to 176 (where one workgroup per segment looks ahead) if one round of one
 // workgroup a compute unit holds them; up to 255 if two do; up to 383 for up to 640 segments.
 static bool band_panels(int32_t nseg, int32_t bmax) {
-  if (bmax <= kStrip || bmax > 383) return true;
+  if (bmax <= kStrip || bmax > kMaxFactorBand) return true;
   if (bmax > 255) return nseg <= 640;
   const int64_t rounds = ((int64_t)nseg * ((bmax + kStrip - 1) / kStrip) + 255) / 256;
   return rounds <= (bmax + kW <= 3 * 64 ? 1 : 2);
@@ -1192,10 +1199,7 @@ mpf_status band_prepare(mpf_problem* p, const std::vector<int32_t>& node_off) {
   W.nband = nband;
   W.bw_h = bw;
   W.bstart_h = bstart;
-  const int lds = (int)(((size_t)(kW + W.bmax) * kW + 3 * kW) * sizeof(double));
-  if (lds > 64 * 1024) return MPF_ERR_ARG;  // half-bandwidth beyond the panel's LDS (about 490 dofs)
-  if (W.bmax >= kBS / 2) return MPF_ERR_ARG;  // each half of the solve's workgroup gives a coupling row one thread
-  static_assert(kW + 493 <= kFBS, "the wide-band panel path gives each panel row one thread");
+  if (W.bmax > kMaxBand) return MPF_ERR_ARG;
   MPF_TRY(W.perm.upload(perm.data(), perm.size(), s));
   MPF_TRY(W.iperm.upload(iperm.data(), iperm.size(), s));
   MPF_TRY(W.cseg.upload(cseg.data(), cseg.size(), s));
@@ -1240,7 +1244,7 @@ mpf_status band_enqueue_solve(mpf_problem* p, const int32_t* active, int32_t ast
   hipStream_t s = p->stream;
   const PatternBufs& P = p->pat;
   const BandArgs A{W->seg.ptr, W->band.ptr, W->y.ptr, W->bad.ptr, W->diag.ptr};
-  static_assert(kFillCols * 494 * sizeof(double) <= 64 * 1024, "the fill's LDS holds columns of b <= 493");
+  static_assert(kFillCols * (kMaxBand + 1) * sizeof(double) <= 64 * 1024, "the fill's LDS holds the widest columns");
   hipLaunchKernelGGL(k_band_fill, dim3(std::max((W->ncols + kFillCols - 1) / kFillCols, 1)), dim3(256),
                      (size_t)kFillCols * (W->bmax + 1) * sizeof(double), s, W->ncols, W->bmax + 1, W->cseg.ptr,
                      P.rowptr.ptr, P.colidx.ptr, p->vals.ptr, p->rhs.ptr, W->perm.ptr, W->iperm.ptr, A, active,
