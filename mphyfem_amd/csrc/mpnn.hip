@@ -505,12 +505,14 @@ __global__ void k_err_free(int64_t n, const int32_t* __restrict__ nmesh_of, cons
   }
 }
 
-// per mesh: sum of r^2 over its free-dof range
+// per mesh: sum of r^2 over its free-dof range.  One workgroup a mesh, bound by its loads' latency: eight of a thread's in
+// flight, added in the same order (one mesh of 6.3e6 dofs, just assembled: 8.6 -> 2.6 ms, k_mesh_dot 10.1 -> 2.0).
 __global__ void __launch_bounds__(256) k_mesh_sq(const int32_t* __restrict__ doff, const double* __restrict__ r,
                                                  double* __restrict__ out) {
   __shared__ double sh[256];
   const int m = blockIdx.x;
   double v = 0.0;
+#pragma unroll 8
   for (int64_t i = doff[m] + threadIdx.x; i < doff[m + 1]; i += 256) v += r[i] * r[i];
   sh[threadIdx.x] = v;
   __syncthreads();
@@ -527,6 +529,7 @@ __global__ void __launch_bounds__(256) k_mesh_dot(const int32_t* __restrict__ do
   __shared__ double sh[256];
   const int m = blockIdx.x;
   double v = 0.0;
+#pragma unroll 8
   for (int64_t i = doff[m] + threadIdx.x; i < doff[m + 1]; i += 256) v += a[i] * b[i];
   sh[threadIdx.x] = v;
   __syncthreads();
