@@ -869,6 +869,37 @@ def test_gather_workgroup_remainders_vs_oracle(mpf, orc, gpu, etype, dims, first
     assert normwise_rel(vals, ov) < TOL_K and normwise_rel(rhs, orhs) < TOL_K
 
 
+@pytest.mark.parametrize("k", [3, 11, 20])
+def test_gather_long_runs_vs_oracle(mpf, orc, gpu, k):
+    """Two layers of k hexahedra around an axis: the middle axis node lies in 2 k elements (40 of at most 64) and couples
+    to 6 k + 3 nodes (123 of at most 128), so that its columns' runs are long and uneven and its items take several
+    wavefronts, shared with its neighbours' where they fit.  K and R against the oracle, as above."""
+    ang = np.pi / k * np.arange(2 * k)
+    ring = np.stack([np.cos(ang), np.sin(ang)], 1) * np.where(np.arange(2 * k) % 2, 1.1, 1.0)[:, None]
+    layer = np.vstack([[[0.0, 0.0]], ring])
+    X = np.vstack([np.column_stack([layer, np.full(len(layer), z)]) for z in (0.0, 0.9, 2.1)])
+    q = np.array([[0, 1 + 2 * i, 2 + 2 * i, 1 + (2 * i + 2) % (2 * k)] for i in range(k)])
+    nl = len(layer)
+    conn = np.vstack([np.hstack([q + z * nl, q + (z + 1) * nl]) for z in (0, 1)]).astype(np.int32)
+    m = mpf.matl_from_E_nu(1e3, 0.3, tangent=1)
+    P = mpf.Problem(mpf.HEX8, X, conn, m)
+    O = orc.Problem(8, X, conn, m.mu, m.Kinv, m.Utype)
+    O.set_tangent(True)
+    u = np.random.default_rng(7).uniform(-0.005, 0.005, 3 * len(X))
+    for Q in (P, O):
+        apply_bcs(Q, [(np.arange(1, nl, 2), -1, None), (np.arange(2 * nl + 1, 3 * nl, 3), 2, -0.02)])
+        Q.prepare_matrix_pattern()
+        Q.set_state(disp=u, disp_prev=u)
+        Q.set_boundary_conditions(1.0)
+    assert P.assembly_mode() == mpf.ASSEMBLY_GATHER
+    for first in (True, False):
+        P.calc_stiffness_and_residual(first, 1.0)
+        vals, rhs = P.system()
+        ov, orhs, st = O.assemble(first, 1.0)
+        assert st == 0
+        assert normwise_rel(vals, ov) < TOL_K and normwise_rel(rhs, orhs) < TOL_K
+
+
 def test_gather_node_in_no_element(mpf, orc, gpu):
     """A free node that no element holds: empty rows, a right-hand side of zero at every assembly (not what the last
     solve or assembly left there), the other rows as without it."""
