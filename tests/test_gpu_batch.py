@@ -222,21 +222,24 @@ def test_tile_length_far_from_the_meshes(mpf, gpu, tile, lanes):
     assert normwise_rel(u[1], u[0]) < 1e-9
 
 
-def test_gather_stage_caps_give_the_same_system(mpf, gpu):
-    """The element-batch candidates of the autotuner that share the row-owner gather (chunk kernel
-    staging 8..32 distinct elements, or direct record reads) assemble bitwise the same K and R."""
+def test_switches_without_effect_are_accepted(mpf, gpu):
+    """ASSEMBLY_GATHER_DIRECT and the staged-element cap are kept for callers that set them: accepted in their old
+    ranges, reported back, and K and R bitwise those of ASSEMBLY_GATHER, whose kernels they run."""
     _, P = _batch(mpf)
     P.set_boundary_conditions(1.0)
     ref = None
-    for mode, cap in ((mpf.ASSEMBLY_GATHER, 32), (mpf.ASSEMBLY_GATHER, 8), (mpf.ASSEMBLY_GATHER, 16),
-                      (mpf.ASSEMBLY_GATHER_DIRECT, 32)):
+    for mode, cap in ((mpf.ASSEMBLY_GATHER, 32), (mpf.ASSEMBLY_GATHER_DIRECT, 0)):
         P.set_assembly_mode(mode)
         P.set_chunk_stage_cap(cap)
+        assert P.assembly_mode() == mode
         P.calc_stiffness_and_residual(True, 1.0)
         vals, rhs = P.system()
         if ref is None:
             ref = (vals.copy(), rhs.copy())
         assert np.array_equal(vals, ref[0]) and np.array_equal(rhs, ref[1]), (mode, cap)
+    for cap in (-1, 33):
+        with pytest.raises(mpf.MpfError):
+            P.set_chunk_stage_cap(cap)
 
 
 def test_batched_q1p0_matches_each_mesh_alone(mpf, gpu):

@@ -113,14 +113,19 @@ def test_guess_without_network_is_linear_extrapolation(mpf, gpu):
     assert torch.allclose(out, ref, rtol=1e-15, atol=1e-15)
 
 
-@pytest.mark.parametrize("edges", [[1], [5, 7], [20]])
+@pytest.mark.parametrize("edges", [[1], [5, 7], [20], [52]])
 def test_mpnn_backward_row_remainders_vs_oracle(mpf, gpu, edges):
-    """Layer gradients over 8, 728 and 9 261 rows: fewer rows than one 32-row chunk, several 256-row
-    workgroups, and last chunks of 8, 24 and 13 rows.  Tolerance: a value that FP32 and FP64 sums put on
-    different sides of a BF16 rounding boundary moves one row's product by 2^-8 of itself, and the sum of
-    n random rows is sqrt(n) rows long; eight such rows adding up are 8 / 256 / sqrt(9261) = 3.2e-4
-    (measured 1e-4 there, 1e-6 and less at the smaller sizes).  Leaving out the last row (planted in the
-    oracle) moves a gradient by about 1 / sqrt(n) >= 1e-2 of its length."""
+    """Layer gradients over 8, 728, 9 261 and 148 877 rows: fewer rows than one 32-row chunk, several 256-row
+    workgroups, workgroups of more (320 of the 148 877), and last chunks of 8, 24, 13 and 13 rows.  Tolerance: a
+    value that FP32 and FP64 sums put on different sides of a BF16 rounding boundary moves one row's product by
+    2^-8 of itself, and the sum of n random rows is sqrt(n) rows long; eight such rows adding up are
+    8 / 256 / sqrt(9261) = 3.2e-4 (measured 1e-4 there, 1e-6 and less at the smaller sizes).  Leaving
+    out the last row (planted in the oracle) moves a gradient by about 1 / sqrt(n) >= 1e-2 of its length; of the
+    148 877 rows, the last chunk's 13 are left out, about sqrt(13 / n) = 9e-3.
+    With 148 877 rows some of the 4e7 ReLU inputs lie within FP32 rounding of zero (7 change sign between an FP32 and
+    the FP64 forward pass of the oracle) and each moves one row's whole product in every layer before it: eight of
+    them adding up are 8 / sqrt(n) = 2.1e-2 of a gradient there, except the output layer's, which no ReLU follows.
+    A workgroup that left out one of its ten chunks would move it by sqrt(0.1) = 0.3."""
     import torch
     tol = 3.2e-4
     B = mpf.mesh_batch_hex(edges)
@@ -144,7 +149,7 @@ def test_mpnn_backward_row_remainders_vs_oracle(mpf, gpu, edges):
     R = O.unpack(O.backward(w.astype(np.float64), cache, dy.astype(np.float64), ptr, nb, bf16_ops=True))
     for k in R:
         print(f"[mpnn] {n} rows, grad {k}: {_rel(G[k], R[k]):.2e}", flush=True)
-        assert _rel(G[k], R[k]) < tol, k
-    dy[-1] = 0.0
+        assert _rel(G[k], R[k]) < (tol if n < 10_000 or k in ("Wo", "bo") else 8 / np.sqrt(n)), k
+    dy[-1 if n < 10_000 else -13:] = 0.0
     bad = O.unpack(O.backward(w.astype(np.float64), cache, dy.astype(np.float64), ptr, nb, bf16_ops=True))
     assert _rel(G["bo"], bad["bo"]) > 4 * tol and _rel(G["Wo"], bad["Wo"]) > 4 * tol

@@ -316,7 +316,7 @@ def test_pattern_and_colouring_bitexact_tet(mpf, orc, gpu):
     assert pat.ncolors == ncol and np.array_equal(pat.color, col)
 
 
-@pytest.mark.parametrize("mode", [0, 1, 2], ids=["gather", "colored_scatter", "gather_direct"])
+@pytest.mark.parametrize("mode", [0, 1], ids=["gather", "colored_scatter"])
 @pytest.mark.parametrize("tangent,traction", [(0, None), (1, (-20.0, 5.0))])
 def test_global_assembly_hex_vs_oracle(mpf, orc, gpu, tangent, traction, mode):
     n = 10
@@ -338,7 +338,7 @@ def test_global_assembly_hex_vs_oracle(mpf, orc, gpu, tangent, traction, mode):
         assert abs(P.rhs_norm() - np.linalg.norm(orhs)) < 1e-12 * np.linalg.norm(orhs)
 
 
-@pytest.mark.parametrize("mode", [0, 1, 2], ids=["gather", "colored_scatter", "gather_direct"])
+@pytest.mark.parametrize("mode", [0, 1], ids=["gather", "colored_scatter"])
 def test_global_assembly_tet_vs_oracle(mpf, orc, gpu, mode):
     n = 4
     X, conn = mpf.mesh_tet10(n, jitter=0.1, seed=2)
@@ -363,12 +363,10 @@ def test_global_assembly_tet_vs_oracle(mpf, orc, gpu, mode):
     assert P.assembly_mode() == mode
 
 
-@pytest.mark.parametrize("mode,cap", [(0, 32), (0, 12), (2, 32), (1, 32)],
-                         ids=["gather", "gather_partly_staged", "gather_direct", "colored_scatter"])
-def test_global_assembly_hex8p0_vs_oracle(mpf, orc, gpu, mode, cap):
+@pytest.mark.parametrize("mode", [0, 1], ids=["gather", "colored_scatter"])
+def test_global_assembly_hex8p0_vs_oracle(mpf, orc, gpu, mode):
     """Hex8 Q1/P0 condensed system (Kc = Kuu - Kup Kpu / Kpp, Fc = Fu - Kup Fp / Kpp) through the
-    row-owner gather (chunk kernel staging the condensed records in LDS, some chunks reading them
-    directly, or every chunk reading directly) and through the coloured scatter: global K and R
+    row-owner gather (condensed element records) and through the coloured scatter: global K and R
     against the oracle's condensed assembly, with the first-iteration lift and without; the gather
     bitwise repeatable."""
     nx, ny, nz = 7, 5, 6
@@ -385,7 +383,6 @@ def test_global_assembly_hex8p0_vs_oracle(mpf, orc, gpu, mode, cap):
         Q.set_state(disp=u, disp_prev=0.5 * u, pres=pe, pres_prev=pe)
         Q.set_boundary_conditions(0.8)
     P.set_assembly_mode(mode)
-    P.set_chunk_stage_cap(cap)
     for first in (True, False):
         P.calc_stiffness_and_residual(first, 0.8)
         vals, rhs = P.system()
@@ -395,16 +392,14 @@ def test_global_assembly_hex8p0_vs_oracle(mpf, orc, gpu, mode, cap):
             assert np.array_equal(vals, v2) and np.array_equal(rhs, r2)
         ov, orhs, st = O.assemble(first, 0.8)
         assert st == 0
-        print("Q1/P0 mode", mode, "cap", cap, "first", first, normwise_rel(vals, ov), normwise_rel(rhs, orhs),
+        print("Q1/P0 mode", mode, "first", first, normwise_rel(vals, ov), normwise_rel(rhs, orhs),
               flush=True)
         assert normwise_rel(vals, ov) < TOL_K
         assert normwise_rel(rhs, orhs) < TOL_K
 
 
-@pytest.mark.parametrize("cap", [32, 20, 0], ids=["staged", "mixed", "direct_reads"])
-def test_hex_chunk_staging_vs_oracle(mpf, orc, gpu, cap):
-    """Hex8 chunked matrix kernel on a jittered box that is not a cube: chunks staged in LDS (cap 32),
-    some staged and some reading the records directly (cap 20), every chunk reading directly (0)."""
+def test_hex_box_assembly_vs_oracle(mpf, orc, gpu):
+    """Hex8 gather on a jittered box that is not a cube: K and R against the oracle, bitwise repeatable."""
     nx, ny, nz = 9, 6, 11
     X, conn = mpf.mesh_hex(nx, ny, nz, L=(1.0, 0.7, 1.6), jitter=0.1, seed=4)
     m = mpf.matl_from_E_nu(1e3, 0.3, tangent=1)
@@ -418,7 +413,6 @@ def test_hex_chunk_staging_vs_oracle(mpf, orc, gpu, cap):
         Q.prepare_matrix_pattern()
         Q.set_state(disp=u, disp_prev=u)
         Q.set_boundary_conditions(0.6)
-    P.set_chunk_stage_cap(cap)
     for first in (True, False):
         P.calc_stiffness_and_residual(first, 0.6)
         vals, rhs = P.system()
@@ -429,8 +423,6 @@ def test_hex_chunk_staging_vs_oracle(mpf, orc, gpu, cap):
         assert st == 0
         assert normwise_rel(vals, ov) < TOL_K
         assert normwise_rel(rhs, orhs) < TOL_K
-    with pytest.raises(mpf.MpfError):
-        P.set_chunk_stage_cap(33)
 
 
 def test_high_valence_node_falls_back_to_scatter(mpf, orc, gpu):
@@ -462,7 +454,7 @@ def test_high_valence_node_falls_back_to_scatter(mpf, orc, gpu):
 
 @pytest.mark.parametrize("etype", ["hex8", "tet10p1"])
 def test_gather_matrix_exactly_symmetric(mpf, gpu, etype):
-    """The gather sums each pair of column blocks once and writes it to both places, so the
+    """The column blocks (n, m) and (m, n) sum the same element blocks in the same order, so the
     assembled matrix (u-u, u-p, p-u and p-p blocks alike) equals its transpose bit for bit."""
     import scipy.sparse as sp
 
@@ -785,7 +777,7 @@ def test_pattern_and_colouring_bitexact_tet10(mpf, orc, gpu):
     assert pat.ncolors == ncol and np.array_equal(pat.color, col)
 
 
-@pytest.mark.parametrize("mode", [0, 1, 2], ids=["gather", "colored_scatter", "gather_direct"])
+@pytest.mark.parametrize("mode", [0, 1], ids=["gather", "colored_scatter"])
 @pytest.mark.parametrize("tangent", [0, 1])
 def test_global_assembly_tet10_vs_oracle(mpf, orc, gpu, tangent, mode):
     X, conn, P, O = _tet10_problems(mpf, orc, 4, tangent, mode)
