@@ -126,8 +126,8 @@ typedef struct mpf_problem mpf_problem;
 
 /* Creates a problem from host arrays (copied to the device).  elem_type MPF_HEX8, MPF_HEX8P0,      */
 /* MPF_TET10P1 or MPF_TET10.  MPF_HEX8P0 assembles the statically condensed system (displacement    */
-/* rows only; the gather's staging records carry each element's Kup and Kpp, so every block adds    */
-/* -Kup_a Kup_b^T / Kpp, and its residual is condensed) in any assembly mode, recovers the element  */
+/* rows only; every element's blocks take -Kup_a Kup_b^T / Kpp and its residual is condensed        */
+/* before either goes into the system) in any assembly mode, recovers the element                   */
 /* pressures in mpf_update (solveForPressure, Elem_Solid_3D_Mixed0.cpp:112-199), and batches like   */
 /* MPF_HEX8.                                                                                         */
 mpf_status mpf_problem_create(mpf_problem** out, int32_t elem_type, int32_t nNode, int32_t nElem,
@@ -347,7 +347,7 @@ typedef struct {
   double cg_rtol;         /* lower bound of the inexact-Newton CG tolerance (Eisenstat-Walker forcing) */
   int32_t use_graph;      /* 1: replay captured HIP graphs; 0: launch the same kernels directly */
   int32_t chunk;          /* CG iterations per graph launch (0: keep) */
-  int32_t tile;           /* dofs per tile (0: keep the autotuned / default value) */
+  int32_t tile;           /* dofs per tile (0: keep the autotuned / default value; longer than a mesh: one tile) */
   int32_t lanes_per_row;  /* SpMV lanes per row, 4, 8 or 16 (0: keep) */
   int32_t solver;         /* 0: Jacobi-PCG per mesh; 1: banded LDL^T direct solve per mesh (MPF_KSP_BAND, */
                           /*    a workgroup per mesh, or per half of a long mesh cut at a separator;    */
@@ -375,7 +375,8 @@ typedef struct {
 /* every (tile, lanes_per_row) candidate over a few CG iterations; the fastest are kept for         */
 /* mpf_batch_newton_solve.                                                                          */
 mpf_status mpf_batch_autotune(mpf_problem* p, int32_t* tile, int32_t* lanes_per_row, double* ms_per_cg_iter);
-/* The autotuner's assembly pick: MPF_ASSEMBLY_* mode, staged-element cap, ms per assembly          */
+/* The autotuner's assembly pick: MPF_ASSEMBLY_* mode, mpf_set_chunk_stage_cap's value, ms per       */
+/* assembly                                                                                         */
 /* (MPF_ERR_STATE before mpf_batch_autotune).                                                      */
 mpf_status mpf_batch_assembly_choice(const mpf_problem* p, int32_t* mode, int32_t* stage_cap, double* ms_per_assembly);
 /* Batched solver 1: milliseconds per direct solve of every mesh (band fill, factorisation, solve and */

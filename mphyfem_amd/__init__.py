@@ -758,7 +758,7 @@ class Problem:
         return ms.value
 
     def batch_assembly_choice(self):
-        """(ASSEMBLY_* mode, staged-element cap, ms per assembly) picked by batch_autotune."""
+        """(ASSEMBLY_* mode, set_chunk_stage_cap's value, ms per assembly) picked by batch_autotune."""
         m, c, ms = C.c_int32(), C.c_int32(), C.c_double()
         _check(lib().mpf_batch_assembly_choice(self._h, C.byref(m), C.byref(c), C.byref(ms)),
                "mpf_batch_assembly_choice")

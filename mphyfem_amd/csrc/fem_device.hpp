@@ -284,7 +284,7 @@ __device__ __forceinline__ void element_point(const double (*X)[3], const double
                                               double* G, double* S, double* R, bool& negJ) {
   GaussState Q;
   // ten nodes unrolled whole take 314 registers in the mixed element, one wavefront a SIMD; two at a time 154 and three
-  // (48 000 Tet10/P1 elements: 237 -> 184 us; their matrices staged in LDS for contiguous stores instead: 223 us).  The
+  // (the kernel on 48 000 Tet10/P1 elements: 237 -> 184 us; their matrices staged in LDS for contiguous stores: 223 us).  The
   // displacement element takes 228 registers whole, two wavefronts, and is slower two at a time (16 000 elements, whole
   // calls: 69 us against 74).
   gauss_state<NPE, NGP, MIXED, NPE == 10 && MIXED ? 2 : NPE>(X, U, UP, Pn, d, gp, wgp, mu, K, Utype, consistent, Q);

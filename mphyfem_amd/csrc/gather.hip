@@ -518,10 +518,10 @@ __global__ void k_morton_mesh(int32_t nNode, int32_t nmesh, const int32_t* __res
   id[i] = i;
 }
 
-// XCD-aware chunk order: consecutive workgroups land on different XCDs (round robin), so each XCD is
+// XCD-aware order of the workgroups: consecutive ones land on different XCDs (round robin), so each XCD is
 // given a contiguous 1/8 of the work.  Work is laid out in Morton order of the nodes, so that share is a
-// compact region of the mesh whose elements' staging records stay in that XCD's L2.
-__device__ __forceinline__ int64_t xcd_chunk(int64_t b, int64_t nb) {
+// compact region of the mesh, whose elements' records that XCD's L2 holds while its nodes' rows read them.
+__device__ __forceinline__ int64_t xcd_share(int64_t b, int64_t nb) {
   const int64_t per = (nb + 7) / 8;
   return (b % 8) * per + b / 8;
 }
@@ -860,12 +860,13 @@ __device__ __forceinline__ void wave_lds_fence() {
 // (up to) three rows of the node and writes the values: consecutive lanes write consecutive values of a
 // row, and a wavefront that holds a whole node writes its rows entirely.
 // Bound by the vector loads' address processing (2.0 of the 3.0 ms on Hex8 128^3 with every record in cache; a
-// block is 72 scattered bytes) and by memory: 9 GB read and 4.1 GB written, exactly the values.
+// block is 72 scattered bytes) and by memory: 9 GB read and 4.1 GB written, exactly the values.  Tet10/P1, 60^3 x 6:
+// 4.7 ms, 5.2 GB written for 4.3 GB of values (Kpu goes into rows that other wavefronts fill).
 // The two kernels replace Gauss-point records from which every item formed its block (Hex8: eight-wavefront chunks
 // with their elements in LDS, symmetric pairs written to both rows from one sum; Tet10: every item from global
-// memory).  Whole assembly, before -> now: Hex8 10^3 54 -> 40 us, 128^3 8.00 -> 6.07 ms; Q1/P0 45 x 31 x 52
-// 358 -> 251 us, 80^3 2.28 -> 1.54 ms; Tet10 30^3 x 6 830 -> 659 us; Tet10/P1 60^3 x 6 7.33 -> 7.06 ms.  Measured and
-// not taken (Hex8 128^3 / Tet10/P1 60^3 x 6, row kernel): non-temporal value stores 3.82 / 5.73 against 3.57 / 5.39 ms;
+// memory).  A whole assembly call, before -> now: Hex8 10^3 53 -> 39.5 us, 128^3 8.00 -> 6.00 ms; Q1/P0 45 x 31 x 52
+// 359 -> 250 us, 80^3 2.28 -> 1.54 ms; Tet10 30^3 x 6 877 -> 682 us; Tet10/P1 60^3 x 6 7.33 -> 7.08 ms (7.0 to 7.15 over
+// several runs).  A residual alone (kernels, Hex8 128^3): 1.57 -> 1.21 ms.  Measured and not taken (Hex8 128^3 / Tet10/P1 60^3 x 6, row kernel): non-temporal value stores 3.82 / 5.73 against 3.57 / 5.39 ms;
 // 1, 2, 8 wavefronts a workgroup 4.11, 3.93, 4.04 against 3.57 with 4; block offsets by distance before node 3.28 /
 // 4.94 against 2.97 / 4.66 by node.
 constexpr int kRowWaves = 4;
@@ -879,7 +880,7 @@ __global__ void __launch_bounds__(64 * kRowWaves) k_rows(RowArgs F) {
   __shared__ int32_t sStartA[kRowWaves][65];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t nwg = (F.nwaves + kRowWaves - 1) / kRowWaves;
-  const int64_t w = xcd_chunk(blockIdx.x, nwg) * kRowWaves + wid;
+  const int64_t w = xcd_share(blockIdx.x, nwg) * kRowWaves + wid;
   if (w >= F.nwaves) return;  // no workgroup barrier below
   double* const part = sPartA[wid];
   int32_t* const start = sStartA[wid];
@@ -1119,7 +1120,7 @@ mpf_status ensure_gather_tables(mpf_problem* p) {
     MPF_TRY(ids.alloc(nNode));
     // positions quantised to a lattice of spacing h = (bounding-box volume / elements)^(1/3), about
     // the element size: on a structured grid each node gets its own lattice point, so 8 consecutive
-    // nodes of the order form an aligned 2x2x2 block (the chunked matrix kernel's unit of reuse)
+    // nodes of the order form an aligned 2x2x2 block, whose items share most of their elements' records
     double ext[3], h = 0.0;
     for (int c = 0; c < 3; ++c) ext[c] = p->xmax[c] - p->xmin[c];
     const double emax = std::max(ext[0], std::max(ext[1], ext[2]));
