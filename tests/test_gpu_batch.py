@@ -50,7 +50,7 @@ def test_batched_newton_matches_each_mesh_alone(mpf, orc, gpu):
 
 
 def test_batched_band_newton_matches_each_mesh_alone(mpf, orc, gpu):
-    """Batched Newton with exact corrections (banded LDL^T per mesh, one workgroup each): every
+    """Batched Newton with exact corrections (banded LDL^T per mesh): every
     mesh against the oracle's Newton with its direct solve; graph replay equal to direct launches."""
     B, P = _batch(mpf)
     iters, rel, rep = P.batch_newton_solve(nsteps=2, dt=0.5, itmax=25, rtol=1e-11, solver=mpf.BATCH_SOLVER_BAND)
